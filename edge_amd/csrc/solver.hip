@@ -13,6 +13,7 @@
 #include "kernels.hpp"
 #include "ec64_pack.hpp"
 #include "kernels_mfma.hpp"
+#include "kernels_sparse.hpp"
 #include "mfma_pack.hpp"
 #include "setup.hpp"
 #include "visco.hpp"
@@ -66,6 +67,14 @@ struct edge_el_solver {
   void* ec_pk = nullptr;
   void* ec_rot = nullptr;
   void* ec_proj = nullptr;
+  // kernels over the matrices' non-zeros (kernels_sparse.hip): per-element
+  // constants, face-orientation maps.  They run as the element-batched
+  // kernels (5) and as the MFMA kernels (2) with projections exchanged.
+  bool want_sp = false;    // set-up builds their data when the mesh qualifies
+  bool sp_ok = false;
+  bool faces_agree = true; // every interior face's two elements are each other's neighbours
+  void* sp_phys = nullptr;
+  void* sp_rot = nullptr;
   // viscoelastic solvers
   int n_rms = 0;
   void* rfs = nullptr;       // [n_rms]
@@ -222,6 +231,9 @@ int build_neigh(edge_el_solver* s, const edge_mesh_in* m) {
         const unsigned v = m->v_id[el * 4 + fa], fi = m->f_id[el * 4 + fa];
         if (n < 0 || n >= ne || v > 2 || fi > 3)
           return edge::fail(EDGE_ERR_MESH, "interior face without a valid neighbour");
+        const int64_t a = m->fa_el[f * 2], b = m->fa_el[f * 2 + 1];
+        if (!((a == el && b == n) || (a == n && b == el)) || a == b || m->el_fa[n * 4 + fi] != f)
+          s->faces_agree = false;
         nb[el * 4 + fa] = (int32_t)n;
         fm[el * 4 + fa] = (uint8_t)(4 + v * 4 + fi);
       }
@@ -230,7 +242,7 @@ int build_neigh(edge_el_solver* s, const edge_mesh_in* m) {
   EDGE_HIP_TRY(hipMalloc(&s->fmat, 4 * ne));
   EDGE_HIP_TRY(hipMemcpy(s->ne, nb.data(), sizeof(int32_t) * 4 * ne, hipMemcpyHostToDevice));
   EDGE_HIP_TRY(hipMemcpy(s->fmat, fm.data(), 4 * ne, hipMemcpyHostToDevice));
-  if (s->kernel != 2 && !s->proj_tables && !s->want_ec) return EDGE_OK;
+  if (s->kernel != 2 && !s->proj_tables && !s->want_ec && !s->want_sp) return EDGE_OK;
   // Face projections: element el's face fa receives the projection that its
   // neighbour n computes through the shared face (n's face fId, or fa itself
   // on a free surface) with el's flux matrix and neighbour-side solver.
@@ -341,6 +353,46 @@ int finish_ec(edge_el_solver* s) {
   return EDGE_OK;
 }
 
+// The sparse kernels' data, once the flux solvers exist: geometry-built
+// solvers (their constants are in sp_phys) whose faces pair up, with one
+// projection slot per element face.  Runs of 8 have no other tuned kernel:
+// they take these as the element-batched kernels.
+int finish_sp(edge_el_solver* s) {
+  if (!s->want_sp) return EDGE_OK;
+  edge::DgTables t;
+  std::vector<double> rot;
+  if (!s->proj_ok || !s->faces_agree || !edge::dg_tables(s->cfg.order, &t) || !edge::ec_rotations(t, &rot)) {
+    (void)hipFree(s->sp_phys);
+    s->sp_phys = nullptr;
+    return EDGE_OK;
+  }
+  std::vector<double> pk(4 * edge::phys::kRotPad, 0.0);
+  for (int v = 0; v < 4; v++)
+    for (int p = 0; p < s->cfg.order; p++)
+      for (int j = 0; j <= p; j++)
+        for (int c = 0; c <= p; c++)
+          pk[v * edge::phys::kRotPad + edge::phys::rot_off(p) + j * (p + 1) + c] =
+              rot[(v * 16 + p * (p + 1) / 2 + j) * 16 + p * (p + 1) / 2 + c];
+  const bool f32 = s->cfg.precision == 32;
+  const int rc = f32 ? upload_as<float>(pk, &s->sp_rot) : upload_as<double>(pk, &s->sp_rot);
+  if (rc) return rc;
+  s->sp_ok = true;
+  if (s->cfg.kernel == 0 && s->kernel == 1) {
+    EDGE_HIP_TRY(hipMalloc(&s->proj, s->real_bytes * edge::sp_proj_values(s->cfg.order, s->cfg.n_runs) * s->n_el));
+    s->kernel = 5;
+  }
+  return EDGE_OK;
+}
+
+template <typename T>
+edge::SpDev<T> sp_view(const edge_el_solver* s) {
+  edge::SpDev<T> x;
+  x.phys = static_cast<const T*>(s->sp_phys);
+  x.rot = static_cast<const T*>(s->sp_rot);
+  x.proj = static_cast<T*>(s->kernel == 5 && s->cfg.n_runs == 1 ? s->ec_proj : s->proj);
+  return x;
+}
+
 template <typename T>
 edge::EcDev<T> ec_view(const edge_el_solver* s) {
   edge::EcDev<T> x;
@@ -358,6 +410,11 @@ int pick_kernel(edge_el_solver* s) {
   // the element-batched kernels' data is built whenever they may run
   // (requested, the default, or an autotuner candidate)
   s->want_ec = ec_ok && (s->cfg.kernel == 0 || s->cfg.kernel == 4 || s->cfg.kernel == 5);
+  // the sparse kernels stand in for the MFMA kernels (2) and the
+  // element-batched ones (5), and for the generic kernels of other run counts
+  s->want_sp = edge::sp_supported(s->cfg.order, s->cfg.n_runs, s->cfg.precision) &&
+               (s->want_ec || (mfma_ok && (s->cfg.kernel == 0 || s->cfg.kernel == 2)) ||
+                (s->cfg.kernel == 0 && !mfma_ok && !p64_ok && gen_ok));
   if (s->cfg.kernel == 5) {
     if (!ec_ok) return edge::fail(EDGE_ERR_UNSUPPORTED, "element-batched kernels: one run, orders 2-5");
     s->kernel = 5;
@@ -411,8 +468,12 @@ int create_common(const edge_el_config* cfg, const edge_mesh_in* mesh, edge_el_s
 // The MFMA kernels exchange face projections between the local and the
 // neighbour step: the neighbour step then reads them instead of tInt.
 bool proj_active(const edge_el_solver* s) {
-  return (s->kernel == 2 && s->fs_rank3 && s->fsf && s->use_proj && s->proj) || (s->kernel == 5 && s->ec_ok);
+  return (s->kernel == 2 && s->fs_rank3 && s->fsf && s->use_proj && s->proj) ||
+         (s->kernel == 5 && (s->ec_ok || s->sp_ok));
 }
+
+// The sparse kernels run this solver's steps.
+bool sp_active(const edge_el_solver* s) { return s->sp_ok && s->n_rms == 0 && proj_active(s); }
 
 // A local step that writes projections records the tInt array it wrote.
 void note_local(edge_el_solver* s, const void* t_int) {
@@ -447,6 +508,8 @@ int local_t(edge_el_solver* s, int64_t first, int64_t n, double dt, void* dofs, 
   if (s->n_rms > 0) return edge::fail(EDGE_ERR_ARG, "viscoelastic solver: the step needs dofs_a (edge_el_local_a)");
   const auto d = dev_view<T>(s);
   note_local(s, t_int);
+  if constexpr (sizeof(T) == 4)
+    if (sp_active(s)) return edge::launch_local_sp<T>(d, sp_view<T>(s), first, n, (T)dt, (T*)dofs, (T*)t_int, st);
   if (s->kernel == 2) return edge::launch_local_mfma<T>(d, first, n, (T)dt, (T*)dofs, (T*)t_int, st);
   if (s->kernel == 5) return edge::launch_local_ec<T>(d, ec_view<T>(s), first, n, (T)dt, (T*)dofs, (T*)t_int, st);
   if constexpr (sizeof(T) == 8)
@@ -459,6 +522,8 @@ int neigh_t(edge_el_solver* s, int64_t first, int64_t n, const void* t_int, void
   if (s->n_rms > 0) return edge::fail(EDGE_ERR_ARG, "viscoelastic solver: the step needs dofs_a (edge_el_neigh_a)");
   const auto d = dev_view<T>(s);
   if (int rc = check_neigh(s, t_int)) return rc;
+  if constexpr (sizeof(T) == 4)
+    if (sp_active(s)) return edge::launch_neigh_sp<T>(d, sp_view<T>(s), first, n, (T*)dofs, st);
   if (s->kernel == 2) return edge::launch_neigh_mfma<T>(d, first, n, (const T*)t_int, (T*)dofs, st);
   if (s->kernel == 5) return edge::launch_neigh_ec<T>(d, ec_view<T>(s), first, n, (T*)dofs, st);
   if constexpr (sizeof(T) == 8)
@@ -512,7 +577,16 @@ int neigh_lts_t(edge_el_solver* s, int64_t first, int64_t n, int first_ts, const
   if (d.rcv) d.rcv = s->rcv_lts;
   int rc = check_neigh(s, t0);
   if (rc) return rc;
-  if (s->kernel == 2)
+  bool done = false;
+  if constexpr (sizeof(T) == 4) {
+    if (sp_active(s)) {
+      rc = edge::launch_neigh_sp<T>(d, sp_view<T>(s), first, n, (T*)dofs, st);
+      done = true;
+    }
+  }
+  if (done)
+    ;
+  else if (s->kernel == 2)
     rc = edge::launch_neigh_mfma<T>(d, first, n, (const T*)t0, (T*)dofs, st);
   else if (s->kernel == 5)
     rc = edge::launch_neigh_ec<T>(d, ec_view<T>(s), first, n, (T*)dofs, st);
@@ -628,6 +702,19 @@ int fused_steps(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void*
   float* P[2] = {static_cast<float*>(s->proj), static_cast<float*>(s->proj_alt)};
   auto d = dev_view<float>(s);
   const float fdt = (float)dt;
+  if (sp_active(s)) {
+    auto x = sp_view<float>(s);
+    x.proj = P[0];
+    int rc = edge::launch_local_sp<float>(d, x, 0, s->n_el, fdt, (float*)dofs, (float*)t_int, st);
+    if (rc == EDGE_OK && s->fault) rc = edge::fault_apply(s->fault, dt, t_int, dofs, st);
+    for (int64_t k = 1; k < n_steps && rc == EDGE_OK; k++) {
+      x.proj = P[k % 2];
+      rc = edge::launch_fused_sp<float>(d, x, fdt, P[(k - 1) % 2], (float*)dofs, (float*)t_int, st);
+      if (rc == EDGE_OK && s->fault) rc = edge::fault_apply(s->fault, dt, t_int, dofs, st);
+    }
+    x.proj = P[(n_steps - 1) % 2];
+    return rc ? rc : edge::launch_neigh_sp<float>(d, x, 0, s->n_el, (float*)dofs, st);
+  }
   d.proj = P[0];
   int rc = edge::launch_local_mfma<float>(d, 0, s->n_el, fdt, (float*)dofs, (float*)t_int, st);
   if (rc == EDGE_OK && s->fault) rc = edge::fault_apply(s->fault, dt, t_int, dofs, st);
@@ -694,17 +781,19 @@ extern "C" int edge_el_create(const edge_el_config* cfg, const edge_mesh_in* mes
                         mesh->fa_el, mesh->fa_type, mesh->normals, mesh->tangents, mesh->areas, rho,
                         lam,         mu};
     s->sparse_star = true;  // built from the Jacobians' pattern only
-    if (hipMalloc(&s->jdet, sizeof(double) * s->n_el) != hipSuccess)
-      rc = edge::fail(EDGE_ERR_HIP, "allocation of Jacobian determinants");
+    if (hipMalloc(&s->jdet, sizeof(double) * s->n_el) != hipSuccess ||
+        (s->want_sp && hipMalloc(&s->sp_phys, s->real_bytes * edge::phys::values(s->n_el)) != hipSuccess))
+      rc = edge::fail(EDGE_ERR_HIP, "allocation of the element constants");
     else
       rc = cfg->precision == 64
                ? edge::build_setup<double>(in, (double*)s->star, (double*)s->fs, s->jdet, (double*)s->fsf,
-                                           &s->fs_rank3, nullptr, nullptr, nullptr, nullptr)
+                                           &s->fs_rank3, nullptr, nullptr, nullptr, (double*)s->sp_phys, nullptr)
                : edge::build_setup<float>(in, (float*)s->star, (float*)s->fs, s->jdet, (float*)s->fsf,
-                                          &s->fs_rank3, nullptr, nullptr, nullptr, nullptr);
+                                          &s->fs_rank3, nullptr, nullptr, nullptr, (float*)s->sp_phys, nullptr);
     if (rc == EDGE_OK) rc = zero_fault_faces(s);
     if (rc == EDGE_OK) rc = finish_mfma(s);
     if (rc == EDGE_OK) rc = finish_ec(s);
+    if (rc == EDGE_OK) rc = finish_sp(s);
     if (rc == EDGE_OK) rc = upload_element_data(s, mesh, rho, lam, mu);
   }
   if (rc != EDGE_OK) {
@@ -783,6 +872,8 @@ extern "C" int edge_el_destroy(edge_el_solver* s) {
   (void)hipFree(s->ec_pk);
   (void)hipFree(s->ec_rot);
   (void)hipFree(s->ec_proj);
+  (void)hipFree(s->sp_phys);
+  (void)hipFree(s->sp_rot);
   drop_lts(s);
   delete s;
   return EDGE_OK;
@@ -909,10 +1000,10 @@ extern "C" int edge_el_create_visco(const edge_el_config* cfg, const edge_visco_
       rc = cfg->precision == 64
                ? edge::build_setup<double>(in, (double*)s->star, (double*)s->fs, s->jdet, (double*)s->fsf,
                                            &s->fs_rank3, (double*)s->star_a, (double*)s->fs_a, (double*)s->fsfa,
-                                           nullptr)
+                                           nullptr, nullptr)
                : edge::build_setup<float>(in, (float*)s->star, (float*)s->fs, s->jdet, (float*)s->fsf,
                                           &s->fs_rank3, (float*)s->star_a, (float*)s->fs_a, (float*)s->fsfa,
-                                          nullptr);
+                                          nullptr, nullptr);
     if (rc == EDGE_OK) rc = zero_fault_faces(s);
     if (rc == EDGE_OK) rc = upload_element_data(s, mesh, rho, s->lam_e.data(), s->mu_e.data());
     if (rc == EDGE_OK && p64_ok && src_pattern && (cfg->kernel == 0 || cfg->kernel == 4)) s->kernel = 4;
@@ -1066,7 +1157,7 @@ std::vector<TuneCand> tune_candidates(edge_el_solver* s) {
     const bool p64 = edge::plain64_supported(s->cfg.order, s->cfg.n_runs, prec_bytes);
     for (int x = 1; x >= 0; x--) {  // XCD-aware schedule, then the linear one
       if (p64) c.push_back({4, false, x == 1});
-      if (s->ec_ok) c.push_back({5, true, x == 1});  // element-batched: projections always exchanged
+      if (s->ec_ok || s->sp_ok) c.push_back({5, true, x == 1});  // element-batched: projections always exchanged
     }
   }
   if (gen || c.empty()) c.push_back({1, false});
@@ -1413,8 +1504,15 @@ extern "C" int edge_el_neigh_local(edge_el_solver* s, double dt, void* dofs, voi
   if (!s->proj_alt) EDGE_HIP_TRY(hipMalloc(&s->proj_alt, sizeof(float) * 4 * 768 * s->n_el));
   auto d = dev_view<float>(s);
   d.proj = static_cast<float*>(s->proj_alt);
-  rc = edge::launch_fused_mfma(d, (float)dt, static_cast<const float*>(s->proj), (float*)dofs, (float*)t_int,
-                               (hipStream_t)stream);
+  if (sp_active(s)) {
+    auto x = sp_view<float>(s);
+    x.proj = static_cast<float*>(s->proj_alt);
+    rc = edge::launch_fused_sp<float>(d, x, (float)dt, static_cast<const float*>(s->proj), (float*)dofs,
+                                      (float*)t_int, (hipStream_t)stream);
+  } else {
+    rc = edge::launch_fused_mfma(d, (float)dt, static_cast<const float*>(s->proj), (float*)dofs, (float*)t_int,
+                                 (hipStream_t)stream);
+  }
   if (rc) return rc;
   std::swap(s->proj, s->proj_alt);
   note_local(s, t_int);

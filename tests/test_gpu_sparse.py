@@ -1,0 +1,101 @@
+"""The FP32 kernels over the matrices' non-zeros (kernels_sparse_impl.hpp),
+64 (element, run) columns per workgroup, against the FP64 oracle: every order
+and run count on meshes whose last tile is partly filled, element ranges that
+start inside a tile, free-surface, outflow and periodic faces in every
+orientation; and a mesh whose neighbour relations do not pair up, which takes
+the general kernels."""
+import numpy as np
+import pytest
+
+import oracle as orc
+from edge_amd import mesh as M
+from edge_amd import setups as S
+from edge_amd.mesh import FA_FREE_SURFACE, FA_OUTFLOW, FA_PERIODIC
+from edge_amd.solver import ElasticSolver
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-5  # FP32 against the FP64 oracle, as every FP32 path
+
+
+def rel(a, b):
+    a, b = np.asarray(a, np.float64), np.asarray(b, np.float64)
+    return float(np.linalg.norm((a - b).ravel()) / np.linalg.norm(b.ravel()))
+
+
+def _problem(runs, order, n=(3, 4, 3), seed=5):
+    import torch
+    m = M.box(n, bc=(FA_FREE_SURFACE, FA_OUTFLOW, FA_PERIODIC), jitter=0.1, seed=seed)
+    rho, lam, mu = S.random_materials(m.n_el, seed=seed)
+    d0 = np.random.default_rng(order).normal(size=(m.n_el, 9, S.n_modes(order), runs)).astype(np.float32)
+    dev = torch.from_numpy(d0).cuda()
+    return m, (rho, lam, mu), S.dt_cfl(m, rho, lam, mu, order), d0.astype(np.float64), dev
+
+
+@pytest.mark.parametrize("runs", [1, 8, 16])
+@pytest.mark.parametrize("order", [2, 3, 4, 5])
+def test_steps_match_oracle(gpu, order, runs):
+    """216 elements (3.4, 27 and 54 tiles of 64, 8 and 4): local, neighbour,
+    then three steps in one call."""
+    import torch
+    m, mat, dt, d, gd = _problem(runs, order)
+    s = ElasticSolver(m, order, runs, 32, *mat)
+    mo = orc.MeshOracle(m, order, runs, rho=mat[0], lam=mat[1], mu=mat[2])
+    t, gt = np.zeros_like(d), torch.zeros_like(gd)
+    mo.local(d, t, dt)
+    s.local(gd, gt, dt)
+    assert rel(gt.cpu().numpy(), t) <= TOL
+    assert rel(gd.cpu().numpy(), d) <= TOL
+    mo.neigh(d, t)
+    s.neigh(gd, gt)
+    assert rel(gd.cpu().numpy(), d) <= TOL
+    mo.step(d, t, dt, 3)
+    s.step(gd, gt, dt, 3)
+    assert rel(gt.cpu().numpy(), t) <= TOL
+    assert rel(gd.cpu().numpy(), d) <= TOL
+    s.close()
+
+
+@pytest.mark.parametrize("runs", [1, 8, 16])
+def test_ranges_equal_whole(gpu, runs):
+    """Element ranges that start and end inside a tile (and inside a block of
+    the constants) write their elements only, and the same values as one call."""
+    import torch
+    order = 4
+    m, mat, dt, _, gd = _problem(runs, order)
+    s = ElasticSolver(m, order, runs, 32, *mat)
+    cuts = [0, 1, 62, 67, 130, 131, 215, m.n_el]
+    a, ta = gd.clone(), torch.zeros_like(gd)
+    s.local(a, ta, dt)
+    local = a.clone()
+    s.neigh(a, ta)
+    b, tb = gd.clone(), torch.zeros_like(gd)
+    for lo, hi in zip(cuts[:-1], cuts[1:]):
+        before, tbefore = b.clone(), tb.clone()
+        s.local(b, tb, dt, first=lo, n=hi - lo)
+        assert torch.equal(b[:lo], before[:lo]) and torch.equal(b[hi:], before[hi:])
+        assert torch.equal(tb[:lo], tbefore[:lo]) and torch.equal(tb[hi:], tbefore[hi:])
+    assert torch.equal(local, b) and torch.equal(ta, tb)
+    for lo, hi in zip(cuts[:-1], cuts[1:]):
+        before = b.clone()
+        s.neigh(b, tb, first=lo, n=hi - lo)
+        assert torch.equal(b[:lo], before[:lo]) and torch.equal(b[hi:], before[hi:])
+    assert torch.equal(a, b)
+    s.close()
+
+
+@pytest.mark.parametrize("runs", [1, 16])
+def test_neighbours_that_do_not_pair(gpu, runs):
+    """One face's neighbour replaced by another element: the projections no
+    longer have one receiver each, so the general kernels run."""
+    import torch
+    order = 3
+    m, mat, dt, d, gd = _problem(runs, order)
+    el, fa = np.argwhere((m.fa_el[m.el_fa] >= 0).all(axis=2) & (m.fa_type[m.el_fa] == 0))[5]
+    m.el_fa_el[el, fa] = (m.el_fa_el[el, fa] + 7) % m.n_el
+    s = ElasticSolver(m, order, runs, 32, *mat)
+    mo = orc.MeshOracle(m, order, runs, rho=mat[0], lam=mat[1], mu=mat[2])
+    t, gt = np.zeros_like(d), torch.zeros_like(gd)
+    mo.step(d, t, dt, 2)
+    s.step(gd, gt, dt, 2)
+    assert rel(gd.cpu().numpy(), d) <= TOL
+    s.close()
