@@ -7,8 +7,11 @@
 namespace edge {
 namespace phys {
 
-// Per-element constants of the elastic update, [el / 64][kSize][el % 64] in
-// the solver's precision, each computed in FP64 and rounded once.  With J^-1
+// Per-element constants of the elastic update, [el / B][kSize][el % B] with
+// B = block(runs): one run's lanes are different elements and read a constant
+// of 64 of them at a time, the few elements of a tile of fused runs are
+// contiguous.  In the solver's precision, each computed in FP64 and rounded
+// once.  With J^-1
 // the inverse Jacobian (j[k][d] = d xi_d / d x_k), n a face's outward normal,
 // sc = -2 |A| / |J|, zp and zs the P and S impedances (1: the element's own
 // side, 2: the other side):
@@ -21,8 +24,8 @@ namespace phys {
 constexpr int kJinv = 0, kLam2 = 9, kLam = 10, kMu = 11, kIrho = 12, kFace = 13;
 constexpr int kNrm = 0, kPrj = 3, kScN = 7, kOwn = 10, kOth = 12, kPerFace = 14;
 constexpr int kSize = kFace + 4 * kPerFace;
-constexpr int kBlock = 64;  // elements per block of the layout
-inline int64_t values(int64_t n_el) { return (n_el + kBlock - 1) / kBlock * kBlock * kSize; }
+constexpr int block(int n_runs) { return n_runs == 1 ? 64 : 1; }
+inline int64_t values(int64_t n_el, int b) { return (n_el + b - 1) / b * b * kSize; }
 
 // Face-orientation maps R_v (ec64_pack.hpp) as their diagonal blocks by
 // face-basis degree p, row-major, padded: [4][kRotPad] (0: the identity).
@@ -31,17 +34,21 @@ constexpr int rot_off(int p) { return p * (p + 1) * (2 * p + 1) / 6; }  // 0, 1,
 
 }  // namespace phys
 
+// Vectors of four values per face projection (3 NF values, padded).
+constexpr int sp_proj_vectors(int order) { return (3 * n_face_modes(order) + 3) / 4; }
+// Values of the face projections per element.
+constexpr int64_t sp_proj_values(int order, int n_runs) { return (int64_t)16 * sp_proj_vectors(order) * n_runs; }
+
 template <typename T>
 struct SpDev {
   const T* phys = nullptr;  // per-element constants
   const T* rot = nullptr;   // face-orientation maps
-  T* proj = nullptr;        // face projections [nEl][4][12][R][(NF + 3) / 4] of this step
+  T* proj = nullptr;        // face projections [nEl][4][vectors][R][4] of this step
+  // tInt is written for every element, or only for those of need (a step
+  // whose tInt nothing else reads)
+  bool tint = true;
+  const uint8_t* need = nullptr;  // [nEl], null: none
 };
-
-// Values of the face projections per element.
-constexpr int64_t sp_proj_values(int order, int n_runs) {
-  return (int64_t)48 * ((n_face_modes(order) + 3) / 4) * n_runs;
-}
 
 // One operation of one order (kernels_sparse_o*.hip).
 constexpr int kSpLocal = 0, kSpNeigh = 1, kSpFused = 2;
@@ -56,7 +63,7 @@ int launch_local_sp(const SolverDev<T>& s, const SpDev<T>& x, int64_t first, int
 template <typename T>
 int launch_neigh_sp(const SolverDev<T>& s, const SpDev<T>& x, int64_t first, int64_t n, T* dofs, hipStream_t st);
 // The neighbour step of step k - 1 (from proj_in) and the local step of step
-// k (projections to x.proj) as one launch over all elements (8 or 16 runs).
+// k (projections to x.proj) as one launch over all elements.
 template <typename T>
 int launch_fused_sp(const SolverDev<T>& s, const SpDev<T>& x, T dt, const T* proj_in, T* dofs, T* t_int,
                     hipStream_t st);

@@ -4,14 +4,14 @@
 // In the hierarchical orthogonal basis 82 % of the stiffness and 58 % of the
 // flux matrices' entries are zero, and which ones is known when the kernels
 // are compiled.  A lane holds one column, one (element, run) pair, and a
-// workgroup of four waves works on 64 columns (64 / R elements).  Wave w owns
-// a quarter of the modes of every quantity (Own): it keeps their DOFs in
+// workgroup of W waves works on 64 columns (64 / R elements).  Each wave owns
+// a share of the modes of every quantity (Deal): it keeps their DOFs in
 // registers, so everything that mixes quantities at one mode is lane-local,
 // and it computes the outputs of its modes of every matrix product.  The
 // inputs of a product pass through LDS: the owners publish a column
 // [mode][64] and every wave reads the modes its outputs need.  Each non-zero
 // is one v_fmac_f32 with the entry as a literal: no operand loads, no
-// padding, no work on zeros.  The four waves run different code (their own
+// padding, no work on zeros.  The waves run different code (their own
 // non-zeros), the partition of the modes balances it.
 //
 // Instead of the 9 x 9 star matrices and flux solvers the kernels use what
@@ -29,12 +29,18 @@
 // map R_v (ec64_pack.hpp).
 //
 // What bounds it: vector-ALU issue (about 40,000 instructions per tile and
-// 64 columns at order 5 against 131,000 cycles of padded MFMA tiles) and, with
-// two workgroups per CU, the LDS and memory latency they leave exposed.
+// 64 columns at order 5 against 131,000 cycles of padded MFMA tiles; 46 % of
+// the issue slots are used) and the memory latency that two (order 5) or
+// three workgroups per CU leave exposed.  A load behind output stores waits
+// for all of them, so constants come first, the projections leave last and
+// tInt is written while they are formed.
+// Eight waves of half the modes (128 registers) took 10.9 ms per order-5 step
+// against 7.7 for four.
 // Measured against the kernels that did the same before (ms per step): order
-// 5, 196,608 tets, 16 runs 8.59 -> 7.70 (MFMA, runs on N); one run 1.19 ->
-// 1.01 (MFMA, 16 elements on N); order 5, 36,720 tets, 8 runs 6.81 -> 0.87
-// (generic); order 4 with a fault, 331,776 tets, 16 runs 10.3 -> 6.69.
+// 5, 196,608 tets, 16 runs with sources and receivers 8.60 -> 6.3 (MFMA, runs
+// on N); one run 1.19 -> 0.57 (MFMA, 16 elements on N); order 5, 36,720 tets,
+// 8 runs 6.81 -> 0.69 (generic); order 4 with a fault, 331,776 tets, 16 runs
+// 10.3 -> 5.3.
 //
 // Operations (src/impl/seismic/solvers/AderDg.hpp:362-533, :553-722):
 //   local: CK time prediction (TimePredVanilla.hpp:200-306), volume integral
@@ -62,66 +68,56 @@ namespace {
 constexpr int kCols = 64;  // columns (lanes) per workgroup tile
 constexpr int kWaves = 4;
 
-// Modes and face modes of each wave: found by balancing the waves' non-zeros
-// per product, with the modes of every lower order spread evenly as well (a
-// derivative's outputs are a prefix of each list).  -1: none.
+// The order in which the modes and face modes are dealt to the waves: wave w
+// of W owns the modes at positions j W + w, and a column's LDS row is the
+// position.  Found by balancing the waves' non-zeros per product; the modes
+// of every lower order come first (a derivative's outputs are a prefix).
 template <int O>
-struct Own;
+struct Deal;
 template <>
-struct Own<2> {
-  static constexpr int mode[4][1] = {{0}, {1}, {2}, {3}};
-  static constexpr int face[4][1] = {{0}, {1}, {2}, {-1}};
+struct Deal<2> {
+  static constexpr int mode[4] = {0, 2, 1, 3};
+  static constexpr int face[3] = {0, 2, 1};
 };
 template <>
-struct Own<3> {
-  static constexpr int mode[4][3] = {{0, 6, -1}, {1, 5, 7}, {3, 4, 9}, {2, 8, -1}};
-  static constexpr int face[4][2] = {{3, 4}, {2, 5}, {1, -1}, {0, -1}};
+struct Deal<3> {
+  static constexpr int mode[10] = {0, 1, 3, 2, 6, 5, 9, 8, 4, 7};
+  static constexpr int face[6] = {2, 3, 0, 1, 5, 4};
 };
 template <>
-struct Own<4> {
-  static constexpr int mode[4][5] = {{0, 8, 10, 12, 16}, {1, 7, 11, 15, 17}, {2, 5, 9, 13, 18}, {3, 4, 6, 14, 19}};
-  static constexpr int face[4][3] = {{4, 6, 8}, {1, 7, 9}, {0, 5, -1}, {2, 3, -1}};
+struct Deal<4> {
+  static constexpr int mode[20] = {0, 3, 2, 1, 9, 4, 5, 6, 8, 7, 19, 12, 11, 16, 14, 17, 10, 15, 13, 18};
+  static constexpr int face[10] = {7, 8, 0, 2, 9, 6, 5, 3, 1, 4};
 };
 template <>
-struct Own<5> {
-  static constexpr int mode[4][9] = {{0, 6, 11, 13, 19, 22, 27, 33, -1},
-                                     {1, 7, 10, 16, 18, 25, 26, 29, 30},
-                                     {2, 5, 9, 14, 15, 20, 24, 28, 31},
-                                     {3, 4, 8, 12, 17, 21, 23, 32, 34}};
-  static constexpr int face[4][4] = {{2, 5, 10, 12}, {6, 7, 8, 13}, {1, 4, 11, 14}, {0, 3, 9, -1}};
+struct Deal<5> {
+  static constexpr int mode[35] = {0,  3,  2,  1,  8,  4,  5,  7,  9,  6,  14, 19, 13, 15, 11, 10, 16, 18,
+                                   17, 12, 30, 34, 29, 33, 21, 25, 32, 31, 20, 23, 27, 24, 28, 26, 22};
+  static constexpr int face[15] = {5, 8, 4, 9, 12, 13, 14, 0, 11, 7, 10, 2, 1, 6, 3};
 };
 
 template <int O>
 struct Dim {
   static constexpr int N = n_modes(O), NF = n_face_modes(O);
-  static constexpr int M = (N + 3) / 4, MF = (NF + 3) / 4;  // most modes / face modes of a wave
-  // most of the modes below nn that a wave owns: a column of nn modes takes
-  // 4 own(nn) LDS rows, mode Own[w][j] in row 4 j + w
-  static constexpr int own(int nn) {
-    int most = 0;
-    for (int w = 0; w < 4; w++) {
-      int c = 0;
-      for (int j = 0; j < M; j++) c += Own<O>::mode[w][j] >= 0 && Own<O>::mode[w][j] < nn;
-      most = c > most ? c : most;
-    }
-    return most;
-  }
+  static constexpr int W = kWaves;
+  static constexpr int own(int nn) { return (nn + W - 1) / W; }  // most modes below nn of a wave
+  static constexpr int M = own(N), MF = own(NF);
+  // mode / face mode at position j of wave w, -1: none
+  static constexpr int mode(int w, int j) { return j * W + w < N ? Deal<O>::mode[j * W + w] : -1; }
+  static constexpr int face(int w, int j) { return j * W + w < NF ? Deal<O>::face[j * W + w] : -1; }
   static constexpr int row(int k) {
-    for (int w = 0; w < 4; w++)
-      for (int j = 0; j < M; j++)
-        if (Own<O>::mode[w][j] == k) return 4 * j + w;
+    for (int p = 0; p < N; p++)
+      if (Deal<O>::mode[p] == k) return p;
     return -1;
   }
   static constexpr int face_row(int k) {
-    for (int w = 0; w < 4; w++)
-      for (int j = 0; j < MF; j++)
-        if (Own<O>::face[w][j] == k) return 4 * j + w;
+    for (int p = 0; p < NF; p++)
+      if (Deal<O>::face[p] == k) return p;
     return -1;
   }
-  static constexpr int FR = 4 * MF;                 // rows of a face column
-  static constexpr int WROWS = 12 * FR;             // all four faces' w
-  static constexpr int CROWS = 4 * 4 * own(N);      // four columns of the CK's first stage
-  static constexpr int LROWS = 2 * CROWS > WROWS + 3 * 4 * M ? 2 * CROWS : WROWS + 3 * 4 * M;
+  static constexpr int WROWS = 12 * NF;    // all four faces' w
+  static constexpr int CROWS = 4 * N;      // four columns of the CK's first stage
+  static constexpr int LROWS = 2 * CROWS > WROWS + 3 * N ? 2 * CROWS : WROWS + 3 * N;
 };
 
 template <int V>
@@ -182,7 +178,7 @@ __device__ __forceinline__ void term(T x, T& out) {
 }
 template <int O, int NN, int W, int J>
 constexpr int mode_of() {
-  return Own<O>::mode[W][J] < NN ? Own<O>::mode[W][J] : -1;
+  return Dim<O>::mode(W, J) < NN ? Dim<O>::mode(W, J) : -1;
 }
 template <int O, int NN, int W, typename Mat, int K, typename T, int... J>
 __device__ __forceinline__ void terms(T x, T* out, std::integer_sequence<int, J...>) {
@@ -190,85 +186,199 @@ __device__ __forceinline__ void terms(T x, T* out, std::integer_sequence<int, J.
 }
 template <int O, int W, typename Mat, int K, typename T, int... J>
 __device__ __forceinline__ void face_terms(T x, T* out, std::integer_sequence<int, J...>) {
-  (term<Mat, K, Own<O>::face[W][J], starts<Mat, K, Own<O>::face[W][J]>()>(x, out[J]), ...);
+  (term<Mat, K, Dim<O>::face(W, J), starts<Mat, K, Dim<O>::face(W, J)>()>(x, out[J]), ...);
 }
-// The same with the sum running over three matrices per input.
-template <int O, int NN, int W, typename M0, typename M1, typename M2, int K, typename T, int J>
-__device__ __forceinline__ void term3(T x0, T x1, T x2, T& out) {
+// The same with the sum running over three matrices per input (x: input K
+// of matrix D).
+template <int O, int NN, int W, typename M0, typename M1, typename M2, int K, int D, int J, typename T>
+__device__ __forceinline__ void term3(T x, T& out) {
   constexpr int N = mode_of<O, NN, W, J>();
   if constexpr (N >= 0) {
     constexpr bool s = starts<M0, K, N>() && starts<M1, K, N>() && starts<M2, K, N>();
     constexpr bool n0 = M0::at(K, N) != 0.0, n1 = M1::at(K, N) != 0.0;
-    term<M0, K, N, s>(x0, out);
-    term<M1, K, N, s && !n0>(x1, out);
-    term<M2, K, N, s && !n0 && !n1>(x2, out);
+    if constexpr (D == 0) term<M0, K, N, s>(x, out);
+    if constexpr (D == 1) term<M1, K, N, s && !n0>(x, out);
+    if constexpr (D == 2) term<M2, K, N, s && !n0 && !n1>(x, out);
   }
 }
-template <int O, int NN, int W, typename M0, typename M1, typename M2, int K, typename T, int... J>
-__device__ __forceinline__ void terms3(T x0, T x1, T x2, T* out, std::integer_sequence<int, J...>) {
-  (term3<O, NN, W, M0, M1, M2, K, T, J>(x0, x1, x2, out[J]), ...);
+template <int O, int NN, int W, typename M0, typename M1, typename M2, int K, int D, typename T, int... J>
+__device__ __forceinline__ void terms3(T x, T* out, std::integer_sequence<int, J...>) {
+  (term3<O, NN, W, M0, M1, M2, K, D, J>(x, out[J]), ...);
 }
 
 template <int O, bool CK, int D>
 using Stiff = std::conditional_t<CK, Ck<O, D>, Vol<O, D>>;
 
+// The LDS reads of a product in the order of its sums, each with the columns
+// and inputs it feeds.  A wave takes them in groups of G: the next group is
+// requested before the present one's multiply-adds, which keeps the LDS
+// latency behind about 30 of them (left to itself the compiler reads just
+// ahead of each use).
+struct Read {
+  int col, k;
+};
+template <int MAX>
+struct Reads {
+  int n = 0;
+  Read r[MAX] = {};
+  constexpr void add(int col, int k) {
+    r[n].col = col;
+    r[n].k = k;
+    n++;
+  }
+};
+
 // One published component: column 0 (the raw velocity) times all three
 // stiffness matrices into p[d], columns 1 + d times matrix d, summed, into v;
-// outputs of wave W below NN, inputs below NK.  l: the lane's first row;
-// RK: rows per column.
-template <int O, bool CK, int NK, int NN, int W, typename T, int... K>
-__device__ __forceinline__ void stiff_mul(const T* l, T (&p)[3][Dim<O>::own(NN)], T (&v)[Dim<O>::own(NN)],
-                                          std::integer_sequence<int, K...>) {
-  constexpr int RK = 4 * Dim<O>::own(NK) * kCols;
-  using J = std::make_integer_sequence<int, Dim<O>::own(NN)>;
-  (
-      [&]() EDGE_INLINE {
-        const T x = l[Dim<O>::row(K) * kCols];
-        terms<O, NN, W, Stiff<O, CK, 0>, K>(x, p[0], J{});
-        terms<O, NN, W, Stiff<O, CK, 1>, K>(x, p[1], J{});
-        terms<O, NN, W, Stiff<O, CK, 2>, K>(x, p[2], J{});
-      }(),
-      ...);
-  (
-      [&]() EDGE_INLINE {
-        terms3<O, NN, W, Stiff<O, CK, 0>, Stiff<O, CK, 1>, Stiff<O, CK, 2>, K>(
-            l[RK + Dim<O>::row(K) * kCols], l[2 * RK + Dim<O>::row(K) * kCols], l[3 * RK + Dim<O>::row(K) * kCols], v,
-            J{});
-      }(),
-      ...);
-}
+// outputs of wave V below NN, inputs below NK.
+template <int O, bool CK, int NK, int NN, int V>
+struct StiffReads {
+  static constexpr int J = Dim<O>::own(NN), G = 12, ROWS = NK;
+  template <int D>
+  static constexpr bool feeds(int k) {
+    for (int j = 0; j < J; j++) {
+      const int n = Dim<O>::mode(V, j);
+      if (n >= 0 && n < NN && Stiff<O, CK, D>::at(k, n) != 0.0) return true;
+    }
+    return false;
+  }
+  static constexpr Reads<4 * NK> list() {
+    Reads<4 * NK> l;
+    for (int k = 0; k < NK; k++)
+      if (feeds<0>(k) || feeds<1>(k) || feeds<2>(k)) l.add(0, k);
+    for (int k = 0; k < NK; k++) {
+      if (feeds<0>(k)) l.add(1, k);
+      if (feeds<1>(k)) l.add(2, k);
+      if (feeds<2>(k)) l.add(3, k);
+    }
+    return l;
+  }
+  static constexpr int row(int k) { return Dim<O>::row(k); }
+  template <int COL, int K, typename T>
+  static __device__ __forceinline__ void use(T x, T (&p)[3][J], T (&v)[J]) {
+    using M0 = Stiff<O, CK, 0>;
+    using M1 = Stiff<O, CK, 1>;
+    using M2 = Stiff<O, CK, 2>;
+    using JS = std::make_integer_sequence<int, J>;
+    if constexpr (COL == 0) {
+      terms<O, NN, V, M0, K>(x, p[0], JS{});
+      terms<O, NN, V, M1, K>(x, p[1], JS{});
+      terms<O, NN, V, M2, K>(x, p[2], JS{});
+    } else {
+      terms3<O, NN, V, M0, M1, M2, K, COL - 1>(x, v, JS{});
+    }
+  }
+};
 
 // One column of a face's w in the element's modes to the wave's face modes.
-template <int O, int F, int W, typename T, int... K>
-__device__ __forceinline__ void project_mul(const T* l, T (&u)[Dim<O>::MF], std::integer_sequence<int, K...>) {
-  (face_terms<O, W, Prj<O, F>, K>(l[Dim<O>::row(K) * kCols], u, std::make_integer_sequence<int, Dim<O>::MF>{}), ...);
-}
+template <int O, int F, int V>
+struct ProjectReads {
+  static constexpr int N = Dim<O>::N, J = Dim<O>::MF, G = 12, ROWS = 0;
+  static constexpr Reads<N> list() {
+    Reads<N> l;
+    for (int k = 0; k < N; k++) {
+      bool on = false;
+      for (int j = 0; j < J; j++) {
+        const int n = Dim<O>::face(V, j);
+        on = on || (n >= 0 && Prj<O, F>::at(k, n) != 0.0);
+      }
+      if (on) l.add(0, k);
+    }
+    return l;
+  }
+  static constexpr int row(int k) { return Dim<O>::row(k); }
+  template <int COL, int K, typename T>
+  static __device__ __forceinline__ void use(T x, T (&u)[J]) {
+    face_terms<O, V, Prj<O, F>, K>(x, u, std::make_integer_sequence<int, J>{});
+  }
+};
 
 // One face column to the wave's modes.
-template <int O, int F, int W, typename T, int... K>
-__device__ __forceinline__ void lift_mul(const T* l, T (&u)[Dim<O>::M], std::integer_sequence<int, K...>) {
-  (terms<O, Dim<O>::N, W, Lift<O, F>, K>(l[Dim<O>::face_row(K) * kCols], u,
-                                         std::make_integer_sequence<int, Dim<O>::M>{}),
-   ...);
+template <int O, int F, int V>
+struct LiftReads {
+  static constexpr int NF = Dim<O>::NF, J = Dim<O>::M, G = 16, ROWS = 0;
+  static constexpr Reads<NF> list() {
+    Reads<NF> l;
+    for (int k = 0; k < NF; k++) {
+      bool on = false;
+      for (int j = 0; j < J; j++) {
+        const int n = Dim<O>::mode(V, j);
+        on = on || (n >= 0 && Lift<O, F>::at(k, n) != 0.0);
+      }
+      if (on) l.add(0, k);
+    }
+    return l;
+  }
+  static constexpr int row(int k) { return Dim<O>::face_row(k); }
+  template <int COL, int K, typename T>
+  static __device__ __forceinline__ void use(T x, T (&u)[J]) {
+    terms<O, Dim<O>::N, V, Lift<O, F>, K>(x, u, std::make_integer_sequence<int, J>{});
+  }
+};
+
+// Group C of the reads of S into x / its multiply-adds.
+template <typename S, int C, typename T, int... I>
+__device__ __forceinline__ void fetch(const T* l, T (&x)[S::G], std::integer_sequence<int, I...>) {
+  constexpr auto list = S::list();
+  (
+      [&]() EDGE_INLINE {
+        constexpr int at = C * S::G + I;
+        if constexpr (at < list.n) {
+          constexpr int off = (list.r[at].col * S::ROWS + S::row(list.r[at].k)) * kCols;
+          x[I] = l[off];
+        }
+      }(),
+      ...);
+}
+template <typename S, int C, typename T, int... I, typename... Out>
+__device__ __forceinline__ void consume(const T (&x)[S::G], std::integer_sequence<int, I...>, Out&... out) {
+  constexpr auto list = S::list();
+  (
+      [&]() EDGE_INLINE {
+        constexpr int at = C * S::G + I;
+        if constexpr (at < list.n) {
+          constexpr int col = list.r[at].col, k = list.r[at].k;
+          S::template use<col, k>(x[I], out...);
+        }
+      }(),
+      ...);
+}
+template <typename S, int C, typename T, typename... Out>
+__device__ __forceinline__ void stream(const T* l, const T (&x)[S::G], Out&... out) {
+  constexpr int n = S::list().n;
+  using GS = std::make_integer_sequence<int, S::G>;
+  T next[S::G];
+  if constexpr ((C + 1) * S::G < n) fetch<S, C + 1>(l, next, GS{});
+  __builtin_amdgcn_sched_barrier(0);
+  consume<S, C>(x, GS{}, out...);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr ((C + 1) * S::G < n) stream<S, C + 1>(l, next, out...);
+}
+// out += S (columns at the lane's first row l)
+template <typename S, typename T, typename... Out>
+__device__ __forceinline__ void product(const T* l, Out&... out) {
+  if constexpr (S::list().n > 0) {
+    T x[S::G];
+    fetch<S, 0>(l, x, std::make_integer_sequence<int, S::G>{});
+    stream<S, 0>(l, x, out...);
+  }
 }
 
 // The calling wave's code (w is uniform across the wave).  The (empty, but
 // different) last statements keep the branches from being merged over the
 // registers they update, which would put those into memory.
-template <typename F>
+template <int W, int I = 0, typename F>
 __device__ __forceinline__ void by_wave(int w, F f) {
-  if (w == 0) {
-    f(Int<0>{});
-    asm volatile("; wave 0");
-  } else if (w == 1) {
-    f(Int<1>{});
-    asm volatile("; wave 1");
-  } else if (w == 2) {
-    f(Int<2>{});
-    asm volatile("; wave 2");
+  if constexpr (I + 1 < W) {
+    if (w == I) {
+      f(Int<I>{});
+      asm volatile("; wave %0" ::"n"(I));
+    } else {
+      by_wave<W, I + 1>(w, f);
+    }
   } else {
-    f(Int<3>{});
-    asm volatile("; wave 3");
+    f(Int<I>{});
+    asm volatile("; wave %0" ::"n"(I));
   }
 }
 template <typename F>
@@ -341,21 +451,46 @@ __device__ __forceinline__ void add_stress(T (&y)[9][MY], const T (&g)[3][M], co
 template <typename T, int O, int R>
 struct Tile {
   using D = Dim<O>;
-  static constexpr int N = D::N, SZ = 9 * N * R, M = D::M;
+  static constexpr int N = D::N, SZ = 9 * N * R, M = D::M, W = D::W;
   T* lds;
   int w, lane;
   int64_t el;      // the lane's element (the last one's for lanes past the range)
   int64_t first;   // first element of the tile
   int n_el;        // elements of the tile inside the range
   bool valid;
-  Buf<T> ph;       // constants of the tile's elements
+  const T* cst;    // the element's constants: in LDS (fused runs) ...
+  Buf<T> ph;       // ... or in memory
   unsigned ph_off;
-  T ji[3][3];
-  Mat4<T> mat;
+  // The inverse Jacobian and the material: in registers, at order 5 with
+  // fused runs read from LDS where they are used (the registers are full).
+  static constexpr bool HELD = R == 1 || O < 5;
+  T ji1[3][3];
+  Mat4<T> mat1;
 
+  static constexpr int PB = phys::block(R);
   __device__ __forceinline__ Tile(const T* phys_el, int64_t first_)
-      : first(first_), ph(phys_el + first_ / phys::kBlock * (phys::kSize * phys::kBlock), 2 * phys::kSize * phys::kBlock) {}
-  __device__ __forceinline__ T c(int k) const { return ph.load(ph_off, k * phys::kBlock * (unsigned)sizeof(T)); }
+      : first(first_), ph(phys_el + first_ / PB * (phys::kSize * PB), R == 1 ? 2 * phys::kSize * PB : 0) {}
+  // With fused runs the few elements' constants are copied to LDS before
+  // anything else: a load of them between the output stores would wait for
+  // the stores (the counter runs in order; it took half of the time).
+  __device__ __forceinline__ T c(int k) const {
+    if constexpr (R == 1)
+      return ph.load(ph_off, k * PB * (unsigned)sizeof(T));
+    else
+      return cst[k];
+  }
+  __device__ __forceinline__ T jinv(int k, int d) const {
+    if constexpr (HELD)
+      return ji1[k][d];
+    else
+      return cst[phys::kJinv + 3 * k + d];
+  }
+  __device__ __forceinline__ Mat4<T> mat() const {
+    if constexpr (HELD)
+      return mat1;
+    else
+      return {cst[phys::kLam2], cst[phys::kLam], cst[phys::kMu], cst[phys::kIrho]};
+  }
   // byte offset of the lane's column in a DOF array of the tile
   __device__ __forceinline__ unsigned column() const {
     return (unsigned)((el - first) * SZ + lane % R) * (unsigned)sizeof(T);
@@ -364,41 +499,44 @@ struct Tile {
   // the wave's modes, six bits each (where it has fewer than M, its first
   // mode again: those registers hold copies that nothing reads)
   uint64_t modes;
-  static constexpr uint64_t pack(int w) {
+  static constexpr uint64_t pack(int v) {
     uint64_t b = 0;
-    for (int j = 0; j < M; j++)
-      b |= (uint64_t)(Own<O>::mode[w][j] < 0 ? Own<O>::mode[w][0] : Own<O>::mode[w][j]) << (6 * j);
+    for (int j = 0; j < M; j++) b |= (uint64_t)D::mode(v, D::mode(v, j) < 0 ? 0 : j) << (6 * j);
     return b;
   }
   __device__ __forceinline__ int mode(int j) const { return (int)(modes >> (6 * j)) & 63; }
-  static constexpr bool every(int j) {  // every wave has a j-th mode
-    for (int w = 0; w < 4; w++)
-      if (Own<O>::mode[w][j] < 0) return false;
-    return true;
-  }
-  __device__ __forceinline__ bool has(int j) const { return every(j) || j == 0 || mode(j) != mode(0); }
+  // position j of the wave is below nn (known at compile time but for the last)
+  __device__ __forceinline__ bool has(int j, int nn) const { return (j + 1) * W <= nn || j * W + w < nn; }
 
   // the wave's modes of a DOF array (zeros past the last one)
   __device__ __forceinline__ void load(const T* __restrict__ a, T (&x)[9][M]) {
     if constexpr (R == 1) {
       // one element is contiguous: three quantities of the 64 elements at a
-      // time pass through LDS (rows of 65 columns: no bank conflicts)
+      // time pass through LDS (rows of 65 columns: no bank conflicts); every
+      // load is requested before the first is waited for
+      constexpr int PER = (kCols * 3 * N + 64 * W - 1) / (64 * W);
+      T v[3][PER];
+      const Buf<T> src(a + first * SZ, n_el * SZ);
 #pragma unroll
-      for (int qb = 0; qb < 9; qb += 3) {
+      for (int qb = 0; qb < 3; qb++)
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+          const unsigned k = threadIdx.x + i * 64 * W;
+          v[qb][i] = src.load((k / (3 * N) * SZ + k % (3 * N)) * (unsigned)sizeof(T), qb * 3 * N * (unsigned)sizeof(T));
+        }
+#pragma unroll
+      for (int qb = 0; qb < 3; qb++) {
         __syncthreads();
-        const T* src = a + first * SZ + qb * N;
-#pragma unroll 4
-        for (int i = threadIdx.x; i < kCols * 3 * N; i += 64 * kWaves) {
-          const int e = i / (3 * N), v = i % (3 * N);
-          lds[v * (kCols + 1) + e] = src[(e < n_el ? e : n_el - 1) * SZ + v];
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+          const unsigned k = threadIdx.x + i * 64 * W;
+          if (k < kCols * 3 * N) lds[k % (3 * N) * (kCols + 1) + k / (3 * N)] = v[qb][i];
         }
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < 3; q++)
 #pragma unroll
-          for (int j = 0; j < M; j++) {
-            x[qb + q][j] = lds[(q * N + mode(j)) * (kCols + 1) + lane];
-          }
+          for (int j = 0; j < M; j++) x[3 * qb + q][j] = lds[(q * N + mode(j)) * (kCols + 1) + lane];
       }
       __syncthreads();
     } else {
@@ -411,10 +549,9 @@ struct Tile {
     }
   }
 
-  // stores the wave's modes (fused runs: of the lanes with `on`); ADD: adds
-  // them to the array (one run only)
-  template <bool ADD = false>
-  __device__ __forceinline__ void store(T* __restrict__ a, const T (&x)[9][M], bool on) {
+  // stores the wave's modes (fused runs: of the lanes with `on`), SC: times sca
+  template <bool SC = false>
+  __device__ __forceinline__ void store(T* __restrict__ a, const T (&x)[9][M], bool on, T sca = T(1)) {
     if constexpr (R == 1) {
 #pragma unroll
       for (int qb = 0; qb < 9; qb += 3) {
@@ -423,52 +560,88 @@ struct Tile {
         for (int q = 0; q < 3; q++)
 #pragma unroll
           for (int j = 0; j < M; j++) {
-            if (has(j)) lds[(q * N + mode(j)) * (kCols + 1) + lane] = x[qb + q][j];
+            if (has(j, N)) lds[(q * N + mode(j)) * (kCols + 1) + lane] = SC ? sca * x[qb + q][j] : x[qb + q][j];
           }
+        constexpr int PER = (kCols * 3 * N + 64 * W - 1) / (64 * W);
+        const Buf<T> dst(a + first * SZ, n_el * SZ);
         __syncthreads();
-        T* dst = a + first * SZ + qb * N;
-#pragma unroll 4
-        for (int i = threadIdx.x; i < n_el * 3 * N; i += 64 * kWaves) {
-          const int e = i / (3 * N), v = i % (3 * N);
-          const T y = lds[v * (kCols + 1) + e];
-          dst[e * SZ + v] = ADD ? dst[e * SZ + v] + y : y;
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+          const unsigned k = threadIdx.x + i * 64 * W;
+          const bool in = k < kCols * 3 * N;
+          dst.store(in ? lds[k % (3 * N) * (kCols + 1) + k / (3 * N)] : T(0),
+                    in ? (k / (3 * N) * SZ + k % (3 * N)) * (unsigned)sizeof(T) : kSkip, qb * N * (unsigned)sizeof(T));
         }
       }
     } else {
-      static_assert(!ADD || R == 1, "fused runs start from the DOFs");
       const Buf<T> dst(a + first * SZ, n_el * SZ);
       const unsigned off = on ? column() : kSkip;
 #pragma unroll
       for (int j = 0; j < M; j++) {
-        if (!has(j)) continue;
+        if (!has(j, N)) continue;
 #pragma unroll
-        for (int q = 0; q < 9; q++) dst.store(x[q][j], off, (unsigned)((mode(j) + q * N) * R * (int)sizeof(T)));
+        for (int q = 0; q < 9; q++)
+          dst.store(SC ? sca * x[q][j] : x[q][j], off, (unsigned)((mode(j) + q * N) * R * (int)sizeof(T)));
       }
     }
   }
 
   // Publishes velocity component I and the three star-combined rows
   // sum_k j[k][d] sigma_Ik of the modes below NK.
-  template <int I, int MK>
+  template <int I, int NK, int MK>
   __device__ __forceinline__ void publish(T* l, const T (&x)[9][MK], const T (&j3)[3][3], Int<I>) const {
-    constexpr int RK = 4 * MK * kCols;
 #pragma unroll
     for (int j = 0; j < MK; j++) {
-      T* o = l + 4 * j * kCols;
+      if (!has(j, NK)) continue;
+      T* o = l + j * W * kCols;
       o[0] = x[6 + I][j];
 #pragma unroll
       for (int d = 0; d < 3; d++)
-        o[(d + 1) * RK] = dot3(j3[0][d], x[voigt(I, 0)][j], j3[1][d], x[voigt(I, 1)][j], j3[2][d], x[voigt(I, 2)][j]);
+        o[(d + 1) * NK * kCols] =
+            dot3(j3[0][d], x[voigt(I, 0)][j], j3[1][d], x[voigt(I, 1)][j], j3[2][d], x[voigt(I, 2)][j]);
     }
   }
 
-  // y += S (stiffness products of x), x on the modes below NK, y below NN:
-  // per velocity component i one published set of columns; buffers alternate
-  // (step counts them), so one barrier per component is enough.
-  template <bool CK, int NK, int NN, int MX, int MY>
-  __device__ __forceinline__ void stiffness(const T (&x)[9][MX], T (&y)[9][MY], int& step) {
-    constexpr int MK = D::own(NK), MN = D::own(NN);
-    static_assert(MX >= MK && MY >= MN, "registers of the wave's modes");
+  // Component i of S (stiffness products of x), x on the modes below NK,
+  // outputs below NN: the gradients g of velocity component i and the stress
+  // divergence v of its row; buf holds the published columns.
+  template <bool CK, int NK, int NN, bool SC = false, int MK, int MN>
+  __device__ __forceinline__ void component(int i, const T (&x)[9][MK], T* buf, T (&g)[3][MN], T (&v)[MN],
+                                            T sca = T(1)) {
+    // (opaque to the optimiser: the combined rows of every component would
+    // otherwise be formed ahead of the loop and spilled)
+    T j3[3][3];
+    auto load_j = [&]() EDGE_INLINE {
+#pragma unroll
+    for (int k = 0; k < 3; k++)
+#pragma unroll
+      for (int d = 0; d < 3; d++) {
+        j3[k][d] = SC ? sca * jinv(k, d) : jinv(k, d);
+        asm volatile("" : "+v"(j3[k][d]));
+      }
+    };
+    load_j();
+    by_axis(i, [&](auto I) EDGE_INLINE { publish<decltype(I)::value, NK>(buf + w * kCols + lane, x, j3, I); });
+    __syncthreads();
+    T p[3][MN];
+#pragma unroll
+    for (int j = 0; j < MN; j++) p[0][j] = p[1][j] = p[2][j] = v[j] = T(0);
+    by_wave<W>(w, [&](auto V) EDGE_INLINE {
+      product<StiffReads<O, CK, NK, NN, decltype(V)::value>>(buf + lane, p, v);
+    });
+    if constexpr (!HELD) load_j();
+#pragma unroll
+    for (int j = 0; j < MN; j++)
+#pragma unroll
+      for (int k = 0; k < 3; k++) g[k][j] = dot3(j3[k][0], p[0][j], j3[k][1], p[1][j], j3[k][2], p[2][j]);
+  }
+
+  // y += S (stiffness products of x): per velocity component one published
+  // set of columns; buffers alternate (step counts them), so one barrier per
+  // component is enough.
+  template <int NK, int NN, int MX, int MN>
+  __device__ __forceinline__ void stiffness(const T (&x)[9][MX], T (&y)[9][MN], int& step) {
+    constexpr int MK = D::own(NK);
     T xk[9][MK];
 #pragma unroll
     for (int q = 0; q < 9; q++)
@@ -476,35 +649,14 @@ struct Tile {
       for (int j = 0; j < MK; j++) xk[q][j] = x[q][j];
 #pragma unroll 1
     for (int i = 0; i < 3; i++) {
-      T* buf = lds + (step & 1) * D::CROWS * kCols;
+      T g[3][MN], v[MN];
+      component<true, NK, NN>(i, xk, lds + (step & 1) * D::CROWS * kCols, g, v);
       step++;
-      // (opaque to the optimiser: the combined rows of every component would
-      // otherwise be formed ahead of the loop and spilled)
-      T j3[3][3];
-#pragma unroll
-      for (int k = 0; k < 3; k++)
-#pragma unroll
-        for (int d = 0; d < 3; d++) {
-          j3[k][d] = ji[k][d];
-          asm volatile("" : "+v"(j3[k][d]));
-        }
-      by_axis(i, [&](auto I) EDGE_INLINE { publish(buf + w * kCols + lane, xk, j3, I); });
-      __syncthreads();
-      T p[3][MN], v[MN];
-#pragma unroll
-      for (int j = 0; j < MN; j++) p[0][j] = p[1][j] = p[2][j] = v[j] = T(0);
-      by_wave(w, [&](auto W) EDGE_INLINE {
-        stiff_mul<O, CK, NK, NN, decltype(W)::value>(buf + lane, p, v, std::make_integer_sequence<int, NK>{});
-      });
-      T g[3][MN];
-#pragma unroll
-      for (int k = 0; k < 3; k++)
-#pragma unroll
-        for (int j = 0; j < MN; j++) g[k][j] = dot3(ji[k][0], p[0][j], ji[k][1], p[1][j], ji[k][2], p[2][j]);
+      const Mat4<T> m = mat();
       by_axis(i, [&](auto I) EDGE_INLINE {
-        add_stress<decltype(I)::value>(y, g, mat);
+        add_stress<decltype(I)::value>(y, g, m);
 #pragma unroll
-        for (int j = 0; j < MN; j++) y[6 + decltype(I)::value][j] = fma_(mat.irho, v[j], y[6 + decltype(I)::value][j]);
+        for (int j = 0; j < MN; j++) y[6 + decltype(I)::value][j] = fma_(m.irho, v[j], y[6 + decltype(I)::value][j]);
       });
     }
   }
@@ -520,7 +672,7 @@ struct Tile {
       for (int q = 0; q < 9; q++)
 #pragma unroll
         for (int j = 0; j < MN; j++) y[q][j] = T(0);
-      stiffness<true, NK, NN>(x, y, step);
+      stiffness<NK, NN>(x, y, step);
       sca *= dt / T(DE + 1);
 #pragma unroll
       for (int q = 0; q < 9; q++)
@@ -530,64 +682,101 @@ struct Tile {
     }
   }
 
-  // acc += the lifted flux of the w of all faces in the first WROWS rows of
-  // LDS; KC: phys::kOwn (the element's side) or phys::kOth (the other side)
+  // Component i of the faces' lifted flux, the w of all faces in the first
+  // WROWS rows of LDS: velocities into acc, gradients into g; KC: phys::kOwn
+  // (the element's side) or phys::kOth (the other side)
   template <int KC>
-  __device__ __forceinline__ void lifts(T (&acc)[9][M]) {
+  __device__ __forceinline__ void lift(int i, T (&acc)[9][M], T (&g)[3][M]) {
+    const T* li = lds + i * D::NF * kCols + lane;
+    each(
+        [&](auto F) EDGE_INLINE {
+          constexpr int f = decltype(F)::value;
+          T u[M], n[3], sn[3], e[3];
+#pragma unroll
+          for (int k = 0; k < 3; k++) n[k] = face(f, phys::kNrm + k);
+#pragma unroll
+          for (int k = 0; k < 3; k++) sn[k] = face(f, phys::kScN + k);
+          const T c1 = face(f, KC + 1), c0 = face(f, KC);
+#pragma unroll
+          for (int j = 0; j < M; j++) u[j] = T(0);
+          by_wave<W>(w, [&](auto V) EDGE_INLINE {
+            product<LiftReads<O, f, decltype(V)::value>>(li + 3 * f * D::NF * kCols, u);
+          });
+          const T ni = c1 * (i == 0 ? n[0] : i == 1 ? n[1] : n[2]);
+#pragma unroll
+          for (int k = 0; k < 3; k++) e[k] = fma_(ni, n[k], k == i ? c0 : T(0));
+#pragma unroll
+          for (int k = 0; k < 3; k++)
+#pragma unroll
+            for (int j = 0; j < M; j++) {
+              g[k][j] = fma_(sn[k], u[j], g[k][j]);
+              acc[6 + k][j] = fma_(e[k], u[j], acc[6 + k][j]);
+            }
+        },
+        std::make_integer_sequence<int, 4>{});
+  }
+
+  // acc += the neighbours' side of the faces' flux
+  __device__ __forceinline__ void neigh(T (&acc)[9][M]) {
 #pragma unroll 1
     for (int i = 0; i < 3; i++) {
       T g[3][M];
 #pragma unroll
       for (int j = 0; j < M; j++) g[0][j] = g[1][j] = g[2][j] = T(0);
-      const T* li = lds + i * D::FR * kCols + lane;
-      each(
-          [&](auto F) EDGE_INLINE {
-            constexpr int f = decltype(F)::value;
-            T u[M], n[3], sn[3], e[3];
-#pragma unroll
-            for (int k = 0; k < 3; k++) n[k] = face(f, phys::kNrm + k);
-#pragma unroll
-            for (int k = 0; k < 3; k++) sn[k] = face(f, phys::kScN + k);
-            const T c1 = face(f, KC + 1), c0 = face(f, KC);
-#pragma unroll
-            for (int j = 0; j < M; j++) u[j] = T(0);
-            by_wave(w, [&](auto W) EDGE_INLINE {
-              lift_mul<O, f, decltype(W)::value>(li + 3 * f * D::FR * kCols, u,
-                                                 std::make_integer_sequence<int, D::NF>{});
-            });
-            const T ni = c1 * (i == 0 ? n[0] : i == 1 ? n[1] : n[2]);
-#pragma unroll
-            for (int k = 0; k < 3; k++) e[k] = fma_(ni, n[k], k == i ? c0 : T(0));
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-              const T m = sn[k];
-#pragma unroll
-              for (int j = 0; j < M; j++) {
-                g[k][j] = fma_(m, u[j], g[k][j]);
-                acc[6 + k][j] = fma_(e[k], u[j], acc[6 + k][j]);
-              }
-            }
-          },
-          std::make_integer_sequence<int, 4>{});
-      by_axis(i, [&](auto I) EDGE_INLINE { add_stress<decltype(I)::value>(acc, g, mat); });
+      lift<phys::kOth>(i, acc, g);
+      const Mat4<T> m = mat();
+      by_axis(i, [&](auto I) EDGE_INLINE { add_stress<decltype(I)::value>(acc, g, m); });
     }
   }
 
-  // w of every face in the element's face coordinates: to LDS rows
-  // [f][i][FR] and to the projections proj
-  __device__ __forceinline__ void project(const T (&t)[9][M], T* __restrict__ proj) {
+  // acc += volume integral and the element's side of the faces' flux, one
+  // velocity component of both at a time (t: tInt / dt)
+  __device__ __forceinline__ void space(const T (&t)[9][M], T (&acc)[9][M], T dt) {
+
+    constexpr int NK = n_modes(O - 1), MK = D::own(NK);
+    T* buf = lds + D::WROWS * kCols;
+    T xk[9][MK];
+#pragma unroll
+    for (int q = 0; q < 9; q++)
+#pragma unroll
+      for (int j = 0; j < MK; j++) xk[q][j] = t[q][j];
+#pragma unroll 1
+    for (int i = 0; i < 3; i++) {
+      T g[3][M], v[M];
+      __syncthreads();  // the previous columns have been read
+      component<false, NK, D::N, true>(i, xk, buf, g, v, dt);
+      const T irho = mat().irho;
+      by_axis(i, [&](auto I) EDGE_INLINE {
+#pragma unroll
+        for (int j = 0; j < M; j++) acc[6 + decltype(I)::value][j] = fma_(irho, v[j], acc[6 + decltype(I)::value][j]);
+      });
+      lift<phys::kOwn>(i, acc, g);
+      const Mat4<T> m = mat();
+      by_axis(i, [&](auto I) EDGE_INLINE { add_stress<decltype(I)::value>(acc, g, m); });
+    }
+  }
+
+  // w of every face in the element's face coordinates, to LDS rows [f][i][NF]
+  // (t: tInt / dt)
+  __device__ __forceinline__ void project(const T (&t)[9][M], T dt) {
     T* cols = lds + D::WROWS * kCols;
     T* own = cols + w * kCols + lane;
+    T next[7];  // the next face's normal and factors, a face ahead
+#pragma unroll
+    for (int k = 0; k < 7; k++) next[k] = face(0, k);
 #pragma unroll 1
     for (int f = 0; f < 4; f++) {
       T n[3], a[4];
 #pragma unroll
-      for (int k = 0; k < 3; k++) n[k] = face(f, phys::kNrm + k);
+      for (int k = 0; k < 3; k++) n[k] = next[phys::kNrm + k];
 #pragma unroll
-      for (int k = 0; k < 4; k++) a[k] = face(f, phys::kPrj + k);
+      for (int k = 0; k < 4; k++) a[k] = dt * next[phys::kPrj + k];
+#pragma unroll
+      for (int k = 0; k < 7; k++) next[k] = face(f < 3 ? f + 1 : 3, k);
       __syncthreads();  // the previous columns have been read
 #pragma unroll
       for (int j = 0; j < M; j++) {
+        if (!has(j, N)) continue;
         T tr[3];
 #pragma unroll
         for (int k = 0; k < 3; k++)
@@ -596,7 +785,7 @@ struct Tile {
         const T tn = dot3(n[0], tr[0], n[1], tr[1], n[2], tr[2]);
         const T b = fma_(a[2], vn, -(a[3] * tn));
 #pragma unroll
-        for (int k = 0; k < 3; k++) own[(k * 4 * M + 4 * j) * kCols] = fma_(n[k], b, fma_(a[0], t[6 + k][j], -(a[1] * tr[k])));
+        for (int k = 0; k < 3; k++) own[(k * N + j * W) * kCols] = fma_(n[k], b, fma_(a[0], t[6 + k][j], -(a[1] * tr[k])));
       }
       __syncthreads();
 #pragma unroll 1
@@ -604,74 +793,89 @@ struct Tile {
         T u[D::MF];
 #pragma unroll
         for (int j = 0; j < D::MF; j++) u[j] = T(0);
-        const T* li = cols + i * 4 * M * kCols + lane;
-        by_wave(w, [&](auto W) EDGE_INLINE {
-          constexpr int wv = decltype(W)::value;
-          using K = std::make_integer_sequence<int, N>;
+        const T* li = cols + i * N * kCols + lane;
+        by_wave<W>(w, [&](auto V) EDGE_INLINE {
+          constexpr int wv = decltype(V)::value;
           if (f == 0)
-            project_mul<O, 0, wv>(li, u, K{});
+            product<ProjectReads<O, 0, wv>>(li, u);
           else if (f == 1)
-            project_mul<O, 1, wv>(li, u, K{});
+            product<ProjectReads<O, 1, wv>>(li, u);
           else if (f == 2)
-            project_mul<O, 2, wv>(li, u, K{});
+            product<ProjectReads<O, 2, wv>>(li, u);
           else
-            project_mul<O, 3, wv>(li, u, K{});
+            product<ProjectReads<O, 3, wv>>(li, u);
         });
-        T* o = lds + ((f * 3 + i) * D::FR + w) * kCols + lane;
+        T* o = lds + ((f * 3 + i) * D::NF + w) * kCols + lane;
 #pragma unroll
-        for (int j = 0; j < D::MF; j++) o[4 * j * kCols] = u[j];
-        if (valid) {
-          T* g = proj + ((((el * 4 + f) * 12 + i * 4 + w) * R) + lane % R) * D::MF;
-#pragma unroll
-          for (int j = 0; j < D::MF; j++) g[j] = u[j];
-        }
+        for (int j = 0; j < D::MF; j++)
+          if (has(j, D::NF)) o[j * W * kCols] = u[j];
       }
     }
   }
 
+  // the faces' w from LDS to the projections of the tile's elements, four
+  // values per store: vector v of 4 NV goes to wave v % W
+  typedef T vec4 __attribute__((ext_vector_type(4)));
+  static constexpr int NV = sp_proj_vectors(O);
+  __device__ __forceinline__ void send(T* __restrict__ proj) const {
+    if (!valid) return;
+    vec4* o = reinterpret_cast<vec4*>(proj) + el * 4 * NV * R + lane % R;
+#pragma unroll
+    for (int f = 0; f < 4; f++)
+#pragma unroll
+      for (int v = 0; v < (NV + W - 1) / W; v++) {
+        const int k = v * W + w;
+        if (k >= NV) continue;
+        vec4 x;
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = lds[(f * 3 * D::NF + (4 * k + j < 3 * D::NF ? 4 * k + j : 0)) * kCols + lane];
+        o[(f * NV + k) * R] = x;
+      }
+  }
+
   // the neighbours' w (projections p), taken to the element's face
-  // coordinates, to LDS rows [f][i][FR]: wave w takes face w
-  __device__ __forceinline__ void receive(const SolverDev<T>& s, const T* __restrict__ rot, const T* __restrict__ p) {
-    const int32_t slot = s.rcv[el * 4 + w];
-    const int fm = s.nb.fmat[el * 4 + w];
-    const T* rv = rot + (fm < 4 ? 0 : 1 + (fm - 4) / 4) * phys::kRotPad;
-    const T* src = p + (((int64_t)(slot < 0 ? 0 : slot) * 12 * R) + lane % R) * D::MF;
-    T* dst = lds + w * 3 * D::FR * kCols + lane;
-    T u[3][D::FR];
+  // coordinates, to LDS rows [f][i][NF]: wave f takes face f (slot, fm: its
+  // projection slot and flux matrix)
+  __device__ __forceinline__ void receive(int32_t slot, int fm, const T* __restrict__ rot, const T* __restrict__ p,
+                                          T (&u)[4 * NV], T (&r)[phys::kRotPad]) const {
+    const vec4* src = reinterpret_cast<const vec4*>(p) + (int64_t)(slot < 0 ? 0 : slot) * NV * R + lane % R;
+    const vec4* rv = reinterpret_cast<const vec4*>(rot) + (fm < 4 ? 0 : 1 + (fm - 4) / 4) * (phys::kRotPad / 4);
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      const vec4 x = src[v * R];
+#pragma unroll
+      for (int j = 0; j < 4; j++) u[4 * v + j] = x[j];
+    }
+#pragma unroll
+    for (int v = 0; v < (phys::rot_off(O) + 3) / 4; v++) {
+      const vec4 x = rv[v];
+#pragma unroll
+      for (int j = 0; j < 4; j++) r[4 * v + j] = x[j];
+    }
+  }
+  __device__ __forceinline__ void rotate(int32_t slot, const T (&u)[4 * NV], const T (&r)[phys::kRotPad]) {
+    T* dst = lds + w * 3 * D::NF * kCols + lane;
 #pragma unroll
     for (int i = 0; i < 3; i++)
-#pragma unroll
-      for (int o = 0; o < 4; o++)
-#pragma unroll
-        for (int j = 0; j < D::MF; j++) u[i][4 * j + o] = src[((i * 4 + o) * R) * D::MF + j];
-    if (slot < 0) {  // outflow, fault and time-step interfaces: nothing
-#pragma unroll
-      for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < D::FR; j++) u[i][j] = T(0);
-    }
-    each(
-        [&](auto P) EDGE_INLINE {
-          constexpr int p0 = decltype(P)::value, lo = p0 * (p0 + 1) / 2;
-          T r[p0 + 1][p0 + 1];
-#pragma unroll
-          for (int k = 0; k <= p0; k++)
-#pragma unroll
-            for (int m = 0; m <= p0; m++) r[k][m] = rv[phys::rot_off(p0) + k * (p0 + 1) + m];
-          each(
-              [&](auto Mo) EDGE_INLINE {
-                constexpr int m = decltype(Mo)::value;
-#pragma unroll
-                for (int i = 0; i < 3; i++) {
+      each(
+          [&](auto P) EDGE_INLINE {
+            constexpr int p0 = decltype(P)::value, lo = p0 * (p0 + 1) / 2;
+            each(
+                [&](auto Mo) EDGE_INLINE {
+                  constexpr int m = decltype(Mo)::value;
                   T v = T(0);
-                  each([&](auto K) EDGE_INLINE { v = fma_(r[decltype(K)::value][m], u[i][D::face_row(lo + decltype(K)::value)], v); },
-                       std::make_integer_sequence<int, p0 + 1>{});
-                  dst[(i * D::FR + D::face_row(lo + m)) * kCols] = v;
-                }
-              },
-              std::make_integer_sequence<int, p0 + 1>{});
-        },
-        std::make_integer_sequence<int, O>{});
+                  each(
+                      [&](auto K) EDGE_INLINE {
+                        constexpr int k = decltype(K)::value;
+                        v = fma_(r[phys::rot_off(p0) + k * (p0 + 1) + m], u[i * D::NF + D::face_row(lo + k)], v);
+                      },
+                      std::make_integer_sequence<int, p0 + 1>{});
+                  // (no slot: an outflow, fault or time-step interface face gives nothing)
+                  dst[(i * D::NF + D::face_row(lo + m)) * kCols] = slot < 0 ? T(0) : v;
+                },
+                std::make_integer_sequence<int, p0 + 1>{});
+          },
+          std::make_integer_sequence<int, O>{});
   }
 };
 
@@ -681,66 +885,84 @@ __device__ __forceinline__ int64_t tile_index(int64_t n, bool xcd) {
   return xcd ? (b & 7) * chunk + (b >> 3) : b;
 }
 
+// Waves per SIMD the registers are limited for: what the tiles' LDS allows.
+constexpr int waves_per_simd(int order) { return order == 5 ? 2 : 3; }
+
 // NB: the neighbouring surface integral from the projections proj_in; LOC:
 // the local step (projections to x.proj).  Both: the neighbour step of the
-// previous time step first, its DOFs go back to global memory (and to s.tap
-// for the elements s.tap_on marks) and are read again for the output.
+// previous time step first (its DOFs also go to s.tap for the elements
+// s.tap_on marks).
 template <typename T, int O, int R, bool NB, bool LOC>
-__global__ __launch_bounds__(64 * kWaves) __attribute__((amdgpu_waves_per_eu(2)))
-void k_sparse(SolverDev<T> s, SpDev<T> x, int64_t first, int64_t n, T dt, T* __restrict__ dofs, T* __restrict__ t_int,
+__global__ __launch_bounds__(64 * kWaves, waves_per_simd(O)) void k_sparse(SolverDev<T> s, SpDev<T> x, int64_t first, int64_t n, T dt, T* __restrict__ dofs, T* __restrict__ t_int,
               const T* __restrict__ proj_in) {
   using D = Dim<O>;
-  constexpr int M = D::M, E = kCols / R;
+  constexpr int M = D::M, W = D::W, E = kCols / R;
   constexpr int STAGE = R == 1 ? (3 * D::N * (kCols + 1) + kCols - 1) / kCols : 0;
   constexpr int ROWS = !LOC ? D::WROWS : D::LROWS;
-  __shared__ T lds[(ROWS > STAGE ? ROWS : STAGE) * kCols];
+  __shared__ T lds[(ROWS > STAGE ? ROWS : STAGE) * kCols + (R == 1 ? 0 : E * phys::kSize)];
   const int64_t nt = (n + E - 1) / E, tile = tile_index(nt, s.xcd_map);
   if (tile >= nt) return;
   Tile<T, O, R> b(x.phys, first + tile * E);
   b.lds = lds;
   b.w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   b.lane = threadIdx.x & 63;
-  {
-    using Ti = Tile<T, O, R>;
-    constexpr uint64_t m0 = Ti::pack(0), m1 = Ti::pack(1), m2 = Ti::pack(2), m3 = Ti::pack(3);
-    b.modes = b.w == 0 ? m0 : b.w == 1 ? m1 : b.w == 2 ? m2 : m3;
-  }
+  by_wave<W>(b.w, [&](auto V) EDGE_INLINE {
+    constexpr uint64_t m = Tile<T, O, R>::pack(decltype(V)::value);
+    b.modes = m;
+  });
   const int64_t left = n - tile * E;
   b.n_el = left < E ? (int)left : E;
   const int e = b.lane / R;
   b.valid = e < b.n_el;
   b.el = b.first + (b.valid ? e : b.n_el - 1);
-  b.ph_off = (unsigned)((b.el / phys::kBlock - b.first / phys::kBlock) * (phys::kSize * phys::kBlock) +
-                        b.el % phys::kBlock) * (unsigned)sizeof(T);
-  b.mat = {b.c(phys::kLam2), b.c(phys::kLam), b.c(phys::kMu), b.c(phys::kIrho)};
+  // the neighbours first (their projections are the longest chain of loads)
+  int32_t slot = -1;
+  int fm = 0;
+  if constexpr (NB) {
+    slot = s.rcv[b.el * 4 + b.w];
+    fm = s.nb.fmat[b.el * 4 + b.w];
+  }
+  if constexpr (R == 1) {
+    constexpr int PB = phys::block(R);
+    b.ph_off = (unsigned)((b.el / PB - b.first / PB) * (phys::kSize * PB) + b.el % PB) * (unsigned)sizeof(T);
+  } else {
+    constexpr int C0 = (ROWS > STAGE ? ROWS : STAGE) * kCols;
+    for (int i = threadIdx.x; i < b.n_el * phys::kSize; i += 64 * W)
+      lds[C0 + i] = x.phys[b.first * phys::kSize + i];
+    b.cst = lds + C0 + (int)(b.el - b.first) * phys::kSize;
+  }
   T acc[9][M];
-  auto start = [&]() EDGE_INLINE {  // one run: the DOFs are added where the update is stored
-    if constexpr (R == 1) {
+  auto constants = [&]() EDGE_INLINE {
+    if constexpr (Tile<T, O, R>::HELD) {
+      b.mat1 = {b.c(phys::kLam2), b.c(phys::kLam), b.c(phys::kMu), b.c(phys::kIrho)};
 #pragma unroll
-      for (int q = 0; q < 9; q++)
+      for (int k = 0; k < 3; k++)
 #pragma unroll
-        for (int j = 0; j < M; j++) acc[q][j] = T(0);
-    } else {
-      b.load(dofs, acc);
+        for (int d = 0; d < 3; d++) b.ji1[k][d] = b.c(phys::kJinv + 3 * k + d);
     }
   };
   if constexpr (NB) {
-    start();
-    b.receive(s, x.rot, proj_in);
+    T u[4 * Tile<T, O, R>::NV], r[phys::kRotPad];
+    b.receive(slot, fm, x.rot, proj_in, u, r);
+    b.load(dofs, acc);
+    b.rotate(slot, u, r);
     __syncthreads();
-    b.template lifts<phys::kOth>(acc);
-    b.template store<R == 1>(dofs, acc, b.valid);
+    constants();
+    b.neigh(acc);
     if constexpr (LOC) {
-      if (s.tap) b.store(s.tap, acc, b.valid && s.tap_on[b.el]);
+      if (R > 1 && s.tap) b.store(s.tap, acc, b.valid && s.tap_on[b.el]);
       __syncthreads();
+    } else {
+      b.store(dofs, acc, b.valid);
     }
   }
   if constexpr (LOC) {
-#pragma unroll
-    for (int k = 0; k < 3; k++)
-#pragma unroll
-      for (int d = 0; d < 3; d++) b.ji[k][d] = b.c(phys::kJinv + 3 * k + d);
-    T t[9][M];
+    // t = Q, then the time-integrated DOFs over dt.  The CK leaves the
+    // highest modes as they are, so a copy of the others keeps Q in registers
+    // until the volume integral (reading it again, and with NB writing it
+    // first, was a third of the memory traffic).
+    constexpr int NL = n_modes(O - 1), ML = D::own(NL);
+    T t[9][M], low[9][ML];
     if constexpr (NB) {
 #pragma unroll
       for (int q = 0; q < 9; q++)
@@ -748,22 +970,32 @@ void k_sparse(SolverDev<T> s, SpDev<T> x, int64_t first, int64_t n, T dt, T* __r
         for (int j = 0; j < M; j++) t[q][j] = acc[q][j];
     } else {
       b.load(dofs, t);
+      if constexpr (R > 1) __syncthreads();  // the constants are in LDS
+      constants();
     }
-    int step = 0;
-    b.template ck<1>(t, t, dt, T(1), step);
 #pragma unroll
     for (int q = 0; q < 9; q++)
 #pragma unroll
-      for (int j = 0; j < M; j++) t[q][j] *= dt;
-    if constexpr (R == 1) __syncthreads();  // (the staging buffer is the products' buffer)
-    b.store(t_int, t, b.valid);
-    if constexpr (R == 1) __syncthreads();
-    start();
-    b.template stiffness<false, n_modes(O - 1), D::N>(t, acc, step);
-    b.project(t, x.proj);
-    __syncthreads();
-    b.template lifts<phys::kOwn>(acc);
-    b.template store<R == 1>(dofs, acc, b.valid);
+      for (int j = 0; j < ML; j++) low[q][j] = t[q][j];
+    int step = 0;
+    b.template ck<1>(t, t, dt, T(1), step);
+    // tInt: all of it, or of the elements in x.need; the projections (which
+    // load nothing) run while it is written
+    const bool on = b.valid && (x.tint || (x.need && x.need[b.el]));
+    if constexpr (R > 1)
+      if (__any(on)) b.template store<true>(t_int, t, on, dt);
+    b.project(t, dt);
+#pragma unroll
+    for (int q = 0; q < 9; q++)
+#pragma unroll
+      for (int j = 0; j < M; j++) acc[q][j] = j < ML ? low[q][j < ML ? j : 0] : t[q][j];
+    b.space(t, acc, dt);
+    b.send(x.proj);
+    if constexpr (R == 1) {
+      if (x.tint || x.need) b.template store<true>(t_int, t, on, dt);
+      __syncthreads();
+    }
+    b.store(dofs, acc, b.valid);
   }
 }
 
@@ -783,8 +1015,7 @@ int by_op(int op, const SolverDev<T>& s, const SpDev<T>& x, int64_t first, int64
           const T* proj_in, hipStream_t st) {
   if (op == kSpLocal) return launch<T, O, R, false, true>(s, x, first, n, dt, dofs, t_int, proj_in, st);
   if (op == kSpNeigh) return launch<T, O, R, true, false>(s, x, first, n, dt, dofs, t_int, proj_in, st);
-  if constexpr (R > 1) return launch<T, O, R, true, true>(s, x, first, n, dt, dofs, t_int, proj_in, st);
-  return fail(EDGE_ERR_UNSUPPORTED, "fused sparse step: 8 or 16 runs");
+  return launch<T, O, R, true, true>(s, x, first, n, dt, dofs, t_int, proj_in, st);
 }
 
 }  // namespace

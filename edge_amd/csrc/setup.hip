@@ -47,7 +47,7 @@ __device__ void load_ve(const double* crds, const int64_t* el_ve, int64_t el, do
 
 template <typename T>
 __global__ void k_star(int64_t n_el, const double* crds, const int64_t* el_ve, const double* rho,
-                       const double* lam, const double* mu, T* star, double* jdet, T* star_a, T* ph, int* bad) {
+                       const double* lam, const double* mu, T* star, double* jdet, T* star_a, T* ph, int pb, int* bad) {
   const int64_t el = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (el >= n_el) return;
   double ve[12], det, ji[9];
@@ -68,12 +68,12 @@ __global__ void k_star(int64_t n_el, const double* crds, const int64_t* el_ve, c
       for (int e = 0; e < 8; e++) s[d * 81 + rc[k][e][0] * 9 + rc[k][e][1]] += va[k][e] * ji[k * 3 + d];
   for (int i = 0; i < 243; i++) star[el * 243 + i] = (T)s[i];
   if (ph) {
-    T* o = ph + el / phys::kBlock * (int64_t)(phys::kSize * phys::kBlock) + el % phys::kBlock;
-    for (int i = 0; i < 9; i++) o[(phys::kJinv + i) * phys::kBlock] = (T)ji[i];
-    o[phys::kLam2 * phys::kBlock] = (T)lp;
-    o[phys::kLam * phys::kBlock] = (T)l;
-    o[phys::kMu * phys::kBlock] = (T)m;
-    o[phys::kIrho * phys::kBlock] = (T)ir;
+    T* o = ph + el / pb * (int64_t)(phys::kSize * pb) + el % pb;
+    for (int i = 0; i < 9; i++) o[(phys::kJinv + i) * pb] = (T)ji[i];
+    o[phys::kLam2 * pb] = (T)lp;
+    o[phys::kLam * pb] = (T)l;
+    o[phys::kMu * pb] = (T)m;
+    o[phys::kIrho * pb] = (T)ir;
   }
   if (star_a) {
     // anelastic star matrices [3][6][3]: memory variables from the velocity
@@ -323,7 +323,7 @@ template <typename T>
 __global__ void k_flux_solvers(int64_t n_fa, int64_t n_el, const int64_t* fa_el, const int64_t* el_fa,
                                const int32_t* fa_type, const double* normals, const double* tangents,
                                const double* areas, const double* jdet, const double* rho, const double* lam,
-                               const double* mu, T* fs, T* fsf, T* fs_a, T* fsfa, T* ph, int* bad) {
+                               const double* mu, T* fs, T* fsf, T* fs_a, T* fsfa, T* ph, int pb, int* bad) {
   const int64_t fa = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (fa >= n_fa) return;
   const int64_t eL = fa_el[fa * 2], eR = fa_el[fa * 2 + 1];
@@ -389,12 +389,11 @@ __global__ void k_flux_solvers(int64_t n_fa, int64_t n_el, const int64_t* fa_el,
     const double zp1 = sqrt((l1 + 2 * m1) * r1), zs1 = sqrt(m1 * r1), zp2 = sqrt((l2 + 2 * m2) * r2),
                  zs2 = sqrt(m2 * r2), ap = 1.0 / (zp1 + zp2), as = 1.0 / (zs1 + zs2);
     const double sc = fault ? 0.0 : -2.0 * areas[fa] / jdet[e];
-    T* o = ph + e / phys::kBlock * (int64_t)(phys::kSize * phys::kBlock) + e % phys::kBlock +
-           (phys::kFace + phys::kPerFace * f) * phys::kBlock;
+    T* o = ph + e / pb * (int64_t)(phys::kSize * pb) + e % pb + (phys::kFace + phys::kPerFace * f) * pb;
     const double v[phys::kPerFace] = {sign * n[0], sign * n[1], sign * n[2], zs1 * as, as, zp1 * ap - zs1 * as,
                                       ap - as, sc * sign * n[0], sc * sign * n[1], sc * sign * n[2], sc * zs2 / r1,
                                       sc * (zp2 - zs2) / r1, -sc * zs1 / r1, -sc * (zp1 - zs1) / r1};
-    for (int i = 0; i < phys::kPerFace; i++) o[i * phys::kBlock] = (T)v[i];
+    for (int i = 0; i < phys::kPerFace; i++) o[i * pb] = (T)v[i];
   };
   emit_phys(eL, fL, 1.0, rL, lL, mL, rR, lR, mR);
   if (eR >= 0) emit_phys(eR, fR, -1.0, rR, lR, mR, rL, lL, mL);
@@ -413,7 +412,7 @@ __global__ void k_flux_solvers(int64_t n_fa, int64_t n_el, const int64_t* fa_el,
 
 template <typename T>
 int build_setup(const SetupInput& in, T* d_star, T* d_fs, double* d_jdet, T* d_fsf, bool* rank3, T* d_star_a,
-                T* d_fs_a, T* d_fsfa, T* d_phys, hipStream_t st) {
+                T* d_fs_a, T* d_fsfa, T* d_phys, int phys_block, hipStream_t st) {
   double *d_crds = nullptr, *d_rho = nullptr, *d_lam = nullptr, *d_mu = nullptr, *d_nrm = nullptr,
          *d_tan = nullptr, *d_area = nullptr;
   int64_t *d_elve = nullptr, *d_fael = nullptr, *d_elfa = nullptr;
@@ -463,11 +462,11 @@ int build_setup(const SetupInput& in, T* d_star, T* d_fs, double* d_jdet, T* d_f
   if (d_fs_a) EDGE_SETUP_TRY(hipMemsetAsync(d_fs_a, 0xFF, sizeof(T) * 2 * 4 * 54 * ne, st));
   const int bs = 128;
   hipLaunchKernelGGL(k_star<T>, dim3((unsigned)((ne + bs - 1) / bs)), dim3(bs), 0, st, ne, d_crds, d_elve, d_rho,
-                     d_lam, d_mu, d_star, d_jdet, d_star_a, d_phys, d_bad);
+                     d_lam, d_mu, d_star, d_jdet, d_star_a, d_phys, phys_block, d_bad);
   EDGE_SETUP_TRY(hipGetLastError());
   hipLaunchKernelGGL(k_flux_solvers<T>, dim3((unsigned)((nf + bs - 1) / bs)), dim3(bs), 0, st, nf, ne, d_fael,
                      d_elfa, d_type, d_nrm, d_tan, d_area, d_jdet, d_rho, d_lam, d_mu, d_fs, d_fsf, d_fs_a, d_fsfa,
-                     d_phys, d_bad);
+                     d_phys, phys_block, d_bad);
   EDGE_SETUP_TRY(hipGetLastError());
   int bad = 0;
   EDGE_SETUP_TRY(hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, st));
@@ -482,9 +481,9 @@ int build_setup(const SetupInput& in, T* d_star, T* d_fs, double* d_jdet, T* d_f
 }
 
 template int build_setup<double>(const SetupInput&, double*, double*, double*, double*, bool*, double*, double*,
-                                  double*, double*, hipStream_t);
+                                  double*, double*, int, hipStream_t);
 template int build_setup<float>(const SetupInput&, float*, float*, double*, float*, bool*, float*, float*, float*,
-                                 float*, hipStream_t);
+                                 float*, int, hipStream_t);
 
 template <typename T>
 int factor_flux_solvers(const double* h_fs, int64_t n_mats, T* d_fsf, bool* rank3) {

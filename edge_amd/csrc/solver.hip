@@ -75,6 +75,7 @@ struct edge_el_solver {
   bool faces_agree = true; // every interior face's two elements are each other's neighbours
   void* sp_phys = nullptr;
   void* sp_rot = nullptr;
+  uint8_t* sp_need = nullptr;  // [nEl] elements on a fault: its phase reads their tInt in every step
   // viscoelastic solvers
   int n_rms = 0;
   void* rfs = nullptr;       // [n_rms]
@@ -377,6 +378,12 @@ int finish_sp(edge_el_solver* s) {
   const int rc = f32 ? upload_as<float>(pk, &s->sp_rot) : upload_as<double>(pk, &s->sp_rot);
   if (rc) return rc;
   s->sp_ok = true;
+  if (!s->h_fault_ef.empty()) {
+    std::vector<uint8_t> need(s->n_el, 0);
+    for (const int64_t ef : s->h_fault_ef) need[ef / 4] = 1;
+    EDGE_HIP_TRY(hipMalloc(&s->sp_need, s->n_el));
+    EDGE_HIP_TRY(hipMemcpy(s->sp_need, need.data(), s->n_el, hipMemcpyHostToDevice));
+  }
   if (s->cfg.kernel == 0 && s->kernel == 1) {
     EDGE_HIP_TRY(hipMalloc(&s->proj, s->real_bytes * edge::sp_proj_values(s->cfg.order, s->cfg.n_runs) * s->n_el));
     s->kernel = 5;
@@ -668,6 +675,35 @@ bool fused_active(const edge_el_solver* s) {
          s->cfg.n_runs == (s->n_rms == 0 ? 16 : 8);
 }
 
+// The sparse kernels' form: every run count.
+bool sp_fuses(const edge_el_solver* s) { return sp_active(s) && (s->kernel == 5 || fused_active(s)); }
+
+size_t proj_alt_bytes(const edge_el_solver* s) {
+  const size_t sp = s->real_bytes * edge::sp_proj_values(s->cfg.order, s->cfg.n_runs) * s->n_el;
+  return s->kernel == 2 ? std::max(sp, sizeof(float) * 4 * 768 * s->n_el) : sp;
+}
+
+// One local launch, n_steps - 1 fused ones and the last neighbour launch;
+// only the last step's tInt is the caller's (and, in every step, that of
+// elements on a fault).
+template <typename T>
+int sp_steps(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* t_int, hipStream_t st) {
+  auto d = dev_view<T>(s);
+  auto x = sp_view<T>(s);
+  if (s->kernel == 5) d.tap = nullptr;  // taps: the 16-run fused launches
+  T* P[2] = {x.proj, static_cast<T*>(s->proj_alt)};
+  x.need = s->fault ? s->sp_need : nullptr;
+  int rc = EDGE_OK;
+  for (int64_t k = 0; k < n_steps && rc == EDGE_OK; k++) {
+    x.proj = P[k % 2];
+    x.tint = k + 1 == n_steps || (s->fault && !s->sp_need);
+    rc = k == 0 ? edge::launch_local_sp<T>(d, x, 0, s->n_el, (T)dt, (T*)dofs, (T*)t_int, st)
+                : edge::launch_fused_sp<T>(d, x, (T)dt, P[(k - 1) % 2], (T*)dofs, (T*)t_int, st);
+    if (rc == EDGE_OK && s->fault) rc = edge::fault_apply(s->fault, dt, t_int, dofs, st);
+  }
+  return rc ? rc : edge::launch_neigh_sp<T>(d, x, 0, s->n_el, (T*)dofs, st);
+}
+
 // The viscoelastic form of fused_steps (FP32, 8 runs): the same launch
 // sequence with the anelastic DOFs.
 int fused_steps_a(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* dofs_a, void* t_int,
@@ -691,30 +727,19 @@ int fused_steps(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void*
                 hipStream_t st) {
   // the fused kernels are the FP32 MFMA kernels of 16 elastic or 8
   // viscoelastic runs: nothing else may get here
-  if (!fused_active(s) || (s->n_rms > 0) != (dofs_a != nullptr))
+  const bool sp = sp_fuses(s) && !dofs_a;
+  if (!sp && (!fused_active(s) || (s->n_rms > 0) != (dofs_a != nullptr)))
     return edge::fail(EDGE_ERR_UNSUPPORTED, "fused steps: FP32 MFMA solvers, 16 elastic or 8 viscoelastic runs");
-  if (!s->proj_alt) EDGE_HIP_TRY(hipMalloc(&s->proj_alt, sizeof(float) * 4 * 768 * s->n_el));
+  if (!s->proj_alt) EDGE_HIP_TRY(hipMalloc(&s->proj_alt, proj_alt_bytes(s)));
   // the projection buffers no longer stand for a tInt array a separate
   // neighbour step could be handed
   s->proj_tint = nullptr;
   s->proj_fresh = false;
   if (s->n_rms > 0) return fused_steps_a(s, n_steps, dt, dofs, dofs_a, t_int, st);
+  if (sp) return sp_steps<float>(s, n_steps, dt, dofs, t_int, st);
   float* P[2] = {static_cast<float*>(s->proj), static_cast<float*>(s->proj_alt)};
   auto d = dev_view<float>(s);
   const float fdt = (float)dt;
-  if (sp_active(s)) {
-    auto x = sp_view<float>(s);
-    x.proj = P[0];
-    int rc = edge::launch_local_sp<float>(d, x, 0, s->n_el, fdt, (float*)dofs, (float*)t_int, st);
-    if (rc == EDGE_OK && s->fault) rc = edge::fault_apply(s->fault, dt, t_int, dofs, st);
-    for (int64_t k = 1; k < n_steps && rc == EDGE_OK; k++) {
-      x.proj = P[k % 2];
-      rc = edge::launch_fused_sp<float>(d, x, fdt, P[(k - 1) % 2], (float*)dofs, (float*)t_int, st);
-      if (rc == EDGE_OK && s->fault) rc = edge::fault_apply(s->fault, dt, t_int, dofs, st);
-    }
-    x.proj = P[(n_steps - 1) % 2];
-    return rc ? rc : edge::launch_neigh_sp<float>(d, x, 0, s->n_el, (float*)dofs, st);
-  }
   d.proj = P[0];
   int rc = edge::launch_local_mfma<float>(d, 0, s->n_el, fdt, (float*)dofs, (float*)t_int, st);
   if (rc == EDGE_OK && s->fault) rc = edge::fault_apply(s->fault, dt, t_int, dofs, st);
@@ -781,15 +806,16 @@ extern "C" int edge_el_create(const edge_el_config* cfg, const edge_mesh_in* mes
                         mesh->fa_el, mesh->fa_type, mesh->normals, mesh->tangents, mesh->areas, rho,
                         lam,         mu};
     s->sparse_star = true;  // built from the Jacobians' pattern only
+    const int pb = edge::phys::block(cfg->n_runs);
     if (hipMalloc(&s->jdet, sizeof(double) * s->n_el) != hipSuccess ||
-        (s->want_sp && hipMalloc(&s->sp_phys, s->real_bytes * edge::phys::values(s->n_el)) != hipSuccess))
+        (s->want_sp && hipMalloc(&s->sp_phys, s->real_bytes * edge::phys::values(s->n_el, pb)) != hipSuccess))
       rc = edge::fail(EDGE_ERR_HIP, "allocation of the element constants");
     else
       rc = cfg->precision == 64
                ? edge::build_setup<double>(in, (double*)s->star, (double*)s->fs, s->jdet, (double*)s->fsf,
-                                           &s->fs_rank3, nullptr, nullptr, nullptr, (double*)s->sp_phys, nullptr)
+                                           &s->fs_rank3, nullptr, nullptr, nullptr, (double*)s->sp_phys, pb, nullptr)
                : edge::build_setup<float>(in, (float*)s->star, (float*)s->fs, s->jdet, (float*)s->fsf,
-                                          &s->fs_rank3, nullptr, nullptr, nullptr, (float*)s->sp_phys, nullptr);
+                                          &s->fs_rank3, nullptr, nullptr, nullptr, (float*)s->sp_phys, pb, nullptr);
     if (rc == EDGE_OK) rc = zero_fault_faces(s);
     if (rc == EDGE_OK) rc = finish_mfma(s);
     if (rc == EDGE_OK) rc = finish_ec(s);
@@ -874,6 +900,7 @@ extern "C" int edge_el_destroy(edge_el_solver* s) {
   (void)hipFree(s->ec_proj);
   (void)hipFree(s->sp_phys);
   (void)hipFree(s->sp_rot);
+  (void)hipFree(s->sp_need);
   drop_lts(s);
   delete s;
   return EDGE_OK;
@@ -1000,10 +1027,10 @@ extern "C" int edge_el_create_visco(const edge_el_config* cfg, const edge_visco_
       rc = cfg->precision == 64
                ? edge::build_setup<double>(in, (double*)s->star, (double*)s->fs, s->jdet, (double*)s->fsf,
                                            &s->fs_rank3, (double*)s->star_a, (double*)s->fs_a, (double*)s->fsfa,
-                                           nullptr, nullptr)
+                                           nullptr, 1, nullptr)
                : edge::build_setup<float>(in, (float*)s->star, (float*)s->fs, s->jdet, (float*)s->fsf,
                                           &s->fs_rank3, (float*)s->star_a, (float*)s->fs_a, (float*)s->fsfa,
-                                          nullptr, nullptr);
+                                          nullptr, 1, nullptr);
     if (rc == EDGE_OK) rc = zero_fault_faces(s);
     if (rc == EDGE_OK) rc = upload_element_data(s, mesh, rho, s->lam_e.data(), s->mu_e.data());
     if (rc == EDGE_OK && p64_ok && src_pattern && (cfg->kernel == 0 || cfg->kernel == 4)) s->kernel = 4;
@@ -1413,8 +1440,8 @@ namespace {
 int step_impl(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* dofs_a, void* t_int, int use_graph,
               hipStream_t st) {
   if (n_steps == 0) return EDGE_OK;
-  const bool fuse = n_steps >= 2 && fused_active(s) && (s->n_rms > 0) == (dofs_a != nullptr);
-  if (fuse && !s->proj_alt) EDGE_HIP_TRY(hipMalloc(&s->proj_alt, sizeof(float) * 4 * 768 * s->n_el));
+  const bool fuse = n_steps >= 2 && (fused_active(s) || sp_fuses(s)) && (s->n_rms > 0) == (dofs_a != nullptr);
+  if (fuse && !s->proj_alt) EDGE_HIP_TRY(hipMalloc(&s->proj_alt, proj_alt_bytes(s)));
   if (!use_graph && fuse) return fused_steps(s, n_steps, dt, dofs, dofs_a, t_int, st);
   if (!use_graph) {
     for (int64_t i = 0; i < n_steps; i++) {
@@ -1501,7 +1528,7 @@ extern "C" int edge_el_neigh_local(edge_el_solver* s, double dt, void* dofs, voi
                                     "first, or its neighbour step has run)");
   int rc = check_neigh(s, t_int);
   if (rc) return rc;
-  if (!s->proj_alt) EDGE_HIP_TRY(hipMalloc(&s->proj_alt, sizeof(float) * 4 * 768 * s->n_el));
+  if (!s->proj_alt) EDGE_HIP_TRY(hipMalloc(&s->proj_alt, proj_alt_bytes(s)));
   auto d = dev_view<float>(s);
   d.proj = static_cast<float*>(s->proj_alt);
   if (sp_active(s)) {
