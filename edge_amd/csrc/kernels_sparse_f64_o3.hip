@@ -1,0 +1,7 @@
+// The sparse element kernels of order 3 in FP64.
+#include "kernels_sparse_impl.hpp"
+
+namespace edge {
+template int launch_sp<double, 3>(int, const SolverDev<double>&, const SpDev<double>&, int64_t, int64_t, double,
+                                  double*, double*, const double*, hipStream_t);
+}  // namespace edge

@@ -1,0 +1,8 @@
+// The sparse element kernels of order 5 in FP64.
+#define EDGE_SP_WAVES 8
+#include "kernels_sparse_impl.hpp"
+
+namespace edge {
+template int launch_sp<double, 5>(int, const SolverDev<double>&, const SpDev<double>&, int64_t, int64_t, double,
+                                  double*, double*, const double*, hipStream_t);
+}  // namespace edge

@@ -10,8 +10,9 @@
 // and it computes the outputs of its modes of every matrix product.  The
 // inputs of a product pass through LDS: the owners publish a column
 // [mode][64] and every wave reads the modes its outputs need.  Each non-zero
-// is one v_fmac_f32 with the entry as a literal: no operand loads, no
-// padding, no work on zeros.  The waves run different code (their own
+// is one fused multiply-add with the entry as a literal (FP64: from two scalar
+// moves that serve two columns): no operand loads, no padding, no work on
+// zeros.  The waves run different code (their own
 // non-zeros), the partition of the modes balances it.
 //
 // Instead of the 9 x 9 star matrices and flux solvers the kernels use what
@@ -40,7 +41,8 @@
 // 5, 196,608 tets, 16 runs with sources and receivers 8.60 -> 6.3 (MFMA, runs
 // on N); one run 1.19 -> 0.57 (MFMA, 16 elements on N); order 5, 36,720 tets,
 // 8 runs 6.81 -> 0.69 (generic); order 4 with a fault, 331,776 tets, 16 runs
-// 10.3 -> 5.3.
+// 10.3 -> 5.3; FP64 order 4, 12,870 tets, 16 runs 5.66 -> 0.64
+// (generic); order 5, 10,368 tets, 8 runs 5.85 -> 0.73 (generic).
 //
 // Operations (src/impl/seismic/solvers/AderDg.hpp:362-533, :553-722):
 //   local: CK time prediction (TimePredVanilla.hpp:200-306), volume integral
@@ -66,7 +68,13 @@ namespace {
 #define EDGE_INLINE __attribute__((always_inline))
 
 constexpr int kCols = 64;  // columns (lanes) per workgroup tile
-constexpr int kWaves = 4;
+// Waves per workgroup: four, in FP64 at orders 4 and 5 eight (the DOFs, the
+// time integral and the update of a quarter of the modes need more than the
+// 256 registers that two waves per SIMD leave a lane).
+#ifndef EDGE_SP_WAVES
+#define EDGE_SP_WAVES 4
+#endif
+constexpr int kWaves = EDGE_SP_WAVES;
 
 // The order in which the modes and face modes are dealt to the waves: wave w
 // of W owns the modes at positions j W + w, and a column's LDS row is the
@@ -84,6 +92,19 @@ struct Deal<3> {
   static constexpr int mode[10] = {0, 1, 3, 2, 6, 5, 9, 8, 4, 7};
   static constexpr int face[6] = {2, 3, 0, 1, 5, 4};
 };
+#if EDGE_SP_WAVES == 8
+template <>
+struct Deal<4> {
+  static constexpr int mode[20] = {0, 2, 3, 1, 4, 5, 6, 8, 9, 7, 12, 17, 19, 16, 18, 13, 10, 15, 14, 11};
+  static constexpr int face[10] = {6, 9, 4, 5, 1, 0, 2, 3, 7, 8};
+};
+template <>
+struct Deal<5> {
+  static constexpr int mode[35] = {0,  2,  3,  1,  5,  7,  6,  4,  9,  8,  14, 17, 11, 12, 13, 16, 19, 15,
+                                   10, 18, 24, 34, 26, 31, 21, 25, 28, 32, 33, 23, 27, 22, 20, 30, 29};
+  static constexpr int face[15] = {10, 0, 6, 8, 12, 11, 1, 3, 2, 14, 9, 7, 5, 4, 13};
+};
+#else
 template <>
 struct Deal<4> {
   static constexpr int mode[20] = {0, 3, 2, 1, 9, 4, 5, 6, 8, 7, 19, 12, 11, 16, 14, 17, 10, 15, 13, 18};
@@ -95,6 +116,7 @@ struct Deal<5> {
                                    17, 12, 30, 34, 29, 33, 21, 25, 32, 31, 20, 23, 27, 24, 28, 26, 22};
   static constexpr int face[15] = {5, 8, 4, 9, 12, 13, 14, 0, 11, 7, 10, 2, 1, 6, 3};
 };
+#endif
 
 template <int O>
 struct Dim {
@@ -167,13 +189,32 @@ constexpr bool starts() {
   return true;
 }
 
+// A matrix entry as an operand: a literal in FP32; in FP64 a pair of scalar
+// registers written where it is used (left to the compiler, hundreds of them
+// stay live across a product and spill).
+template <typename T>
+__device__ __forceinline__ T entry(double v) {
+  if constexpr (sizeof(T) == 8) {
+    const long long b = __builtin_bit_cast(long long, v);
+    int lo, hi;
+    asm volatile("s_mov_b32 %0, %1" : "=s"(lo) : "i"((int)b));
+    asm volatile("s_mov_b32 %0, %1" : "=s"(hi) : "i"((int)(b >> 32)));
+    return __builtin_bit_cast(double, (long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
+  } else {
+    return T(v);
+  }
+}
+
 // out[j] += M[k][n_j] x over wave W's outputs n_j < nn with a non-zero entry
 // (out[j] = for the first one).
 template <typename Mat, int K, int N, bool FIRST, typename T>
 __device__ __forceinline__ void term(T x, T& out) {
   if constexpr (N >= 0) {
     constexpr double v = Mat::at(K, N);
-    if constexpr (v != 0.0) out = FIRST ? T(v) * x : fma_(T(v), x, out);
+    if constexpr (v != 0.0) {
+      const T c = entry<T>(v);
+      out = FIRST ? c * x : fma_(c, x, out);
+    }
   }
 }
 template <int O, int NN, int W, int J>
@@ -188,22 +229,27 @@ template <int O, int W, typename Mat, int K, typename T, int... J>
 __device__ __forceinline__ void face_terms(T x, T* out, std::integer_sequence<int, J...>) {
   (term<Mat, K, Dim<O>::face(W, J), starts<Mat, K, Dim<O>::face(W, J)>()>(x, out[J]), ...);
 }
-// The same with the sum running over three matrices per input (x: input K
-// of matrix D).
+// Input K of two columns with matrix D of three: p += M x and, summed over
+// the matrices, v += M y, each entry used for both.
 template <int O, int NN, int W, typename M0, typename M1, typename M2, int K, int D, int J, typename T>
-__device__ __forceinline__ void term3(T x, T& out) {
+__device__ __forceinline__ void pair_term(T x, T y, T& p, T& v) {
   constexpr int N = mode_of<O, NN, W, J>();
   if constexpr (N >= 0) {
-    constexpr bool s = starts<M0, K, N>() && starts<M1, K, N>() && starts<M2, K, N>();
-    constexpr bool n0 = M0::at(K, N) != 0.0, n1 = M1::at(K, N) != 0.0;
-    if constexpr (D == 0) term<M0, K, N, s>(x, out);
-    if constexpr (D == 1) term<M1, K, N, s && !n0>(x, out);
-    if constexpr (D == 2) term<M2, K, N, s && !n0 && !n1>(x, out);
+    using M = std::conditional_t<D == 0, M0, std::conditional_t<D == 1, M1, M2>>;
+    constexpr double m = M::at(K, N);
+    if constexpr (m != 0.0) {
+      constexpr bool s = starts<M0, K, N>() && starts<M1, K, N>() && starts<M2, K, N>();
+      constexpr bool n0 = M0::at(K, N) != 0.0, n1 = M1::at(K, N) != 0.0;
+      constexpr bool first = s && (D < 1 || !n0) && (D < 2 || !n1);
+      const T c = entry<T>(m);
+      p = starts<M, K, N>() ? c * x : fma_(c, x, p);
+      v = first ? c * y : fma_(c, y, v);
+    }
   }
 }
 template <int O, int NN, int W, typename M0, typename M1, typename M2, int K, int D, typename T, int... J>
-__device__ __forceinline__ void terms3(T x, T* out, std::integer_sequence<int, J...>) {
-  (term3<O, NN, W, M0, M1, M2, K, D, J>(x, out[J]), ...);
+__device__ __forceinline__ void pair_terms(T x, T y, T* p, T* v, std::integer_sequence<int, J...>) {
+  (pair_term<O, NN, W, M0, M1, M2, K, D, J>(x, y, p[J], v[J]), ...);
 }
 
 template <int O, bool CK, int D>
@@ -233,7 +279,7 @@ struct Reads {
 // outputs of wave V below NN, inputs below NK.
 template <int O, bool CK, int NK, int NN, int V>
 struct StiffReads {
-  static constexpr int J = Dim<O>::own(NN), G = 12, ROWS = NK;
+  static constexpr int J = Dim<O>::own(NN), G = 64 / kWaves, ROWS = NK;
   template <int D>
   static constexpr bool feeds(int k) {
     for (int j = 0; j < J; j++) {
@@ -242,30 +288,25 @@ struct StiffReads {
     }
     return false;
   }
+  // per input the four columns, one after the other
   static constexpr Reads<4 * NK> list() {
     Reads<4 * NK> l;
     for (int k = 0; k < NK; k++)
-      if (feeds<0>(k) || feeds<1>(k) || feeds<2>(k)) l.add(0, k);
-    for (int k = 0; k < NK; k++) {
-      if (feeds<0>(k)) l.add(1, k);
-      if (feeds<1>(k)) l.add(2, k);
-      if (feeds<2>(k)) l.add(3, k);
-    }
+      if (feeds<0>(k) || feeds<1>(k) || feeds<2>(k))
+        for (int c = 0; c < 4; c++) l.add(c, k);
     return l;
   }
   static constexpr int row(int k) { return Dim<O>::row(k); }
   template <int COL, int K, typename T>
-  static __device__ __forceinline__ void use(T x, T (&p)[3][J], T (&v)[J]) {
-    using M0 = Stiff<O, CK, 0>;
-    using M1 = Stiff<O, CK, 1>;
-    using M2 = Stiff<O, CK, 2>;
-    using JS = std::make_integer_sequence<int, J>;
+  static __device__ __forceinline__ void use(const T* x, T (&p)[3][J], T (&v)[J]) {
     if constexpr (COL == 0) {
-      terms<O, NN, V, M0, K>(x, p[0], JS{});
-      terms<O, NN, V, M1, K>(x, p[1], JS{});
-      terms<O, NN, V, M2, K>(x, p[2], JS{});
-    } else {
-      terms3<O, NN, V, M0, M1, M2, K, COL - 1>(x, v, JS{});
+      using M0 = Stiff<O, CK, 0>;
+      using M1 = Stiff<O, CK, 1>;
+      using M2 = Stiff<O, CK, 2>;
+      using JS = std::make_integer_sequence<int, J>;
+      pair_terms<O, NN, V, M0, M1, M2, K, 0>(x[0], x[1], p[0], v, JS{});
+      pair_terms<O, NN, V, M0, M1, M2, K, 1>(x[0], x[2], p[1], v, JS{});
+      pair_terms<O, NN, V, M0, M1, M2, K, 2>(x[0], x[3], p[2], v, JS{});
     }
   }
 };
@@ -273,7 +314,7 @@ struct StiffReads {
 // One column of a face's w in the element's modes to the wave's face modes.
 template <int O, int F, int V>
 struct ProjectReads {
-  static constexpr int N = Dim<O>::N, J = Dim<O>::MF, G = 12, ROWS = 0;
+  static constexpr int N = Dim<O>::N, J = Dim<O>::MF, G = 48 / kWaves, ROWS = 0;
   static constexpr Reads<N> list() {
     Reads<N> l;
     for (int k = 0; k < N; k++) {
@@ -288,15 +329,15 @@ struct ProjectReads {
   }
   static constexpr int row(int k) { return Dim<O>::row(k); }
   template <int COL, int K, typename T>
-  static __device__ __forceinline__ void use(T x, T (&u)[J]) {
-    face_terms<O, V, Prj<O, F>, K>(x, u, std::make_integer_sequence<int, J>{});
+  static __device__ __forceinline__ void use(const T* x, T (&u)[J]) {
+    face_terms<O, V, Prj<O, F>, K>(x[0], u, std::make_integer_sequence<int, J>{});
   }
 };
 
 // One face column to the wave's modes.
 template <int O, int F, int V>
 struct LiftReads {
-  static constexpr int NF = Dim<O>::NF, J = Dim<O>::M, G = 16, ROWS = 0;
+  static constexpr int NF = Dim<O>::NF, J = Dim<O>::M, G = 64 / kWaves, ROWS = 0;
   static constexpr Reads<NF> list() {
     Reads<NF> l;
     for (int k = 0; k < NF; k++) {
@@ -311,8 +352,8 @@ struct LiftReads {
   }
   static constexpr int row(int k) { return Dim<O>::face_row(k); }
   template <int COL, int K, typename T>
-  static __device__ __forceinline__ void use(T x, T (&u)[J]) {
-    terms<O, Dim<O>::N, V, Lift<O, F>, K>(x, u, std::make_integer_sequence<int, J>{});
+  static __device__ __forceinline__ void use(const T* x, T (&u)[J]) {
+    terms<O, Dim<O>::N, V, Lift<O, F>, K>(x[0], u, std::make_integer_sequence<int, J>{});
   }
 };
 
@@ -338,7 +379,7 @@ __device__ __forceinline__ void consume(const T (&x)[S::G], std::integer_sequenc
         constexpr int at = C * S::G + I;
         if constexpr (at < list.n) {
           constexpr int col = list.r[at].col, k = list.r[at].k;
-          S::template use<col, k>(x[I], out...);
+          S::template use<col, k>(x + I, out...);
         }
       }(),
       ...);
@@ -463,7 +504,7 @@ struct Tile {
   unsigned ph_off;
   // The inverse Jacobian and the material: in registers, at order 5 with
   // fused runs read from LDS where they are used (the registers are full).
-  static constexpr bool HELD = R == 1 || O < 5;
+  static constexpr bool HELD = R == 1 || O < 5 || sizeof(T) == 8;
   T ji1[3][3];
   Mat4<T> mat1;
 
@@ -834,14 +875,16 @@ struct Tile {
   }
 
   // the neighbours' w (projections p), taken to the element's face
-  // coordinates, to LDS rows [f][i][NF]: wave f takes face f (slot, fm: its
-  // projection slot and flux matrix)
+  // coordinates, to LDS rows [f][i][NF]: wave w takes face w % 4 (slot, fm:
+  // its projection slot and flux matrix); of eight waves the first four take
+  // the first two components
   __device__ __forceinline__ void receive(int32_t slot, int fm, const T* __restrict__ rot, const T* __restrict__ p,
                                           T (&u)[4 * NV], T (&r)[phys::kRotPad]) const {
     const vec4* src = reinterpret_cast<const vec4*>(p) + (int64_t)(slot < 0 ? 0 : slot) * NV * R + lane % R;
     const vec4* rv = reinterpret_cast<const vec4*>(rot) + (fm < 4 ? 0 : 1 + (fm - 4) / 4) * (phys::kRotPad / 4);
 #pragma unroll
     for (int v = 0; v < NV; v++) {
+      if (W == 8 && (w < 4 ? 4 * v >= 2 * D::NF : 4 * v + 3 < 2 * D::NF)) continue;
       const vec4 x = src[v * R];
 #pragma unroll
       for (int j = 0; j < 4; j++) u[4 * v + j] = x[j];
@@ -854,9 +897,10 @@ struct Tile {
     }
   }
   __device__ __forceinline__ void rotate(int32_t slot, const T (&u)[4 * NV], const T (&r)[phys::kRotPad]) {
-    T* dst = lds + w * 3 * D::NF * kCols + lane;
+    T* dst = lds + (w % 4) * 3 * D::NF * kCols + lane;
 #pragma unroll
-    for (int i = 0; i < 3; i++)
+    for (int i = 0; i < 3; i++) {
+      if (W == 8 && (w < 4) != (i < 2)) continue;
       each(
           [&](auto P) EDGE_INLINE {
             constexpr int p0 = decltype(P)::value, lo = p0 * (p0 + 1) / 2;
@@ -876,6 +920,7 @@ struct Tile {
                 std::make_integer_sequence<int, p0 + 1>{});
           },
           std::make_integer_sequence<int, O>{});
+    }
   }
 };
 
@@ -885,15 +930,16 @@ __device__ __forceinline__ int64_t tile_index(int64_t n, bool xcd) {
   return xcd ? (b & 7) * chunk + (b >> 3) : b;
 }
 
-// Waves per SIMD the registers are limited for: what the tiles' LDS allows.
-constexpr int waves_per_simd(int order) { return order == 5 ? 2 : 3; }
+// Waves per SIMD the registers are limited for: what the tiles' LDS allows
+// (order 4 with three: 6.44 against 6.69 ms per step with two).
+constexpr int waves_per_simd(int order, int bytes) { return order == 5 || bytes == 8 ? 2 : 3; }
 
 // NB: the neighbouring surface integral from the projections proj_in; LOC:
 // the local step (projections to x.proj).  Both: the neighbour step of the
 // previous time step first (its DOFs also go to s.tap for the elements
 // s.tap_on marks).
 template <typename T, int O, int R, bool NB, bool LOC>
-__global__ __launch_bounds__(64 * kWaves, waves_per_simd(O)) void k_sparse(SolverDev<T> s, SpDev<T> x, int64_t first, int64_t n, T dt, T* __restrict__ dofs, T* __restrict__ t_int,
+__global__ __launch_bounds__(64 * kWaves, waves_per_simd(O, sizeof(T))) void k_sparse(SolverDev<T> s, SpDev<T> x, int64_t first, int64_t n, T dt, T* __restrict__ dofs, T* __restrict__ t_int,
               const T* __restrict__ proj_in) {
   using D = Dim<O>;
   constexpr int M = D::M, W = D::W, E = kCols / R;
@@ -919,8 +965,8 @@ __global__ __launch_bounds__(64 * kWaves, waves_per_simd(O)) void k_sparse(Solve
   int32_t slot = -1;
   int fm = 0;
   if constexpr (NB) {
-    slot = s.rcv[b.el * 4 + b.w];
-    fm = s.nb.fmat[b.el * 4 + b.w];
+    slot = s.rcv[b.el * 4 + b.w % 4];
+    fm = s.nb.fmat[b.el * 4 + b.w % 4];
   }
   if constexpr (R == 1) {
     constexpr int PB = phys::block(R);
@@ -1025,7 +1071,9 @@ int launch_sp(int op, const SolverDev<T>& s, const SpDev<T>& x, int64_t first, i
               const T* proj_in, hipStream_t st) {
   if (n <= 0) return EDGE_OK;
   switch (s.n_runs) {
-    case 1: return by_op<T, O, 1>(op, s, x, first, n, dt, dofs, t_int, proj_in, st);
+    case 1:
+      if constexpr (sizeof(T) == 4 || O < 5) return by_op<T, O, 1>(op, s, x, first, n, dt, dofs, t_int, proj_in, st);
+      break;
     case 8: return by_op<T, O, 8>(op, s, x, first, n, dt, dofs, t_int, proj_in, st);
     case 16: return by_op<T, O, 16>(op, s, x, first, n, dt, dofs, t_int, proj_in, st);
   }

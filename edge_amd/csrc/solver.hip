@@ -515,8 +515,7 @@ int local_t(edge_el_solver* s, int64_t first, int64_t n, double dt, void* dofs, 
   if (s->n_rms > 0) return edge::fail(EDGE_ERR_ARG, "viscoelastic solver: the step needs dofs_a (edge_el_local_a)");
   const auto d = dev_view<T>(s);
   note_local(s, t_int);
-  if constexpr (sizeof(T) == 4)
-    if (sp_active(s)) return edge::launch_local_sp<T>(d, sp_view<T>(s), first, n, (T)dt, (T*)dofs, (T*)t_int, st);
+  if (sp_active(s)) return edge::launch_local_sp<T>(d, sp_view<T>(s), first, n, (T)dt, (T*)dofs, (T*)t_int, st);
   if (s->kernel == 2) return edge::launch_local_mfma<T>(d, first, n, (T)dt, (T*)dofs, (T*)t_int, st);
   if (s->kernel == 5) return edge::launch_local_ec<T>(d, ec_view<T>(s), first, n, (T)dt, (T*)dofs, (T*)t_int, st);
   if constexpr (sizeof(T) == 8)
@@ -529,8 +528,7 @@ int neigh_t(edge_el_solver* s, int64_t first, int64_t n, const void* t_int, void
   if (s->n_rms > 0) return edge::fail(EDGE_ERR_ARG, "viscoelastic solver: the step needs dofs_a (edge_el_neigh_a)");
   const auto d = dev_view<T>(s);
   if (int rc = check_neigh(s, t_int)) return rc;
-  if constexpr (sizeof(T) == 4)
-    if (sp_active(s)) return edge::launch_neigh_sp<T>(d, sp_view<T>(s), first, n, (T*)dofs, st);
+  if (sp_active(s)) return edge::launch_neigh_sp<T>(d, sp_view<T>(s), first, n, (T*)dofs, st);
   if (s->kernel == 2) return edge::launch_neigh_mfma<T>(d, first, n, (const T*)t_int, (T*)dofs, st);
   if (s->kernel == 5) return edge::launch_neigh_ec<T>(d, ec_view<T>(s), first, n, (T*)dofs, st);
   if constexpr (sizeof(T) == 8)
@@ -584,15 +582,8 @@ int neigh_lts_t(edge_el_solver* s, int64_t first, int64_t n, int first_ts, const
   if (d.rcv) d.rcv = s->rcv_lts;
   int rc = check_neigh(s, t0);
   if (rc) return rc;
-  bool done = false;
-  if constexpr (sizeof(T) == 4) {
-    if (sp_active(s)) {
-      rc = edge::launch_neigh_sp<T>(d, sp_view<T>(s), first, n, (T*)dofs, st);
-      done = true;
-    }
-  }
-  if (done)
-    ;
+  if (sp_active(s))
+    rc = edge::launch_neigh_sp<T>(d, sp_view<T>(s), first, n, (T*)dofs, st);
   else if (s->kernel == 2)
     rc = edge::launch_neigh_mfma<T>(d, first, n, (const T*)t0, (T*)dofs, st);
   else if (s->kernel == 5)
@@ -736,7 +727,9 @@ int fused_steps(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void*
   s->proj_tint = nullptr;
   s->proj_fresh = false;
   if (s->n_rms > 0) return fused_steps_a(s, n_steps, dt, dofs, dofs_a, t_int, st);
-  if (sp) return sp_steps<float>(s, n_steps, dt, dofs, t_int, st);
+  if (sp)
+    return s->cfg.precision == 64 ? sp_steps<double>(s, n_steps, dt, dofs, t_int, st)
+                                  : sp_steps<float>(s, n_steps, dt, dofs, t_int, st);
   float* P[2] = {static_cast<float*>(s->proj), static_cast<float*>(s->proj_alt)};
   auto d = dev_view<float>(s);
   const float fdt = (float)dt;

@@ -1,4 +1,4 @@
-"""The FP32 kernels over the matrices' non-zeros (kernels_sparse_impl.hpp),
+"""The kernels over the matrices' non-zeros (kernels_sparse_impl.hpp),
 64 (element, run) columns per workgroup, against the FP64 oracle: every order
 and run count on meshes whose last tile is partly filled, element ranges that
 start inside a tile, free-surface, outflow and periodic faces in every
@@ -14,7 +14,8 @@ from edge_amd.mesh import FA_FREE_SURFACE, FA_OUTFLOW, FA_PERIODIC
 from edge_amd.solver import ElasticSolver
 
 pytestmark = pytest.mark.gpu
-TOL = 1e-5  # FP32 against the FP64 oracle, as every FP32 path
+TOL = {32: 1e-5, 64: 1e-12}  # against the FP64 oracle, as every path of the precision
+NP = {32: np.float32, 64: np.float64}
 
 
 def rel(a, b):
@@ -22,47 +23,53 @@ def rel(a, b):
     return float(np.linalg.norm((a - b).ravel()) / np.linalg.norm(b.ravel()))
 
 
-def _problem(runs, order, n=(3, 4, 3), seed=5):
+def _problem(runs, order, precision=32, n=(3, 4, 3), seed=5):
     import torch
     m = M.box(n, bc=(FA_FREE_SURFACE, FA_OUTFLOW, FA_PERIODIC), jitter=0.1, seed=seed)
     rho, lam, mu = S.random_materials(m.n_el, seed=seed)
-    d0 = np.random.default_rng(order).normal(size=(m.n_el, 9, S.n_modes(order), runs)).astype(np.float32)
+    d0 = np.random.default_rng(order).normal(size=(m.n_el, 9, S.n_modes(order), runs)).astype(NP[precision])
     dev = torch.from_numpy(d0).cuda()
     return m, (rho, lam, mu), S.dt_cfl(m, rho, lam, mu, order), d0.astype(np.float64), dev
 
 
 @pytest.mark.parametrize("runs", [1, 8, 16])
 @pytest.mark.parametrize("order", [2, 3, 4, 5])
-def test_steps_match_oracle(gpu, order, runs):
+@pytest.mark.parametrize("precision", [32, 64])
+def test_steps_match_oracle(gpu, precision, order, runs):
     """216 elements (3.4, 27 and 54 tiles of 64, 8 and 4): local, neighbour,
     then three steps in one call."""
     import torch
-    m, mat, dt, d, gd = _problem(runs, order)
-    s = ElasticSolver(m, order, runs, 32, *mat)
+    if (precision, order, runs) == (64, 5, 16):
+        pytest.skip("refused: FP64 order 5 has at most 8 runs")
+    m, mat, dt, d, gd = _problem(runs, order, precision)
+    tol = TOL[precision]
+    s = ElasticSolver(m, order, runs, precision, *mat)
+    assert s.kernel_info()[0] == (2 if (precision, runs) == (32, 16) else 5)
     mo = orc.MeshOracle(m, order, runs, rho=mat[0], lam=mat[1], mu=mat[2])
     t, gt = np.zeros_like(d), torch.zeros_like(gd)
     mo.local(d, t, dt)
     s.local(gd, gt, dt)
-    assert rel(gt.cpu().numpy(), t) <= TOL
-    assert rel(gd.cpu().numpy(), d) <= TOL
+    assert rel(gt.cpu().numpy(), t) <= tol
+    assert rel(gd.cpu().numpy(), d) <= tol
     mo.neigh(d, t)
     s.neigh(gd, gt)
-    assert rel(gd.cpu().numpy(), d) <= TOL
+    assert rel(gd.cpu().numpy(), d) <= tol
     mo.step(d, t, dt, 3)
     s.step(gd, gt, dt, 3)
-    assert rel(gt.cpu().numpy(), t) <= TOL
-    assert rel(gd.cpu().numpy(), d) <= TOL
+    assert rel(gt.cpu().numpy(), t) <= tol
+    assert rel(gd.cpu().numpy(), d) <= tol
     s.close()
 
 
 @pytest.mark.parametrize("runs", [1, 8, 16])
-def test_ranges_equal_whole(gpu, runs):
+@pytest.mark.parametrize("precision", [32, 64])
+def test_ranges_equal_whole(gpu, precision, runs):
     """Element ranges that start and end inside a tile (and inside a block of
     the constants) write their elements only, and the same values as one call."""
     import torch
     order = 4
-    m, mat, dt, _, gd = _problem(runs, order)
-    s = ElasticSolver(m, order, runs, 32, *mat)
+    m, mat, dt, _, gd = _problem(runs, order, precision)
+    s = ElasticSolver(m, order, runs, precision, *mat)
     cuts = [0, 1, 62, 67, 130, 131, 215, m.n_el]
     a, ta = gd.clone(), torch.zeros_like(gd)
     s.local(a, ta, dt)
@@ -97,5 +104,5 @@ def test_neighbours_that_do_not_pair(gpu, runs):
     t, gt = np.zeros_like(d), torch.zeros_like(gd)
     mo.step(d, t, dt, 2)
     s.step(gd, gt, dt, 2)
-    assert rel(gd.cpu().numpy(), d) <= TOL
+    assert rel(gd.cpu().numpy(), d) <= TOL[32]
     s.close()
