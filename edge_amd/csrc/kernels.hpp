@@ -154,6 +154,8 @@ struct SolverRef {
   int64_t n_el = 0;
   const double* jdet = nullptr;  // [nEl] Jacobian determinants (device), null for caller-given solvers
   const double* mass = nullptr;  // [N] diagonal reference mass matrix (device)
+  const double* mat = nullptr;   // [3][nEl] rho, lambda, mu, null without materials
+  const double* geo = nullptr;   // [nEl][12] v0, v1 - v0, v2 - v0, v3 - v0, null without geometry
   SolverDev<float> f{};
   SolverDev<double> d{};
 };
@@ -164,14 +166,16 @@ int solver_ref(const edge_el_solver* s, SolverRef* out);
 int fault_apply(edge_fault* f, double dt, const void* t_int, void* dofs, hipStream_t st);
 const edge_el_solver* fault_solver(const edge_fault* f);
 
-// Blocks of the L2-norm reduction (their partial sums are added in block
-// order, on the host or on the device).
+// Blocks of the L2-norm reduction (norms.hip).
 constexpr unsigned kL2Blocks = 1024;
 // Per-block partial sums of the FP64 L2 norms of DOF arrays a (and a - b):
 // part[nblk][2][9 R] = (sum |J| M_n (a - b)^2, sum |J| M_n b^2) over each
 // block's element range; every entry is written.
 int l2_partials(edge_el_solver* s, const void* a, int prec_a, const void* b, int prec_b, double* part, unsigned nblk,
                 hipStream_t st);
+// out[i] = sum over the blocks of part[nblk][width] (largest value, at least
+// 0, for i >= first_max), in an order that depends on nblk only.
+int sum_partials(const double* part, unsigned nblk, int width, int first_max, double* out, hipStream_t st);
 
 // Receivers and point sources (points.hip).
 template <typename T>

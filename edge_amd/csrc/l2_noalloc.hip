@@ -1,7 +1,6 @@
 // FP64 L2 norms that allocate nothing: edge_el_l2_norms with its per-block
-// partial sums in a file-scope device array instead of a per-call hipMalloc,
-// and the block sums formed on the device in the same order as the host sum
-// of edge_el_l2_norms (so both return the same bits).
+// partial sums in a file-scope device array instead of a per-call hipMalloc
+// (the same kernels: both return the same bits).
 //
 // For callers that cannot allocate device memory (code under HIP graph
 // capture, tight serving loops).  The array lives on every GPU the library
@@ -44,17 +43,6 @@ int scratch_ptr(double** out) {
   return EDGE_OK;
 }
 
-// sums[i] = sum_k part[k][i] for i < 2 nqr, k in block order (the host loop
-// of edge_el_l2_norms: plain additions from 0, k ascending)
-__global__ __launch_bounds__(256) void k_l2_sum(const double* __restrict__ part, unsigned nblk, int nqr,
-                                                double* __restrict__ sums) {
-  for (int i = threadIdx.x; i < 2 * nqr; i += blockDim.x) {
-    double acc = 0.0;
-    for (unsigned k = 0; k < nblk; k++) acc += part[(size_t)k * 2 * nqr + i];
-    sums[i] = acc;
-  }
-}
-
 }  // namespace
 
 extern "C" int edge_el_l2_norms_noalloc(edge_el_solver* s, const void* a, int prec_a, const void* b, int prec_b,
@@ -80,8 +68,8 @@ extern "C" int edge_el_l2_norms_noalloc(edge_el_solver* s, const void* a, int pr
   // so nothing from an earlier call is read
   const int rc = edge::l2_partials(s, a, prec_a, b, prec_b, part, nblk, st);
   if (rc != EDGE_OK) return rc;
-  hipLaunchKernelGGL(k_l2_sum, dim3(1), dim3(256), 0, st, (const double*)part, nblk, nqr, sums);
-  EDGE_HIP_TRY(hipGetLastError());
+  const int rc2 = edge::sum_partials(part, nblk, 2 * nqr, 2 * nqr, sums, st);
+  if (rc2 != EDGE_OK) return rc2;
   if (diff_sq) EDGE_HIP_TRY(hipMemcpyAsync(diff_sq, sums, sizeof(double) * nqr, hipMemcpyDeviceToHost, st));
   if (ref_sq) EDGE_HIP_TRY(hipMemcpyAsync(ref_sq, sums + nqr, sizeof(double) * nqr, hipMemcpyDeviceToHost, st));
   EDGE_HIP_TRY(hipStreamSynchronize(st));

@@ -1127,6 +1127,8 @@ int solver_ref(const edge_el_solver* s, SolverRef* out) {
   out->n_el = s->n_el;
   out->jdet = s->jdet;
   out->mass = s->mass;
+  out->mat = s->mat;
+  out->geo = s->geo;
   if (s->cfg.precision == 64)
     out->d = dev_view<double>(s);
   else
@@ -1564,289 +1566,5 @@ extern "C" int edge_el_info(const edge_el_solver* s, int64_t* n_el, int32_t* n_m
   if (n_modes) *n_modes = s->n_modes;
   if (n_runs) *n_runs = s->cfg.n_runs;
   if (dof_bytes) *dof_bytes = (int64_t)s->real_bytes * 9 * s->n_modes * s->cfg.n_runs * s->n_el;
-  return EDGE_OK;
-}
-
-namespace {
-
-// Per-block partial sums of |J| M_n (a - b)^2 and |J| M_n b^2 per (quantity, run).
-template <typename TA, typename TB>
-__global__ __launch_bounds__(256) void k_l2(int64_t n_el, int n_md, int n_crs, const double* __restrict__ jdet,
-                                            const double* __restrict__ mass, const TA* __restrict__ a,
-                                            const TB* __restrict__ b, double* __restrict__ part) {
-  // one block per chunk of elements; thread t accumulates entry t of [9][R]
-  const int nqr = 9 * n_crs;
-  const int64_t per = (n_el + gridDim.x - 1) / gridDim.x;
-  const int64_t e0 = blockIdx.x * per, e1 = min(n_el, e0 + per);
-  for (int qr = threadIdx.x; qr < nqr; qr += blockDim.x) {
-    const int q = qr / n_crs, r = qr % n_crs;
-    double d2 = 0, r2 = 0;
-    for (int64_t el = e0; el < e1; el++) {
-      const double j = fabs(jdet[el]);
-      const size_t base = ((size_t)el * 9 + q) * n_md * n_crs + r;
-      for (int md = 0; md < n_md; md++) {
-        const double av = (double)a[base + (size_t)md * n_crs];
-        const double bv = b ? (double)b[base + (size_t)md * n_crs] : av;
-        const double w = j * mass[md];
-        d2 += w * (av - bv) * (av - bv);
-        r2 += w * bv * bv;
-      }
-    }
-    part[(size_t)blockIdx.x * 2 * nqr + qr] = d2;
-    part[(size_t)blockIdx.x * 2 * nqr + nqr + qr] = r2;
-  }
-}
-
-template <typename TA, typename TB>
-int l2_launch(edge_el_solver* s, const void* a, const void* b, double* d_part, unsigned nblk, hipStream_t st) {
-  hipLaunchKernelGGL((k_l2<TA, TB>), dim3(nblk), dim3(256), 0, st, s->n_el, s->n_modes, s->cfg.n_runs, s->jdet,
-                     s->mass, (const TA*)a, (const TB*)b, d_part);
-  EDGE_HIP_TRY(hipGetLastError());
-  return EDGE_OK;
-}
-
-}  // namespace
-
-namespace edge {
-// Per-block partial sums of the L2 norms (k_l2) into part[nblk][2][9 R].
-int l2_partials(edge_el_solver* s, const void* a, int prec_a, const void* b, int prec_b, double* part, unsigned nblk,
-                hipStream_t st) {
-  const int pb = b ? prec_b : prec_a;
-  if (prec_a == 64 && pb == 64) return l2_launch<double, double>(s, a, b, part, nblk, st);
-  if (prec_a == 64) return l2_launch<double, float>(s, a, b, part, nblk, st);
-  if (pb == 64) return l2_launch<float, double>(s, a, b, part, nblk, st);
-  return l2_launch<float, float>(s, a, b, part, nblk, st);
-}
-}  // namespace edge
-
-extern "C" int edge_el_l2_norms(edge_el_solver* s, const void* a, int prec_a, const void* b, int prec_b,
-                                double* diff_sq, double* ref_sq, void* stream) {
-  if (!s) return edge::fail(EDGE_ERR_ARG, "solver handle missing");
-  if (!s->jdet) return edge::fail(EDGE_ERR_UNSUPPORTED, "norms need a solver built from geometry");
-  if (!a || (prec_a != 32 && prec_a != 64) || (b && prec_b != 32 && prec_b != 64))
-    return edge::fail(EDGE_ERR_ARG, "norm arguments");
-  hipStream_t st = (hipStream_t)stream;
-  const int nqr = 9 * s->cfg.n_runs;
-  const unsigned nblk = edge::kL2Blocks;
-  double* d_part = nullptr;
-  EDGE_HIP_TRY(hipMalloc(&d_part, sizeof(double) * 2 * nqr * nblk));
-  int rc = edge::l2_partials(s, a, prec_a, b, prec_b, d_part, nblk, st);
-  std::vector<double> h(2 * nqr * nblk);
-  if (rc == EDGE_OK &&
-      hipMemcpyAsync(h.data(), d_part, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st) == hipSuccess &&
-      hipStreamSynchronize(st) == hipSuccess) {
-    for (int i = 0; i < nqr; i++) {
-      double d2 = 0, r2 = 0;
-      for (unsigned k = 0; k < nblk; k++) {
-        d2 += h[(size_t)k * 2 * nqr + i];
-        r2 += h[(size_t)k * 2 * nqr + nqr + i];
-      }
-      if (diff_sq) diff_sq[i] = d2;
-      if (ref_sq) ref_sq[i] = r2;
-    }
-  } else if (rc == EDGE_OK) {
-    rc = edge::fail(EDGE_ERR_HIP, "norm reduction");
-  }
-  (void)hipFree(d_part);
-  return rc;
-}
-
-namespace {
-// Per-block partial sums per run of the kinetic energy 1/2 rho |v|^2 and the
-// strain energy 1/2 sigma : C^-1 : sigma (isotropic compliance
-// C^-1 sigma = sigma / (2 mu) - lambda / (2 mu (3 lambda + 2 mu)) tr(sigma) I),
-// integrated exactly through |J| and the diagonal reference mass matrix.
-template <typename T>
-__global__ __launch_bounds__(256) void k_energy(int64_t n_el, int n_md, int n_crs, const double* __restrict__ jdet,
-                                                const double* __restrict__ mass, const double* __restrict__ mat,
-                                                const T* __restrict__ dofs, double* __restrict__ part) {
-  __shared__ double sk[256], ss[256];
-  const int64_t per = (n_el + gridDim.x - 1) / gridDim.x;
-  const int64_t e0 = blockIdx.x * per, e1 = min(n_el, e0 + per);
-  const int t = threadIdx.x, r = t % n_crs, m0 = t / n_crs, mstep = blockDim.x / n_crs;
-  double ek = 0, es = 0;
-  if (m0 < mstep) {
-    for (int64_t el = e0; el < e1; el++) {
-      const double j = fabs(jdet[el]), rho = mat[el], lam = mat[n_el + el], mu = mat[2 * n_el + el];
-      const double c1 = 0.5 / mu, c2 = lam / (2 * mu * (3 * lam + 2 * mu));
-      for (int md = m0; md < n_md; md += mstep) {
-        double x[9];
-        for (int q = 0; q < 9; q++) x[q] = (double)dofs[(((size_t)el * 9 + q) * n_md + md) * n_crs + r];
-        const double w = j * mass[md];
-        const double tr = x[0] + x[1] + x[2];
-        const double ss2 = x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + 2 * (x[3] * x[3] + x[4] * x[4] + x[5] * x[5]);
-        ek += w * 0.5 * rho * (x[6] * x[6] + x[7] * x[7] + x[8] * x[8]);
-        es += w * 0.5 * (c1 * ss2 - c2 * tr * tr);
-      }
-    }
-  }
-  sk[t] = ek;
-  ss[t] = es;
-  __syncthreads();
-  if (t < n_crs) {
-    double k = 0, s2 = 0;
-    for (int i = 0; i < mstep; i++) {
-      k += sk[i * n_crs + t];
-      s2 += ss[i * n_crs + t];
-    }
-    part[(size_t)blockIdx.x * 2 * n_crs + t] = k;
-    part[(size_t)blockIdx.x * 2 * n_crs + n_crs + t] = s2;
-  }
-}
-}  // namespace
-
-extern "C" int edge_el_energy(edge_el_solver* s, const void* dofs, double* kinetic, double* strain, void* stream) {
-  if (!s) return edge::fail(EDGE_ERR_ARG, "solver handle missing");
-  if (!s->jdet || !s->mat) return edge::fail(EDGE_ERR_UNSUPPORTED, "the energy needs a solver built from materials");
-  if (!dofs) return edge::fail(EDGE_ERR_ARG, "device DOFs missing");
-  const int R = s->cfg.n_runs;
-  if (256 % R) return edge::fail(EDGE_ERR_UNSUPPORTED, "energy: runs must divide 256");
-  hipStream_t st = (hipStream_t)stream;
-  const unsigned nblk = 1024;
-  double* d_part = nullptr;
-  EDGE_HIP_TRY(hipMalloc(&d_part, sizeof(double) * 2 * R * nblk));
-  if (s->cfg.precision == 64)
-    hipLaunchKernelGGL(k_energy<double>, dim3(nblk), dim3(256), 0, st, s->n_el, s->n_modes, R, s->jdet, s->mass,
-                       s->mat, (const double*)dofs, d_part);
-  else
-    hipLaunchKernelGGL(k_energy<float>, dim3(nblk), dim3(256), 0, st, s->n_el, s->n_modes, R, s->jdet, s->mass,
-                       s->mat, (const float*)dofs, d_part);
-  int rc = EDGE_OK;
-  std::vector<double> h(2 * R * nblk);
-  if (hipGetLastError() != hipSuccess ||
-      hipMemcpyAsync(h.data(), d_part, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st) != hipSuccess ||
-      hipStreamSynchronize(st) != hipSuccess)
-    rc = edge::fail(EDGE_ERR_HIP, "energy reduction");
-  (void)hipFree(d_part);
-  if (rc) return rc;
-  for (int r = 0; r < R; r++) {
-    double k = 0, e = 0;
-    for (unsigned b = 0; b < nblk; b++) {
-      k += h[(size_t)b * 2 * R + r];
-      e += h[(size_t)b * 2 * R + R + r];
-    }
-    if (kinetic) kinetic[r] = k;
-    if (strain) strain[r] = e;
-  }
-  return EDGE_OK;
-}
-
-namespace {
-// Per-block L1, squared L2 and Linf errors per (quantity, run) at the
-// quadrature points of every element against a sum of plane waves
-// q(x, t) = sum_w r_w sin(k_w . x - omega_w t + phase_w) (per run:
-// waves [R][n_waves][14] = r[9], k[3], omega, phase).  Thread t keeps entry
-// t % (9 R) for elements t / (9 R), t / (9 R) + lanes, ... of the block's
-// range; partials summed in a fixed order.
-template <typename T>
-__global__ __launch_bounds__(256) void k_err(int64_t n_el, int n_md, int n_crs, int n_pts, const double* __restrict__ geo,
-                                             const double* __restrict__ jdet, const double* __restrict__ pts,
-                                             const double* __restrict__ wts, const double* __restrict__ basis,
-                                             int n_waves, const double* __restrict__ waves, double time,
-                                             const T* __restrict__ dofs, double* __restrict__ part) {
-  __shared__ double s1[256], s2[256], si[256];
-  const int nqr = 9 * n_crs, lanes = blockDim.x / nqr;
-  const int tid = threadIdx.x, qr = tid % nqr, sub = tid / nqr, q = qr / n_crs, r = qr % n_crs;
-  const int64_t per = (n_el + gridDim.x - 1) / gridDim.x;
-  const int64_t e0 = blockIdx.x * per, e1 = min(n_el, e0 + per);
-  double l1 = 0, l2 = 0, li = 0;
-  if (sub < lanes) {
-    for (int64_t el = e0 + sub; el < e1; el += lanes) {
-      const double* gm = geo + el * 12;
-      const double j = fabs(jdet[el]);
-      const T* a = dofs + ((size_t)el * 9 + q) * n_md * n_crs + r;
-      for (int p = 0; p < n_pts; p++) {
-        double num = 0;
-        for (int n = 0; n < n_md; n++) num += basis[p * n_md + n] * (double)a[(size_t)n * n_crs];
-        double x[3];
-        for (int d = 0; d < 3; d++)
-          x[d] = gm[d] + pts[3 * p] * gm[3 + d] + pts[3 * p + 1] * gm[6 + d] + pts[3 * p + 2] * gm[9 + d];
-        double ref = 0;
-        for (int w = 0; w < n_waves; w++) {
-          const double* wv = waves + ((size_t)r * n_waves + w) * 14;
-          ref += wv[q] * sin(wv[9] * x[0] + wv[10] * x[1] + wv[11] * x[2] - wv[12] * time + wv[13]);
-        }
-        const double d = fabs(num - ref), wj = wts[p] * j;
-        l1 += wj * d;
-        l2 += wj * d * d;
-        li = fmax(li, d);
-      }
-    }
-  }
-  s1[tid] = l1;
-  s2[tid] = l2;
-  si[tid] = li;
-  __syncthreads();
-  if (tid < nqr) {
-    double a1 = 0, a2 = 0, ai = 0;
-    for (int k = 0; k < lanes; k++) {
-      a1 += s1[k * nqr + tid];
-      a2 += s2[k * nqr + tid];
-      ai = fmax(ai, si[k * nqr + tid]);
-    }
-    part[((size_t)blockIdx.x * 3 + 0) * nqr + tid] = a1;
-    part[((size_t)blockIdx.x * 3 + 1) * nqr + tid] = a2;
-    part[((size_t)blockIdx.x * 3 + 2) * nqr + tid] = ai;
-  }
-}
-}  // namespace
-
-extern "C" int edge_el_error_norms(edge_el_solver* s, const void* dofs, int32_t n1d, int32_t n_waves,
-                                   const double* waves, double time, double* l1, double* l2sq, double* linf,
-                                   void* stream) {
-  if (!s) return edge::fail(EDGE_ERR_ARG, "solver handle missing");
-  if (!s->jdet || !s->geo) return edge::fail(EDGE_ERR_UNSUPPORTED, "error norms need a solver built from geometry");
-  if (!dofs || n_waves < 0 || (n_waves > 0 && !waves) || n1d < 0 || n1d > 32)
-    return edge::fail(EDGE_ERR_ARG, "error-norm arguments");
-  const int R = s->cfg.n_runs, nqr = 9 * R, N = s->n_modes;
-  if (nqr > 256) return edge::fail(EDGE_ERR_UNSUPPORTED, "error norms: at most 28 runs");
-  const int n1 = n1d ? n1d : s->cfg.order + 1, np = n1 * n1 * n1;
-  std::vector<double> pts(3 * np), w(np), basis((size_t)np * N);
-  int rc = edge_dg_quad_tet(n1, pts.data(), w.data());
-  if (rc == EDGE_OK) rc = edge_dg_eval_basis(s->cfg.order, np, pts.data(), basis.data());
-  if (rc) return rc;
-  hipStream_t st = (hipStream_t)stream;
-  const unsigned nblk = 1024;
-  double *d_pts = nullptr, *d_w = nullptr, *d_b = nullptr, *d_wv = nullptr, *d_part = nullptr;
-  const size_t nwv = (size_t)R * n_waves * 14;
-  auto ok = [](hipError_t e) { return e == hipSuccess; };
-  std::vector<double> h((size_t)3 * nqr * nblk);
-  if (!ok(hipMalloc(&d_pts, sizeof(double) * 3 * np)) || !ok(hipMalloc(&d_w, sizeof(double) * np)) ||
-      !ok(hipMalloc(&d_b, sizeof(double) * np * N)) || !ok(hipMalloc(&d_wv, sizeof(double) * (nwv ? nwv : 1))) ||
-      !ok(hipMalloc(&d_part, sizeof(double) * h.size())) ||
-      !ok(hipMemcpyAsync(d_pts, pts.data(), sizeof(double) * 3 * np, hipMemcpyHostToDevice, st)) ||
-      !ok(hipMemcpyAsync(d_w, w.data(), sizeof(double) * np, hipMemcpyHostToDevice, st)) ||
-      !ok(hipMemcpyAsync(d_b, basis.data(), sizeof(double) * np * N, hipMemcpyHostToDevice, st)) ||
-      (nwv && !ok(hipMemcpyAsync(d_wv, waves, sizeof(double) * nwv, hipMemcpyHostToDevice, st)))) {
-    rc = edge::fail(EDGE_ERR_HIP, "error norms: buffers");
-  } else {
-    if (s->cfg.precision == 64)
-      hipLaunchKernelGGL(k_err<double>, dim3(nblk), dim3(256), 0, st, s->n_el, N, R, np, s->geo, s->jdet, d_pts, d_w,
-                         d_b, n_waves, d_wv, time, (const double*)dofs, d_part);
-    else
-      hipLaunchKernelGGL(k_err<float>, dim3(nblk), dim3(256), 0, st, s->n_el, N, R, np, s->geo, s->jdet, d_pts, d_w,
-                         d_b, n_waves, d_wv, time, (const float*)dofs, d_part);
-    if (!ok(hipGetLastError()) ||
-        !ok(hipMemcpyAsync(h.data(), d_part, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st)) ||
-        !ok(hipStreamSynchronize(st)))
-      rc = edge::fail(EDGE_ERR_HIP, "error-norm reduction");
-  }
-  (void)hipFree(d_pts);
-  (void)hipFree(d_w);
-  (void)hipFree(d_b);
-  (void)hipFree(d_wv);
-  (void)hipFree(d_part);
-  if (rc) return rc;
-  for (int i = 0; i < nqr; i++) {
-    double a1 = 0, a2 = 0, ai = 0;
-    for (unsigned b = 0; b < nblk; b++) {
-      a1 += h[((size_t)b * 3 + 0) * nqr + i];
-      a2 += h[((size_t)b * 3 + 1) * nqr + i];
-      ai = std::max(ai, h[((size_t)b * 3 + 2) * nqr + i]);
-    }
-    if (l1) l1[i] = a1;
-    if (l2sq) l2sq[i] = a2;
-    if (linf) linf[i] = ai;
-  }
   return EDGE_OK;
 }
