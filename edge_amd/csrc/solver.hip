@@ -377,6 +377,13 @@ int finish_sp(edge_el_solver* s) {
   const bool f32 = s->cfg.precision == 32;
   const int rc = f32 ? upload_as<float>(pk, &s->sp_rot) : upload_as<double>(pk, &s->sp_rot);
   if (rc) return rc;
+  const bool stands_in = s->cfg.kernel == 0 && s->kernel == 1;
+  if (stands_in &&
+      hipMalloc(&s->proj, s->real_bytes * edge::sp_proj_values(s->cfg.order, s->cfg.n_runs) * s->n_el) != hipSuccess) {
+    (void)hipGetLastError();  // no room for projections: the general kernels need none
+    s->proj = nullptr;
+    return EDGE_OK;
+  }
   s->sp_ok = true;
   if (!s->h_fault_ef.empty()) {
     std::vector<uint8_t> need(s->n_el, 0);
@@ -384,10 +391,7 @@ int finish_sp(edge_el_solver* s) {
     EDGE_HIP_TRY(hipMalloc(&s->sp_need, s->n_el));
     EDGE_HIP_TRY(hipMemcpy(s->sp_need, need.data(), s->n_el, hipMemcpyHostToDevice));
   }
-  if (s->cfg.kernel == 0 && s->kernel == 1) {
-    EDGE_HIP_TRY(hipMalloc(&s->proj, s->real_bytes * edge::sp_proj_values(s->cfg.order, s->cfg.n_runs) * s->n_el));
-    s->kernel = 5;
-  }
+  if (stands_in) s->kernel = 5;
   return EDGE_OK;
 }
 
@@ -482,6 +486,12 @@ bool proj_active(const edge_el_solver* s) {
 // The sparse kernels run this solver's steps.
 bool sp_active(const edge_el_solver* s) { return s->sp_ok && s->n_rms == 0 && proj_active(s); }
 
+// Solvers of several runs whose general kernels read tInt in the neighbour
+// step (kernel 5 stands in for them): separate neighbour steps still do, so
+// that a caller may hand them another tInt or change it in between; the
+// projections are for the steps of edge_el_step.
+bool reads_tint(const edge_el_solver* s) { return s->kernel == 5 && s->cfg.n_runs > 1; }
+
 // A local step that writes projections records the tInt array it wrote.
 void note_local(edge_el_solver* s, const void* t_int) {
   if (!proj_active(s)) return;
@@ -524,9 +534,12 @@ int local_t(edge_el_solver* s, int64_t first, int64_t n, double dt, void* dofs, 
 }
 
 template <typename T>
-int neigh_t(edge_el_solver* s, int64_t first, int64_t n, const void* t_int, void* dofs, hipStream_t st) {
+int neigh_t(edge_el_solver* s, int64_t first, int64_t n, const void* t_int, void* dofs, hipStream_t st,
+            bool own_local = false) {
   if (s->n_rms > 0) return edge::fail(EDGE_ERR_ARG, "viscoelastic solver: the step needs dofs_a (edge_el_neigh_a)");
   const auto d = dev_view<T>(s);
+  if (reads_tint(s) && !own_local)
+    return edge::launch_neigh_generic<T>(d, first, n, (const T*)t_int, (T*)dofs, st);
   if (int rc = check_neigh(s, t_int)) return rc;
   if (sp_active(s)) return edge::launch_neigh_sp<T>(d, sp_view<T>(s), first, n, (T*)dofs, st);
   if (s->kernel == 2) return edge::launch_neigh_mfma<T>(d, first, n, (const T*)t_int, (T*)dofs, st);
@@ -580,13 +593,13 @@ int neigh_lts_t(edge_el_solver* s, int64_t first, int64_t n, int first_ts, const
   auto d = dev_view<T>(s);
   d.nb.ne = s->ne_lts;
   if (d.rcv) d.rcv = s->rcv_lts;
-  int rc = check_neigh(s, t0);
+  int rc = reads_tint(s) ? EDGE_OK : check_neigh(s, t0);
   if (rc) return rc;
-  if (sp_active(s))
+  if (sp_active(s) && !reads_tint(s))
     rc = edge::launch_neigh_sp<T>(d, sp_view<T>(s), first, n, (T*)dofs, st);
   else if (s->kernel == 2)
     rc = edge::launch_neigh_mfma<T>(d, first, n, (const T*)t0, (T*)dofs, st);
-  else if (s->kernel == 5)
+  else if (s->kernel == 5 && !reads_tint(s))
     rc = edge::launch_neigh_ec<T>(d, ec_view<T>(s), first, n, (T*)dofs, st);
   else if constexpr (sizeof(T) == 8)
     rc = s->kernel == 4 ? edge::launch_neigh_plain64(d, first, n, (const double*)t0, (double*)dofs, st)
@@ -651,8 +664,8 @@ int one_step(edge_el_solver* s, double dt, void* dofs, void* dofs_a, void* t_int
                                   : local_t<float>(s, 0, s->n_el, dt, dofs, t_int, st);
   if (rc) return rc;
   if (s->fault && (rc = edge::fault_apply(s->fault, dt, t_int, dofs, st))) return rc;
-  return s->cfg.precision == 64 ? neigh_t<double>(s, 0, s->n_el, t_int, dofs, st)
-                                : neigh_t<float>(s, 0, s->n_el, t_int, dofs, st);
+  return s->cfg.precision == 64 ? neigh_t<double>(s, 0, s->n_el, t_int, dofs, st, true)
+                                : neigh_t<float>(s, 0, s->n_el, t_int, dofs, st, true);
 }
 
 // Multi-step calls of FP32 MFMA elastic solvers that exchange face
@@ -674,22 +687,38 @@ size_t proj_alt_bytes(const edge_el_solver* s) {
   return s->kernel == 2 ? std::max(sp, sizeof(float) * 4 * 768 * s->n_el) : sp;
 }
 
+// The second buffer of projections, allocated on first use.  Kernel 5 steps
+// without it (launch by launch) where it cannot be had: out of memory, or on
+// a stream that the caller is capturing.
+bool sp_second_buffer(edge_el_solver* s, hipStream_t st) {
+  if (s->proj_alt || s->kernel == 2) return true;
+  hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &c) == hipSuccess && c == hipStreamCaptureStatusNone &&
+      hipMalloc(&s->proj_alt, proj_alt_bytes(s)) == hipSuccess)
+    return true;
+  (void)hipGetLastError();
+  s->proj_alt = nullptr;
+  return false;
+}
+
 // One local launch, n_steps - 1 fused ones and the last neighbour launch;
 // only the last step's tInt is the caller's (and, in every step, that of
-// elements on a fault).
+// elements on a fault).  The last step's projections are the solver's first
+// buffer, as after separate launches.
 template <typename T>
 int sp_steps(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* t_int, hipStream_t st) {
   auto d = dev_view<T>(s);
   auto x = sp_view<T>(s);
   if (s->kernel == 5) d.tap = nullptr;  // taps: the 16-run fused launches
   T* P[2] = {x.proj, static_cast<T*>(s->proj_alt)};
+  const int64_t last = n_steps - 1;
   x.need = s->fault ? s->sp_need : nullptr;
   int rc = EDGE_OK;
   for (int64_t k = 0; k < n_steps && rc == EDGE_OK; k++) {
-    x.proj = P[k % 2];
-    x.tint = k + 1 == n_steps || (s->fault && !s->sp_need);
+    x.proj = P[(last - k) % 2];
+    x.tint = k == last || (s->fault && !s->sp_need);
     rc = k == 0 ? edge::launch_local_sp<T>(d, x, 0, s->n_el, (T)dt, (T*)dofs, (T*)t_int, st)
-                : edge::launch_fused_sp<T>(d, x, (T)dt, P[(k - 1) % 2], (T*)dofs, (T*)t_int, st);
+                : edge::launch_fused_sp<T>(d, x, (T)dt, P[(last - k + 1) % 2], (T*)dofs, (T*)t_int, st);
     if (rc == EDGE_OK && s->fault) rc = edge::fault_apply(s->fault, dt, t_int, dofs, st);
   }
   return rc ? rc : edge::launch_neigh_sp<T>(d, x, 0, s->n_el, (T*)dofs, st);
@@ -723,8 +752,9 @@ int fused_steps(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void*
     return edge::fail(EDGE_ERR_UNSUPPORTED, "fused steps: FP32 MFMA solvers, 16 elastic or 8 viscoelastic runs");
   if (!s->proj_alt) EDGE_HIP_TRY(hipMalloc(&s->proj_alt, proj_alt_bytes(s)));
   // the projection buffers no longer stand for a tInt array a separate
-  // neighbour step could be handed
-  s->proj_tint = nullptr;
+  // neighbour step could be handed (kernel 5: for the last step's)
+  s->proj_tint = s->kernel == 5 ? t_int : nullptr;
+  s->proj_mixed = false;
   s->proj_fresh = false;
   if (s->n_rms > 0) return fused_steps_a(s, n_steps, dt, dofs, dofs_a, t_int, st);
   if (sp)
@@ -800,8 +830,12 @@ extern "C" int edge_el_create(const edge_el_config* cfg, const edge_mesh_in* mes
                         lam,         mu};
     s->sparse_star = true;  // built from the Jacobians' pattern only
     const int pb = edge::phys::block(cfg->n_runs);
-    if (hipMalloc(&s->jdet, sizeof(double) * s->n_el) != hipSuccess ||
-        (s->want_sp && hipMalloc(&s->sp_phys, s->real_bytes * edge::phys::values(s->n_el, pb)) != hipSuccess))
+    if (s->want_sp && hipMalloc(&s->sp_phys, s->real_bytes * edge::phys::values(s->n_el, pb)) != hipSuccess) {
+      (void)hipGetLastError();  // no room: the other kernels run without these constants
+      s->sp_phys = nullptr;
+      s->want_sp = false;
+    }
+    if (hipMalloc(&s->jdet, sizeof(double) * s->n_el) != hipSuccess)
       rc = edge::fail(EDGE_ERR_HIP, "allocation of the element constants");
     else
       rc = cfg->precision == 64
@@ -1142,7 +1176,7 @@ extern "C" int edge_el_kernel_info(const edge_el_solver* s, int32_t* kernel, int
   if (kernel) *kernel = s->kernel;
   if (flags) {
     const bool r3 = (s->kernel == 2 || s->kernel == 5) && s->fs_rank3 && s->fsf;
-    *flags = (s->sparse_star ? 1 : 0) | (r3 ? 2 : 0) | (proj_active(s) ? 4 : 0) |
+    *flags = (s->sparse_star ? 1 : 0) | (r3 ? 2 : 0) | (proj_active(s) && !reads_tint(s) ? 4 : 0) |
              (s->n_rms > 0 ? 8 : 0) | (fused_active(s) ? 16 : 0) | (s->hi_occ ? 32 : 0);
   }
   return EDGE_OK;
@@ -1435,7 +1469,8 @@ namespace {
 int step_impl(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* dofs_a, void* t_int, int use_graph,
               hipStream_t st) {
   if (n_steps == 0) return EDGE_OK;
-  const bool fuse = n_steps >= 2 && (fused_active(s) || sp_fuses(s)) && (s->n_rms > 0) == (dofs_a != nullptr);
+  const bool fuse = n_steps >= 2 && (fused_active(s) || (sp_fuses(s) && sp_second_buffer(s, st))) &&
+                    (s->n_rms > 0) == (dofs_a != nullptr);
   if (fuse && !s->proj_alt) EDGE_HIP_TRY(hipMalloc(&s->proj_alt, proj_alt_bytes(s)));
   if (!use_graph && fuse) return fused_steps(s, n_steps, dt, dofs, dofs_a, t_int, st);
   if (!use_graph) {
@@ -1486,7 +1521,8 @@ int step_impl(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* d
     s->graph_steps = gsteps;
   }
   if (gsteps) {
-    s->proj_tint = nullptr;  // as after an eager fused sequence
+    s->proj_tint = s->kernel == 5 ? t_int : nullptr;  // as after an eager fused sequence
+    s->proj_mixed = false;
     s->proj_fresh = false;
     EDGE_HIP_TRY(hipGraphLaunch(s->graph_exec, st));
     return EDGE_OK;

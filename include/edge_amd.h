@@ -220,7 +220,10 @@ int edge_el_neigh(edge_el_solver *s, int64_t first, int64_t n_els, const void *t
  * is one graph (recaptured when n_steps changes).  An attached fault's phase
  * runs between the launches.  The DOFs are those of n_steps full steps
  * either way; after the call t_int holds the last step's tInt and no
- * separate edge_el_neigh may follow. */
+ * separate edge_el_neigh may follow.  Kernel 5 over the matrices' non-zeros
+ * fuses the same way (a separate edge_el_neigh may follow); without room for
+ * its second buffer, or with none yet on a stream that the caller captures,
+ * it steps launch by launch. */
 int edge_el_step(edge_el_solver *s, int64_t n_steps, double dt, void *dofs, void *t_int, int use_graph,
                  void *stream);
 
@@ -497,7 +500,10 @@ int edge_el_neigh_lts_a(edge_el_solver *s, int64_t first, int64_t n_els, int32_t
 
 /* Which kernels a solver runs: *kernel = 1 (generic), 2 (MFMA-tiled, runs
  * on the MFMA N dimension), 4 (FP64 single run on FP64 MFMA, quantities on
- * the M dimension) or 5 (single run, 16 elements on the N dimension);
+ * the M dimension) or 5 (single run, 16 elements on the N dimension, or the
+ * kernels over the matrices' non-zeros, which geometry-built elastic solvers
+ * run as 2 with projections, as 5 and, of 8 runs or FP64 with 16, instead of
+ * 1: those report 5 and their edge_el_neigh reads t_int);
  * *flags bit 0: sparse (elastic-pattern) star matrices, bit 1: rank-3
  * factored flux solvers, bit 2: the neighbour step reads face projections,
  * bit 3: viscoelastic (anelastic DOFs), bit 4: multi-step calls fuse the

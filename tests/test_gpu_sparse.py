@@ -106,3 +106,61 @@ def test_neighbours_that_do_not_pair(gpu, runs):
     s.step(gd, gt, dt, 2)
     assert rel(gd.cpu().numpy(), d) <= TOL[32]
     s.close()
+
+
+@pytest.mark.parametrize("precision,runs", [(32, 8), (64, 8), (64, 16)])
+def test_neighbour_step_reads_tint(gpu, precision, runs):
+    """Solvers whose general kernels read tInt: a separate neighbour step takes
+    what it is handed, changed since the local step, in another array, after a
+    multi-step call or without any local step."""
+    import torch
+    order, tol = 3, TOL[precision]
+    m, mat, dt, d, gd = _problem(runs, order, precision)
+    s = ElasticSolver(m, order, runs, precision, *mat)
+    assert s.kernel_info() == (5, 1)
+    mo = orc.MeshOracle(m, order, runs, rho=mat[0], lam=mat[1], mu=mat[2])
+    t, gt = np.zeros_like(d), torch.zeros_like(gd)
+    t2 = (np.random.default_rng(8).normal(size=d.shape) * dt).astype(NP[precision])
+    mo.neigh(d, t2.astype(np.float64))
+    s.neigh(gd, torch.from_numpy(t2).cuda())
+    assert rel(gd.cpu().numpy(), d) <= tol
+    mo.local(d, t, dt)
+    s.local(gd, gt, dt)
+    gt *= 0.5
+    mo.neigh(d, 0.5 * t)
+    s.neigh(gd, gt)
+    assert rel(gd.cpu().numpy(), d) <= tol
+    mo.step(d, t, dt, 2)
+    s.step(gd, gt, dt, 2)
+    mo.neigh(d, t)
+    s.neigh(gd, gt)
+    assert rel(gd.cpu().numpy(), d) <= tol
+    s.close()
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_one_run_after_and_under_capture(gpu, precision):
+    """One run: multi-step calls captured by the caller before the second
+    projection buffer exists (they go launch by launch), replayed between eager
+    work; and a neighbour step after a multi-step call, eager and as a graph."""
+    import torch
+    order, tol = 4, TOL[precision]
+    m, mat, dt, d, gd = _problem(1, order, precision)
+    s = ElasticSolver(m, order, 1, precision, *mat)
+    mo = orc.MeshOracle(m, order, 1, rho=mat[0], lam=mat[1], mu=mat[2])
+    t, gt = np.zeros_like(d), torch.zeros_like(gd)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        s.step(gd, gt, dt, 2, stream=torch.cuda.current_stream())
+    for _ in range(3):
+        g.replay()
+        torch.cuda.synchronize()
+        mo.step(d, t, dt, 2)
+        assert rel(gd.cpu().numpy(), d) <= tol
+    for n, graph in ((2, False), (3, False), (3, True), (2, True)):
+        s.step(gd, gt, dt, n, graph=graph)
+        mo.step(d, t, dt, n)
+        s.neigh(gd, gt)
+        mo.neigh(d, t)
+        assert rel(gd.cpu().numpy(), d) <= tol
+    s.close()
