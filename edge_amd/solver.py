@@ -53,7 +53,7 @@ class ElasticSolver:
 
     # ------------------------------------------------------------------
     def kernel_info(self):
-        """(kernel, flags): 1 generic / 2 MFMA-tiled / 4 FP64 MFMA / 5 element-batched; flags PATH_* bits."""
+        """(kernel, flags): 1 generic / 2 MFMA-tiled / 4 FP64 MFMA / 5 element-batched or sparse; flags PATH_* bits."""
         k, f = C.c_int32(), C.c_int32()
         _lib.check(_lib.lib().edge_el_kernel_info(self._h, C.byref(k), C.byref(f)))
         return k.value, f.value
