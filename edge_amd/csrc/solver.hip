@@ -356,13 +356,15 @@ int finish_ec(edge_el_solver* s) {
 
 // The sparse kernels' data, once the flux solvers exist: geometry-built
 // solvers (their constants are in sp_phys) whose faces pair up, with one
-// projection slot per element face.  Runs of 8 have no other tuned kernel:
-// they take these as the element-batched kernels.
+// projection slot per element face.  One run exchanges its projections through
+// the element-batched kernels' buffer: without their data it stays on the
+// general kernels.  Runs of 8 have no other tuned kernel: they take these as
+// the element-batched kernels.
 int finish_sp(edge_el_solver* s) {
   if (!s->want_sp) return EDGE_OK;
   edge::DgTables t;
   std::vector<double> rot;
-  if (!s->proj_ok || !s->faces_agree || !edge::dg_tables(s->cfg.order, &t) || !edge::ec_rotations(t, &rot)) {
+  if ((s->cfg.n_runs == 1 && !s->ec_ok) || !s->proj_ok || !s->faces_agree || !edge::dg_tables(s->cfg.order, &t) || !edge::ec_rotations(t, &rot)) {
     (void)hipFree(s->sp_phys);
     s->sp_phys = nullptr;
     return EDGE_OK;

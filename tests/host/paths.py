@@ -1,0 +1,142 @@
+"""What the library's host code does with a solver, seen on the CPU with the
+runtime of fake_hip.cpp: which kernels run, on which stream, with which
+buffers.  Run as a program with the runtime's library and a scenario's name
+(tests/test_host_paths.py builds the one and runs the others)."""
+import ctypes as C
+import os
+import re
+import sys
+
+import numpy as np
+
+sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__)))))
+FAKE = None
+DOFS, DOFS2, TINT, TINT2 = 0x100000, 0x200000, 0x300000, 0x400000  # stand for device arrays: nothing reads them
+
+
+def start(lib):
+    """Loads the fake runtime, then the library, whose HIP calls resolve to it."""
+    global FAKE
+    FAKE = C.CDLL(lib, mode=C.RTLD_GLOBAL)
+    FAKE.fake_log.restype = C.c_char_p
+    FAKE.fake_live.restype = FAKE.fake_bytes.restype = FAKE.fake_size.restype = C.c_size_t
+    FAKE.fake_size.argtypes = FAKE.fake_capturing.argtypes = [C.c_void_p]
+
+
+class Launch:
+    def __init__(self, line):
+        self.kernel, self.args = line.split()[1], dict(a.split("=") for a in line.split()[2:])
+        self.stream = int(self.args["stream"], 16)
+        m = re.search(r"(k_[a-z0-9_]+?)(?=[IiPvfdx])", self.kernel)
+        self.name = m.group(1) if m else self.kernel
+        m = re.search(r"k_sparseI(.)Li(\d)ELi(\d+)ELb(\d)ELb(\d)E", self.kernel)
+        if m:
+            self.name = "sparse " + {"01": "local", "10": "neigh", "11": "fused"}[m.group(4) + m.group(5)]
+
+    def addr(self, what):
+        return int(self.args[what], 16)
+
+
+def events():
+    """The runtime calls noted since the last time, in order."""
+    out = []
+    for line in FAKE.fake_log().decode().splitlines():
+        assert not line.startswith("free of"), line
+        out.append(Launch(line) if line.startswith("launch") else tuple(line.replace("stream=", "").split()))
+    FAKE.fake_clear()
+    return out
+
+
+def launches():
+    return [e for e in events() if isinstance(e, Launch)]
+
+
+def names():
+    return [e.name for e in launches()]
+
+
+def mesh(n=(3, 4, 3), **kw):
+    from edge_amd import mesh as M
+    return M.box(n, jitter=0.1, seed=5, **kw)
+
+
+class Solver:
+    def __init__(self, m, order, runs, precision, kernel=0):
+        from edge_amd import _lib
+        from edge_amd import setups as S
+        self.L, self.m = _lib.lib(), m
+        h, mi = C.c_void_p(), m.mesh_in()
+        mat = [np.ascontiguousarray(a, np.float64) for a in S.random_materials(m.n_el, seed=5)]
+        self.rc = self.L.edge_el_create(C.byref(_lib.ElConfig(order, runs, precision, kernel)), C.byref(mi),
+                                        *[a.ctypes.data for a in mat], C.byref(h))
+        self.h = h
+
+    def info(self):
+        k, f = C.c_int32(), C.c_int32()
+        assert self.L.edge_el_kernel_info(self.h, C.byref(k), C.byref(f)) == 0
+        return k.value, f.value
+
+    def local(self, dofs=DOFS, t_int=TINT, stream=None):
+        return self.L.edge_el_local(self.h, 0, self.m.n_el, 1e-3, dofs, t_int, stream)
+
+    def neigh(self, dofs=DOFS, t_int=TINT, stream=None):
+        return self.L.edge_el_neigh(self.h, 0, self.m.n_el, t_int, dofs, stream)
+
+    def step(self, n, dofs=DOFS, t_int=TINT, stream=None, graph=0):
+        return self.L.edge_el_step(self.h, n, 1e-3, dofs, t_int, graph, stream)
+
+    def variant(self, kernel, flags):
+        return self.L.edge_el_set_variant(self.h, kernel, flags)
+
+    def close(self):
+        assert self.L.edge_el_destroy(self.h) == 0
+
+
+def one_run_without_factors():
+    """One run whose flux solvers are found not to have rank 3: the element-
+    batched data (and its projections) does not exist, so neither the default
+    nor a variant may run on it, and no launch gets a null buffer."""
+    for precision, order in ((32, 5), (32, 2), (64, 4), (64, 5)):
+        FAKE.fake_setup_flags(8)
+        s = Solver(mesh(), order, 1, precision)
+        FAKE.fake_setup_flags(0)
+        assert s.rc == 0
+        assert s.info()[0] == (1 if precision == 32 else 4)
+        assert s.variant(5, 3) != 0 and s.variant(5, 1) != 0
+        events()
+        for rc in (s.local(), s.neigh(), s.step(1), s.step(3)):
+            assert rc == 0
+        for e in launches():
+            assert e.name != "sparse local" and e.name != "sparse neigh" and e.name != "sparse fused", e.kernel
+        s.close()
+        assert FAKE.fake_live() == 0
+
+
+def projections_exist():
+    """Every launch of the sparse kernels has its constants, maps and
+    projections, and a buffer large enough for them."""
+    for precision, order, runs in ((32, 5, 1), (32, 3, 8), (32, 4, 16), (64, 4, 1), (64, 3, 8), (64, 4, 16)):
+        s = Solver(mesh(), order, runs, precision)
+        assert s.rc == 0
+        events()
+        for rc in (s.step(1), s.step(2), s.step(5)):
+            assert rc == 0
+        ls = launches()
+        nv = (3 * order * (order + 1) // 2 + 3) // 4
+        need = 16 * nv * runs * precision // 8 * s.m.n_el
+        for e in ls:
+            assert e.name.startswith("sparse"), e.kernel
+            for a in ("phys", "rot"):
+                assert FAKE.fake_size(e.addr(a)) > 0
+            for a, used in (("proj", e.name != "sparse neigh"), ("proj_in", e.name != "sparse local")):
+                assert not used or FAKE.fake_size(e.addr(a)) >= need, (e.kernel, a)
+            assert e.name != "sparse fused" or e.addr("proj") != e.addr("proj_in")
+        assert [e.name.split()[1] for e in ls] == (["local", "neigh", "local", "fused", "neigh", "local"] +
+                                                   4 * ["fused"] + ["neigh"])
+        s.close()
+        assert FAKE.fake_live() == 0
+
+
+if __name__ == "__main__":
+    start(sys.argv[1])
+    globals()[sys.argv[2]]()
