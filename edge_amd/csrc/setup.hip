@@ -460,6 +460,7 @@ int build_setup(const SetupInput& in, T* d_star, T* d_fs, double* d_jdet, T* d_f
   // sentinel values: every (element, face) slot must be written by its face
   EDGE_SETUP_TRY(hipMemsetAsync(d_fs, 0xFF, sizeof(T) * 2 * 4 * 81 * ne, st));
   if (d_fs_a) EDGE_SETUP_TRY(hipMemsetAsync(d_fs_a, 0xFF, sizeof(T) * 2 * 4 * 54 * ne, st));
+  if (d_phys) EDGE_SETUP_TRY(hipMemsetAsync(d_phys, 0xFF, sizeof(T) * phys::values(ne, phys_block), st));
   const int bs = 128;
   hipLaunchKernelGGL(k_star<T>, dim3((unsigned)((ne + bs - 1) / bs)), dim3(bs), 0, st, ne, d_crds, d_elve, d_rho,
                      d_lam, d_mu, d_star, d_jdet, d_star_a, d_phys, phys_block, d_bad);

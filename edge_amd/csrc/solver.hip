@@ -72,7 +72,8 @@ struct edge_el_solver {
   // kernels (5) and as the MFMA kernels (2) with projections exchanged.
   bool want_sp = false;    // set-up builds their data when the mesh qualifies
   bool sp_ok = false;
-  bool faces_agree = true; // every interior face's two elements are each other's neighbours
+  bool faces_agree = true; // every interior face's two elements are each other's neighbours, free surfaces have one
+  bool frames_ok = true;   // every face's normal and tangents are orthonormal
   void* sp_phys = nullptr;
   void* sp_rot = nullptr;
   uint8_t* sp_need = nullptr;  // [nEl] elements on a fault: its phase reads their tInt in every step
@@ -227,6 +228,7 @@ int build_neigh(edge_el_solver* s, const edge_mesh_in* m) {
       } else if ((ty & EDGE_FA_FREE_SURFACE) == EDGE_FA_FREE_SURFACE) {
         nb[el * 4 + fa] = (int32_t)el;
         fm[el * 4 + fa] = (uint8_t)fa;
+        if (m->fa_el[f * 2 + 1] >= 0) s->faces_agree = false;
       } else {
         const int64_t n = m->el_fa_el[el * 4 + fa];
         const unsigned v = m->v_id[el * 4 + fa], fi = m->f_id[el * 4 + fa];
@@ -354,9 +356,28 @@ int finish_ec(edge_el_solver* s) {
   return EDGE_OK;
 }
 
+// The sparse kernels take a face's waves from its normal alone, which equals
+// the flux solvers T F T^-1 only where (normal, tangents) is orthonormal.  A
+// frame that is off by d moves the result by about d.  In FP64 1e-10 passes:
+// rounding alone leaves 1e-15 on a cube's jittered box and 5e-11 on one
+// stretched by 1e5.  In FP32 1e-6, a tenth of the bound that every path is
+// held to against the oracle.
+bool frames_orthonormal(const edge_mesh_in* m, int precision) {
+  const double tol = precision == 64 ? 1e-10 : 1e-6;
+  for (int64_t fa = 0; fa < m->n_fa; fa++) {
+    const double* f[3] = {m->normals + fa * 3, m->tangents + fa * 6, m->tangents + fa * 6 + 3};
+    for (int i = 0; i < 3; i++)
+      for (int j = 0; j <= i; j++) {
+        const double d = f[i][0] * f[j][0] + f[i][1] * f[j][1] + f[i][2] * f[j][2];
+        if (!(std::fabs(d - (i == j)) <= tol)) return false;  // (NaN: not orthonormal)
+      }
+  }
+  return true;
+}
+
 // The sparse kernels' data, once the flux solvers exist: geometry-built
-// solvers (their constants are in sp_phys) whose faces pair up, with one
-// projection slot per element face.  One run exchanges its projections through
+// solvers (their constants are in sp_phys) whose faces pair up and have
+// orthonormal frames, with one projection slot per element face.  One run exchanges its projections through
 // the element-batched kernels' buffer: without their data it stays on the
 // general kernels.  Runs of 8 have no other tuned kernel: they take these as
 // the element-batched kernels.
@@ -364,7 +385,8 @@ int finish_sp(edge_el_solver* s) {
   if (!s->want_sp) return EDGE_OK;
   edge::DgTables t;
   std::vector<double> rot;
-  if ((s->cfg.n_runs == 1 && !s->ec_ok) || !s->proj_ok || !s->faces_agree || !edge::dg_tables(s->cfg.order, &t) || !edge::ec_rotations(t, &rot)) {
+  if ((s->cfg.n_runs == 1 && !s->ec_ok) || !s->proj_ok || !s->faces_agree || !s->frames_ok ||
+      !edge::dg_tables(s->cfg.order, &t) || !edge::ec_rotations(t, &rot)) {
     (void)hipFree(s->sp_phys);
     s->sp_phys = nullptr;
     return EDGE_OK;
@@ -832,6 +854,7 @@ extern "C" int edge_el_create(const edge_el_config* cfg, const edge_mesh_in* mes
                         lam,         mu};
     s->sparse_star = true;  // built from the Jacobians' pattern only
     const int pb = edge::phys::block(cfg->n_runs);
+    s->frames_ok = !s->want_sp || frames_orthonormal(mesh, cfg->precision);
     if (s->want_sp && hipMalloc(&s->sp_phys, s->real_bytes * edge::phys::values(s->n_el, pb)) != hipSuccess) {
       (void)hipGetLastError();  // no room: the other kernels run without these constants
       s->sp_phys = nullptr;

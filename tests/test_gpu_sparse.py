@@ -108,6 +108,30 @@ def test_neighbours_that_do_not_pair(gpu, runs):
     s.close()
 
 
+@pytest.mark.parametrize("form", ["skew frame", "long normal", "free surface inside"])
+@pytest.mark.parametrize("precision,runs", [(32, 1), (32, 8), (32, 16), (64, 1), (64, 8)])
+def test_general_forms_of_a_face(gpu, precision, runs, form):
+    """Faces that only their flux solvers describe: tangents or a normal off
+    the orthonormal frame, a free surface that two elements share."""
+    import torch
+    order = 3
+    m, mat, dt, d, gd = _problem(runs, order, precision)
+    f = np.argwhere((m.fa_el >= 0).all(axis=1) & (m.fa_type == 0))[17, 0]
+    if form == "skew frame":
+        m.tangents[f, 0] += 0.1 * m.tangents[f, 1]
+    elif form == "long normal":
+        m.normals[f] *= 1.01
+    else:
+        m.fa_type[f] = FA_FREE_SURFACE
+    s = ElasticSolver(m, order, runs, precision, *mat)
+    mo = orc.MeshOracle(m, order, runs, rho=mat[0], lam=mat[1], mu=mat[2])
+    t, gt = np.zeros_like(d), torch.zeros_like(gd)
+    mo.step(d, t, dt, 2)
+    s.step(gd, gt, dt, 2)
+    assert rel(gd.cpu().numpy(), d) <= TOL[precision]
+    s.close()
+
+
 @pytest.mark.parametrize("precision,runs", [(32, 8), (64, 8), (64, 16)])
 def test_neighbour_step_reads_tint(gpu, precision, runs):
     """Solvers whose general kernels read tInt: a separate neighbour step takes
