@@ -43,7 +43,9 @@ template <typename T>
 struct SpDev {
   const T* phys = nullptr;  // per-element constants
   const T* rot = nullptr;   // face-orientation maps
-  T* proj = nullptr;        // face projections [nEl][4][vectors][R][4] of this step
+  // face projections [nEl][4][vectors][R][4] of this step (a local step
+  // whose projections nothing reads: null)
+  T* proj = nullptr;
   // tInt is written for every element, or only for those of need (a step
   // whose tInt nothing else reads)
   bool tint = true;

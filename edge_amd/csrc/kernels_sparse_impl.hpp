@@ -935,7 +935,7 @@ __device__ __forceinline__ int64_t tile_index(int64_t n, bool xcd) {
 constexpr int waves_per_simd(int order, int bytes) { return order == 5 || bytes == 8 ? 2 : 3; }
 
 // NB: the neighbouring surface integral from the projections proj_in; LOC:
-// the local step (projections to x.proj).  Both: the neighbour step of the
+// the local step (projections to x.proj, of a local step alone: unless null).  Both: the neighbour step of the
 // previous time step first (its DOFs also go to s.tap for the elements
 // s.tap_on marks).
 template <typename T, int O, int R, bool NB, bool LOC>
@@ -1036,7 +1036,9 @@ __global__ __launch_bounds__(64 * kWaves, waves_per_simd(O, sizeof(T))) void k_s
 #pragma unroll
       for (int j = 0; j < M; j++) acc[q][j] = j < ML ? low[q][j < ML ? j : 0] : t[q][j];
     b.space(t, acc, dt);
-    b.send(x.proj);
+    // (one run and FP32 with 16: always, their neighbour steps read nothing else)
+    constexpr bool ALWAYS = NB || R == 1 || (R == 16 && sizeof(T) == 4);
+    if (ALWAYS || x.proj) b.send(x.proj);
     if constexpr (R == 1) {
       if (x.tint || x.need) b.template store<true>(t_int, t, on, dt);
       __syncthreads();

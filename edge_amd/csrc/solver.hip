@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <new>
 #include <utility>
 #include <vector>
@@ -76,6 +77,12 @@ struct edge_el_solver {
   bool frames_ok = true;   // every face's normal and tangents are orthonormal
   void* sp_phys = nullptr;
   void* sp_rot = nullptr;
+  // Several runs on kernel 5: calls may overlap on several streams and
+  // threads, as the general kernels allow that keep nothing in the handle.
+  // The projections of one call at a time are in flight: each call of
+  // edge_el_step waits for the event of the one before it.
+  std::mutex sp_mutex;
+  hipEvent_t sp_done = nullptr;
   uint8_t* sp_need = nullptr;  // [nEl] elements on a fault: its phase reads their tInt in every step
   // viscoelastic solvers
   int n_rms = 0;
@@ -518,7 +525,7 @@ bool reads_tint(const edge_el_solver* s) { return s->kernel == 5 && s->cfg.n_run
 
 // A local step that writes projections records the tInt array it wrote.
 void note_local(edge_el_solver* s, const void* t_int) {
-  if (!proj_active(s)) return;
+  if (!proj_active(s) || reads_tint(s)) return;
   if (!s->proj_fresh) {
     s->proj_tint = t_int;
     s->proj_mixed = false;
@@ -532,7 +539,7 @@ void note_local(edge_el_solver* s, const void* t_int) {
 // from local steps that wrote this very array (a substituted tInt, such as a
 // receive buffer, would be silently ignored otherwise).
 int check_neigh(edge_el_solver* s, const void* t_int) {
-  if (!proj_active(s)) return EDGE_OK;
+  if (!proj_active(s) || reads_tint(s)) return EDGE_OK;
   if (!s->proj_tint)
     return edge::fail(EDGE_ERR_ARG, "neighbour step: no local step has written the face projections since set-up "
                                     "or the last autotune (run the local step first)");
@@ -544,12 +551,18 @@ int check_neigh(edge_el_solver* s, const void* t_int) {
   return EDGE_OK;
 }
 
+// own_neigh / own_local: the other half of the step is the solver's own (one_step).
 template <typename T>
-int local_t(edge_el_solver* s, int64_t first, int64_t n, double dt, void* dofs, void* t_int, hipStream_t st) {
+int local_t(edge_el_solver* s, int64_t first, int64_t n, double dt, void* dofs, void* t_int, hipStream_t st,
+            bool own_neigh = false) {
   if (s->n_rms > 0) return edge::fail(EDGE_ERR_ARG, "viscoelastic solver: the step needs dofs_a (edge_el_local_a)");
   const auto d = dev_view<T>(s);
   note_local(s, t_int);
-  if (sp_active(s)) return edge::launch_local_sp<T>(d, sp_view<T>(s), first, n, (T)dt, (T*)dofs, (T*)t_int, st);
+  if (sp_active(s)) {
+    auto x = sp_view<T>(s);
+    if (reads_tint(s) && !own_neigh) x.proj = nullptr;
+    return edge::launch_local_sp<T>(d, x, first, n, (T)dt, (T*)dofs, (T*)t_int, st);
+  }
   if (s->kernel == 2) return edge::launch_local_mfma<T>(d, first, n, (T)dt, (T*)dofs, (T*)t_int, st);
   if (s->kernel == 5) return edge::launch_local_ec<T>(d, ec_view<T>(s), first, n, (T)dt, (T*)dofs, (T*)t_int, st);
   if constexpr (sizeof(T) == 8)
@@ -617,7 +630,7 @@ int neigh_lts_t(edge_el_solver* s, int64_t first, int64_t n, int first_ts, const
   auto d = dev_view<T>(s);
   d.nb.ne = s->ne_lts;
   if (d.rcv) d.rcv = s->rcv_lts;
-  int rc = reads_tint(s) ? EDGE_OK : check_neigh(s, t0);
+  int rc = check_neigh(s, t0);
   if (rc) return rc;
   if (sp_active(s) && !reads_tint(s))
     rc = edge::launch_neigh_sp<T>(d, sp_view<T>(s), first, n, (T*)dofs, st);
@@ -675,21 +688,22 @@ int neigh_lts_a_t(edge_el_solver* s, int64_t first, int64_t n, int first_ts, con
                                          st);
 }
 
-int one_step(edge_el_solver* s, double dt, void* dofs, void* dofs_a, void* t_int, hipStream_t st) {
+// own_proj: the step may exchange projections through the handle.
+int one_step(edge_el_solver* s, double dt, void* dofs, void* dofs_a, void* t_int, hipStream_t st,
+             bool own_proj = true) {
   // a whole step writes the projections its neighbour step reads: a local
   // step pending from before is superseded
-  s->proj_fresh = false;
-  s->proj_mixed = false;
+  if (!reads_tint(s)) s->proj_fresh = s->proj_mixed = false;
   if (s->n_rms > 0) {
     const int rc = edge_el_local_a(s, 0, s->n_el, dt, dofs, dofs_a, t_int, st);
     return rc ? rc : edge_el_neigh_a(s, 0, s->n_el, t_int, dofs, dofs_a, st);
   }
-  int rc = s->cfg.precision == 64 ? local_t<double>(s, 0, s->n_el, dt, dofs, t_int, st)
-                                  : local_t<float>(s, 0, s->n_el, dt, dofs, t_int, st);
+  int rc = s->cfg.precision == 64 ? local_t<double>(s, 0, s->n_el, dt, dofs, t_int, st, own_proj)
+                                  : local_t<float>(s, 0, s->n_el, dt, dofs, t_int, st, own_proj);
   if (rc) return rc;
   if (s->fault && (rc = edge::fault_apply(s->fault, dt, t_int, dofs, st))) return rc;
-  return s->cfg.precision == 64 ? neigh_t<double>(s, 0, s->n_el, t_int, dofs, st, true)
-                                : neigh_t<float>(s, 0, s->n_el, t_int, dofs, st, true);
+  return s->cfg.precision == 64 ? neigh_t<double>(s, 0, s->n_el, t_int, dofs, st, own_proj)
+                                : neigh_t<float>(s, 0, s->n_el, t_int, dofs, st, own_proj);
 }
 
 // Multi-step calls of FP32 MFMA elastic solvers that exchange face
@@ -953,6 +967,7 @@ extern "C" int edge_el_destroy(edge_el_solver* s) {
   (void)hipFree(s->sp_phys);
   (void)hipFree(s->sp_rot);
   (void)hipFree(s->sp_need);
+  if (s->sp_done) (void)hipEventDestroy(s->sp_done);
   drop_lts(s);
   delete s;
   return EDGE_OK;
@@ -1259,6 +1274,7 @@ extern "C" int edge_el_autotune(edge_el_solver* s, double dt, int32_t n_reps, vo
   const int old_kernel = s->kernel;
   const bool old_proj = s->use_proj, old_xcd = s->xcd_map, old_fused = s->use_fused, old_occ = s->hi_occ;
   std::vector<double> t(cand.size(), 0.0);
+  if (s->sp_done) EDGE_HIP_TRY(hipStreamWaitEvent(st, s->sp_done, 0));  // a step on another stream
   int rc = EDGE_OK;
   auto hip = [&](hipError_t e, const char* what) {
     if (e != hipSuccess && rc == EDGE_OK) rc = edge::fail(EDGE_ERR_HIP, std::string("autotune: ") + what + ": " +
@@ -1491,9 +1507,19 @@ extern "C" int edge_el_neigh_lts(edge_el_solver* s, int64_t first, int64_t n_els
 }
 
 namespace {
-int step_impl(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* dofs_a, void* t_int, int use_graph,
-              hipStream_t st) {
-  if (n_steps == 0) return EDGE_OK;
+// The projections of the handle (reads_tint solvers), for a call on st.
+int acquire_projections(edge_el_solver* s, hipStream_t st) {
+  if (!s->sp_done) EDGE_HIP_TRY(hipEventCreateWithFlags(&s->sp_done, hipEventDisableTiming));
+  else EDGE_HIP_TRY(hipStreamWaitEvent(st, s->sp_done, 0));
+  return EDGE_OK;
+}
+int release_projections(edge_el_solver* s, hipStream_t st) {
+  EDGE_HIP_TRY(hipEventRecord(s->sp_done, st));
+  return EDGE_OK;
+}
+
+int steps_on(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* dofs_a, void* t_int, int use_graph,
+             hipStream_t st) {
   const bool fuse = n_steps >= 2 && (fused_active(s) || (sp_fuses(s) && sp_second_buffer(s, st))) &&
                     (s->n_rms > 0) == (dofs_a != nullptr);
   if (fuse && !s->proj_alt) EDGE_HIP_TRY(hipMalloc(&s->proj_alt, proj_alt_bytes(s)));
@@ -1554,6 +1580,25 @@ int step_impl(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* d
   }
   for (int64_t i = 0; i < n_steps; i++) EDGE_HIP_TRY(hipGraphLaunch(s->graph_exec, st));
   return EDGE_OK;
+}
+
+int step_impl(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* dofs_a, void* t_int, int use_graph,
+              hipStream_t st) {
+  if (n_steps == 0) return EDGE_OK;
+  if (!reads_tint(s)) return steps_on(s, n_steps, dt, dofs, dofs_a, t_int, use_graph, st);
+  hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &c) != hipSuccess) (void)hipGetLastError();
+  if (!use_graph && c != hipStreamCaptureStatusNone) {
+    // the caller's graph may be replayed beside any other call: nothing of the handle in it
+    int rc = EDGE_OK;
+    for (int64_t i = 0; i < n_steps && rc == EDGE_OK; i++) rc = one_step(s, dt, dofs, dofs_a, t_int, st, false);
+    return rc;
+  }
+  std::lock_guard<std::mutex> lock(s->sp_mutex);
+  if (int rc = acquire_projections(s, st)) return rc;
+  const int rc = steps_on(s, n_steps, dt, dofs, dofs_a, t_int, use_graph, st);
+  const int rc2 = release_projections(s, st);  // also after an error: what was launched before it
+  return rc ? rc : rc2;
 }
 }  // namespace
 

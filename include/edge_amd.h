@@ -223,7 +223,14 @@ int edge_el_neigh(edge_el_solver *s, int64_t first, int64_t n_els, const void *t
  * separate edge_el_neigh may follow.  Kernel 5 over the matrices' non-zeros
  * fuses the same way (a separate edge_el_neigh may follow); without room for
  * its second buffer, or with none yet on a stream that the caller captures,
- * it steps launch by launch. */
+ * it steps launch by launch.
+ * Solvers that exchange face projections hold them in the handle, so calls
+ * on one handle that overlap on several streams would mix them up: order
+ * them.  The exception are the solvers whose edge_el_neigh reads t_int
+ * (flag bit 2 clear, kernel 5 included): their calls may overlap on several
+ * streams and threads, with DOF and tInt arrays of their own; edge_el_step
+ * lets one call after the other through on the device, and on a stream that
+ * the caller captures it steps launch by launch without the projections. */
 int edge_el_step(edge_el_solver *s, int64_t n_steps, double dt, void *dofs, void *t_int, int use_graph,
                  void *stream);
 

@@ -24,6 +24,9 @@ def start(lib):
 
 
 class Launch:
+    def __getitem__(self, i):
+        return "launch" if i == 0 else self.name
+
     def __init__(self, line):
         self.kernel, self.args = line.split()[1], dict(a.split("=") for a in line.split()[2:])
         self.stream = int(self.args["stream"], 16)
@@ -139,6 +142,42 @@ def general_forms_of_a_face():
             assert not [n for n in names() if n.startswith("sparse")], (change.__name__, precision, runs)
             s.close()
             assert FAKE.fake_live() == 0
+
+
+def streams_do_not_share_projections():
+    """Solvers of several runs whose neighbour step reads tInt: a step waits
+    for the one before it, whatever its stream; separate local steps and
+    steps that the caller captures leave the handle's projections alone."""
+    a, b = 0x51, 0x52
+    for precision, order, runs in ((32, 5, 8), (64, 3, 8), (64, 4, 16)):
+        s = Solver(mesh(), order, runs, precision)
+        assert s.info() == (5, 1)
+        events()
+        done = None
+        for n, stream, graph in ((2, a, 0), (1, b, 0), (3, b, 0), (3, a, 0), (3, b, 1), (1, a, 1), (2, None, 0)):
+            assert s.step(n, DOFS, TINT, stream, graph) == 0
+            ev = events()
+            sparse = [i for i, e in enumerate(ev) if isinstance(e, Launch) or e[0] == "graph"]
+            assert sparse
+            if done is not None:
+                waits = [i for i, e in enumerate(ev) if e == ("wait", done, hex(stream or 0)[2:])]
+                assert waits and waits[0] < sparse[0]
+            rec = [i for i, e in enumerate(ev) if e[0] == "record"]
+            assert len(rec) == 1 and rec[0] > sparse[-1] and ev[rec[0]][2] == hex(stream or 0)[2:]
+            done = ev[rec[0]][1]
+        assert s.local(DOFS2, TINT2, a) == 0 and s.neigh(DOFS2, TINT2, a) == 0
+        ev = events()
+        assert [e.name for e in ev if isinstance(e, Launch)][0] == "sparse local" and len(ev) == 2
+        assert ev[0].addr("proj") == 0 and not ev[1].name.startswith("sparse")
+        FAKE.fake_capturing(b)
+        assert s.step(3, DOFS2, TINT2, b) == 0
+        ev = events()
+        assert all(isinstance(e, Launch) and e.stream == b for e in ev) and len(ev) == 6
+        assert all(e.addr("proj") == 0 for e in ev if e.name == "sparse local")
+        assert not [e for e in ev if e.name in ("sparse neigh", "sparse fused")]
+        FAKE.fake_capturing(None)
+        s.close()
+        assert FAKE.fake_live() == 0
 
 
 def projections_exist():

@@ -188,3 +188,53 @@ def test_one_run_after_and_under_capture(gpu, precision):
         mo.neigh(d, t)
         assert rel(gd.cpu().numpy(), d) <= tol
     s.close()
+
+
+@pytest.mark.parametrize("precision,runs", [(32, 8), (64, 16)])
+def test_overlapping_steps_on_two_streams(gpu, precision, runs):
+    """Solvers whose neighbour step reads tInt: steps of independent arrays
+    that overlap on two streams, eager, as the solver's own graph, and captured
+    by the caller and replayed beside eager ones, give the bits of steps one
+    after the other (captured by the caller: with the neighbour kernel that
+    reads tInt, so to rounding)."""
+    import torch
+    order, n, tol = 4, 3, TOL[precision]
+    m, mat, dt, _, gd = _problem(runs, order, precision, n=(9, 8, 10))
+    s = ElasticSolver(m, order, runs, precision, *mat)
+    start = [gd, torch.flip(gd, dims=[0]) * 0.5]
+    want = []
+    for x in start:
+        x = x.clone()
+        t = torch.zeros_like(x)
+        s.step(x, t, dt, 1)
+        for _ in range(3):
+            s.step(x, t, dt, n)
+        want.append(x)
+    streams = [torch.cuda.Stream() for _ in start]
+    torch.cuda.synchronize()
+    for graph in (False, True):  # (the first array's steps of one call as the solver's graph)
+        got, tint = [x.clone() for x in start], [torch.zeros_like(x) for x in start]
+        torch.cuda.synchronize()
+        for k in (1, n, n, n):
+            s.step(got[0], tint[0], dt, k, graph=graph and k == n, stream=streams[0])
+            s.step(got[1], tint[1], dt, k, stream=streams[1])
+        torch.cuda.synchronize()
+        for x, w in zip(got, want):
+            assert torch.equal(x, w)
+    x, t = start[0].clone(), torch.zeros_like(gd)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=streams[0]):
+        s.step(x, t, dt, n, stream=torch.cuda.current_stream())
+    x.copy_(start[0])
+    y, ty = start[1].clone(), torch.zeros_like(gd)
+    torch.cuda.synchronize()
+    s.step(x, t, dt, 1, stream=streams[0])
+    s.step(y, ty, dt, 1, stream=streams[1])
+    for _ in range(3):
+        with torch.cuda.stream(streams[0]):
+            g.replay()
+        s.step(y, ty, dt, n, stream=streams[1])
+    torch.cuda.synchronize()
+    assert rel(x.cpu().numpy(), want[0].cpu().numpy()) <= tol
+    assert torch.equal(y, want[1])
+    s.close()
