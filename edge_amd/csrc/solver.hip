@@ -390,14 +390,19 @@ bool frames_orthonormal(const edge_mesh_in* m, int precision) {
 // the element-batched kernels.
 int finish_sp(edge_el_solver* s) {
   if (!s->want_sp) return EDGE_OK;
+  // the kernels chosen so far run without any of this
+  auto without = [&]() {
+    (void)hipGetLastError();
+    for (void* p : {s->sp_phys, s->sp_rot, (void*)s->sp_need}) (void)hipFree(p);
+    s->sp_phys = s->sp_rot = nullptr;
+    s->sp_need = nullptr;
+    return EDGE_OK;
+  };
   edge::DgTables t;
   std::vector<double> rot;
   if ((s->cfg.n_runs == 1 && !s->ec_ok) || !s->proj_ok || !s->faces_agree || !s->frames_ok ||
-      !edge::dg_tables(s->cfg.order, &t) || !edge::ec_rotations(t, &rot)) {
-    (void)hipFree(s->sp_phys);
-    s->sp_phys = nullptr;
-    return EDGE_OK;
-  }
+      !edge::dg_tables(s->cfg.order, &t) || !edge::ec_rotations(t, &rot))
+    return without();
   std::vector<double> pk(4 * edge::phys::kRotPad, 0.0);
   for (int v = 0; v < 4; v++)
     for (int p = 0; p < s->cfg.order; p++)
@@ -405,24 +410,25 @@ int finish_sp(edge_el_solver* s) {
         for (int c = 0; c <= p; c++)
           pk[v * edge::phys::kRotPad + edge::phys::rot_off(p) + j * (p + 1) + c] =
               rot[(v * 16 + p * (p + 1) / 2 + j) * 16 + p * (p + 1) / 2 + c];
-  const bool f32 = s->cfg.precision == 32;
-  const int rc = f32 ? upload_as<float>(pk, &s->sp_rot) : upload_as<double>(pk, &s->sp_rot);
-  if (rc) return rc;
-  const bool stands_in = s->cfg.kernel == 0 && s->kernel == 1;
-  if (stands_in &&
-      hipMalloc(&s->proj, s->real_bytes * edge::sp_proj_values(s->cfg.order, s->cfg.n_runs) * s->n_el) != hipSuccess) {
-    (void)hipGetLastError();  // no room for projections: the general kernels need none
-    s->proj = nullptr;
-    return EDGE_OK;
-  }
-  s->sp_ok = true;
+  if (s->cfg.precision == 32 ? upload_as<float>(pk, &s->sp_rot) : upload_as<double>(pk, &s->sp_rot)) return without();
   if (!s->h_fault_ef.empty()) {
     std::vector<uint8_t> need(s->n_el, 0);
     for (const int64_t ef : s->h_fault_ef) need[ef / 4] = 1;
-    EDGE_HIP_TRY(hipMalloc(&s->sp_need, s->n_el));
+    if (hipMalloc(&s->sp_need, s->n_el) != hipSuccess) {
+      s->sp_need = nullptr;
+      return without();
+    }
     EDGE_HIP_TRY(hipMemcpy(s->sp_need, need.data(), s->n_el, hipMemcpyHostToDevice));
   }
-  if (stands_in) s->kernel = 5;
+  if (s->cfg.kernel == 0 && s->kernel == 1) {
+    if (hipMalloc(&s->proj, s->real_bytes * edge::sp_proj_values(s->cfg.order, s->cfg.n_runs) * s->n_el) !=
+        hipSuccess) {
+      s->proj = nullptr;
+      return without();
+    }
+    s->kernel = 5;
+  }
+  s->sp_ok = true;
   return EDGE_OK;
 }
 
@@ -727,13 +733,18 @@ size_t proj_alt_bytes(const edge_el_solver* s) {
 
 // The second buffer of projections, allocated on first use.  Kernel 5 steps
 // without it (launch by launch) where it cannot be had: out of memory, or on
-// a stream that the caller is capturing.
+// a stream that the caller is capturing.  (A capture on another stream must
+// not be ended by the allocation: relaxed mode.)
 bool sp_second_buffer(edge_el_solver* s, hipStream_t st) {
   if (s->proj_alt || s->kernel == 2) return true;
   hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &c) == hipSuccess && c == hipStreamCaptureStatusNone &&
-      hipMalloc(&s->proj_alt, proj_alt_bytes(s)) == hipSuccess)
-    return true;
+  if (hipStreamIsCapturing(st, &c) == hipSuccess && c == hipStreamCaptureStatusNone) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    const bool set = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+    const hipError_t e = hipMalloc(&s->proj_alt, proj_alt_bytes(s));
+    if (set) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e == hipSuccess) return true;
+  }
   (void)hipGetLastError();
   s->proj_alt = nullptr;
   return false;

@@ -10,6 +10,7 @@
 #include <map>
 #include <mutex>
 #include <string>
+#include <utility>
 
 namespace {
 std::recursive_mutex lock_;
@@ -19,6 +20,7 @@ std::string log_;
 int fail_after_ = -1;         // allocations until one fails (0: the next), -1: none does
 size_t largest_ = 1ull << 36; // a larger allocation fails
 int setup_flags_ = 0;         // what the flux solver set-up kernel reports
+int mode_ = 0;                // the thread's capture mode (2: relaxed)
 void* capturing_ = nullptr;   // a stream that its owner captures
 int last_ = 0;
 uintptr_t next_ = 0x1000;
@@ -54,7 +56,10 @@ extern "C" {
 // for the tests
 const char* fake_log() { return log_.c_str(); }
 void fake_clear() { log_.clear(); }
-void fake_fail_after(int n) { fail_after_ = n; }
+int fake_fail_after(int n) {  // and what was left of the count (below 0: it has failed, or was not set)
+  std::swap(n, fail_after_);
+  return n;
+}
 void fake_setup_flags(int f) { setup_flags_ = f; }
 void fake_capturing(void* st) { capturing_ = st; }
 size_t fake_live() { return live_.size(); }
@@ -100,6 +105,10 @@ int hipLaunchKernel(const void* f, Dim3 g, Dim3, void** args, size_t, void* st) 
 }
 int hipMalloc(void** p, size_t n) {
   std::lock_guard<std::recursive_mutex> l(lock_);
+  if (capturing_ && mode_ != 2) {
+    note("allocation that ends a capture");
+    return last_ = kOom;
+  }
   if (n > largest_ || (fail_after_ >= 0 && fail_after_-- == 0)) {
     *p = nullptr;
     return last_ = kOom;
@@ -164,6 +173,10 @@ int hipStreamDestroy(void*) { return 0; }
 int hipStreamSynchronize(void*) { return 0; }
 int hipStreamIsCapturing(void* st, int* c) {
   *c = st && st == capturing_;
+  return 0;
+}
+int hipThreadExchangeStreamCaptureMode(int* m) {
+  std::swap(*m, mode_);
   return 0;
 }
 int hipStreamBeginCapture(void* st, int) {

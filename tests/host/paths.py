@@ -44,7 +44,7 @@ def events():
     """The runtime calls noted since the last time, in order."""
     out = []
     for line in FAKE.fake_log().decode().splitlines():
-        assert not line.startswith("free of"), line
+        assert not line.startswith(("free of", "allocation that")), line
         out.append(Launch(line) if line.startswith("launch") else tuple(line.replace("stream=", "").split()))
     FAKE.fake_clear()
     return out
@@ -58,9 +58,9 @@ def names():
     return [e.name for e in launches()]
 
 
-def mesh(n=(3, 4, 3), **kw):
+def mesh(n=(3, 4, 3), jitter=0.1, **kw):
     from edge_amd import mesh as M
-    return M.box(n, jitter=0.1, seed=5, **kw)
+    return M.box(n, jitter=jitter, seed=5, **kw)
 
 
 class Solver:
@@ -176,6 +176,53 @@ def streams_do_not_share_projections():
         assert all(e.addr("proj") == 0 for e in ev if e.name == "sparse local")
         assert not [e for e in ev if e.name in ("sparse neigh", "sparse fused")]
         FAKE.fake_capturing(None)
+        s.close()
+        assert FAKE.fake_live() == 0
+
+
+def no_room():
+    """Each allocation of the set-up failing in turn: the constants, maps, fault
+    marks and projections of the sparse kernels leave a solver on the general
+    kernels, with nothing of them kept; any other is an error.  Without room
+    for the second projection buffer a multi-step call goes launch by launch."""
+    from edge_amd import fault as FL
+    for precision, order, runs, general in ((32, 3, 8, 1), (32, 4, 1, 5), (32, 3, 16, 2), (64, 3, 16, 1), (64, 4, 1, 5)):
+        m = mesh((4, 4, 4), jitter=0)
+        assert len(FL.tag_plane(m, 2, 0.5)) > 0
+        s = Solver(m, order, runs, precision)
+        full, k, left = FAKE.fake_bytes(), 0, []
+        assert s.rc == 0, s.L.edge_last_error()
+        s.close()
+        while True:
+            FAKE.fake_fail_after(k)
+            s = Solver(m, order, runs, precision)
+            fired = FAKE.fake_fail_after(-1) < 0
+            FAKE.hipGetLastError()
+            if not fired:
+                assert s.rc == 0
+                s.close()
+                break
+            if s.rc == 0:
+                left.append(FAKE.fake_bytes())
+                events()
+                assert s.local() == 0 and s.neigh() == 0
+                assert not [n for n in names() if n.startswith("sparse")] and s.info()[0] == general
+                s.close()
+            assert FAKE.fake_live() == 0
+            k += 1
+        # phys, maps, marks; projections too where the solver has no others
+        assert len(left) == (4 if general == 1 else 3) and len(set(left)) == 1 and left[0] < full, (left, full)
+    for precision, order, runs in ((32, 3, 8), (32, 4, 1), (64, 3, 16)):
+        s = Solver(mesh(), order, runs, precision)
+        events()
+        FAKE.fake_fail_after(0)
+        assert s.step(3) == 0
+        FAKE.fake_fail_after(-1)
+        assert names() == 3 * ["sparse local", "sparse neigh"]
+        FAKE.fake_capturing(0x77)  # a capture on another stream goes on
+        assert s.step(2, stream=0x51) == 0
+        FAKE.fake_capturing(None)
+        assert names() == ["sparse local", "sparse fused", "sparse neigh"]
         s.close()
         assert FAKE.fake_live() == 0
 
