@@ -1292,6 +1292,7 @@ extern "C" int edge_el_autotune(edge_el_solver* s, double dt, int32_t n_reps, vo
                                                                         hipGetErrorString(e));
     return rc == EDGE_OK;
   };
+  const bool had_alt = s->proj_alt;
   // scratch DOFs (zeros: the same instruction stream as any data)
   if (hip(hipMalloc(&dofs, dof_bytes), "allocation") && hip(hipMalloc(&t_int, dof_bytes), "allocation") &&
       (s->n_rms == 0 || hip(hipMalloc(&dofs_a, a_bytes), "allocation")) &&
@@ -1307,9 +1308,10 @@ extern "C" int edge_el_autotune(edge_el_solver* s, double dt, int32_t n_reps, vo
       s->hi_occ = cand[i].occ;
       rc = one_step(s, dt, dofs, dofs_a, t_int, st);  // warm-up
       if (rc == EDGE_OK) hip(hipEventRecord(e0, st), "event");
-      if (cand[i].fused)  // one fused sequence of n_reps steps (n_reps + 1 launches)
-        rc = n_reps >= 2 ? fused_steps(s, n_reps, dt, dofs, dofs_a, t_int, st)
-                         : one_step(s, dt, dofs, dofs_a, t_int, st);
+      // as edge_el_step runs n_reps steps: kernel 5 of the sparse kernels fuses them like the fused variants
+      const bool fuse = cand[i].fused || (s->kernel == 5 && sp_fuses(s));
+      if (fuse && n_reps >= 2 && sp_second_buffer(s, st))  // one sequence of n_reps steps (n_reps + 1 launches)
+        rc = fused_steps(s, n_reps, dt, dofs, dofs_a, t_int, st);
       else
         for (int r = 0; r < n_reps && rc == EDGE_OK; r++) rc = one_step(s, dt, dofs, dofs_a, t_int, st);
       if (rc == EDGE_OK && hip(hipEventRecord(e1, st), "event") && hip(hipEventSynchronize(e1), "sync")) {
@@ -1343,6 +1345,10 @@ extern "C" int edge_el_autotune(edge_el_solver* s, double dt, int32_t n_reps, vo
   s->xcd_map = cand[best].xcd;
   s->use_fused = cand[best].fused;
   s->hi_occ = cand[best].occ;
+  if (!had_alt && s->kernel != 2 && s->kernel != 5) {  // only the candidates used it
+    (void)hipFree(s->proj_alt);
+    s->proj_alt = nullptr;
+  }
   if (n_cands) {
     const int32_t cap = *n_cands;
     *n_cands = (int32_t)cand.size();

@@ -513,9 +513,10 @@ int edge_el_neigh_lts_a(edge_el_solver *s, int64_t first, int64_t n_els, int32_t
  * 1: those report 5 and their edge_el_neigh reads t_int);
  * *flags bit 0: sparse (elastic-pattern) star matrices, bit 1: rank-3
  * factored flux solvers, bit 2: the neighbour step reads face projections,
- * bit 3: viscoelastic (anelastic DOFs), bit 4: multi-step calls fuse the
- * neighbour step of step k - 1 with the local step of step k (edge_el_step),
- * bit 5: the higher-occupancy variant of the kernels (FP32 viscoelastic MFMA
+ * bit 3: viscoelastic (anelastic DOFs), bit 4: edge_el_neigh_local
+ * and its viscoelastic form in edge_el_step_a are available (kernel 2 with
+ * projections; multi-step calls of kernel 5 over the matrices' non-zeros
+ * fuse without this bit), bit 5: the higher-occupancy variant of the kernels (FP32 viscoelastic MFMA
  * local kernel: tIntA in LDS, five waves per SIMD).
  * Diagnostic with no counterpart in the reference (for tests and tools). */
 int edge_el_kernel_info(const edge_el_solver *s, int32_t *kernel, int32_t *flags);

@@ -227,6 +227,26 @@ def no_room():
         assert FAKE.fake_live() == 0
 
 
+def autotuner_times_what_steps_run():
+    """A candidate of n repetitions is launched as edge_el_step(n) launches it."""
+    for precision, order, runs in ((32, 4, 1), (64, 4, 1), (32, 3, 8), (64, 3, 16), (32, 3, 16), (64, 5, 1)):
+        s = Solver(mesh(), order, runs, precision)
+        events()
+        n, kernels, flags = C.c_int32(16), (C.c_int32 * 16)(), (C.c_int32 * 16)()
+        ms = (C.c_double * 16)()
+        assert s.L.edge_el_autotune(s.h, 1e-3, 3, None, C.byref(n), kernels, flags, ms) == 0
+        ev = [e for e in events() if isinstance(e, Launch) or e[0] == "record"]
+        marks = [i for i, e in enumerate(ev) if e[0] == "record"]
+        timed = [[e.name for e in ev[a + 1:b]] for a, b in zip(marks[::2], marks[1::2])]
+        assert len(timed) == n.value
+        for i in range(n.value):
+            assert s.variant(kernels[i], flags[i]) == 0
+            assert s.step(3) == 0
+            assert timed[i] == names(), (precision, runs, kernels[i], flags[i])
+        s.close()
+        assert FAKE.fake_live() == 0
+
+
 def projections_exist():
     """Every launch of the sparse kernels has its constants, maps and
     projections, and a buffer large enough for them."""
