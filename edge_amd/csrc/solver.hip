@@ -8,6 +8,7 @@
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <tuple>
 #include <utility>
 #include <vector>
 
@@ -106,12 +107,11 @@ struct edge_el_solver {
   // graph path
   hipGraph_t graph = nullptr;
   hipGraphExec_t graph_exec = nullptr;
-  void* graph_dofs = nullptr;
-  void* graph_dofs_a = nullptr;
-  void* graph_tint = nullptr;
-  double graph_dt = 0;
-  hipStream_t graph_stream = nullptr;
-  int64_t graph_steps = 0;  // > 0: the graph holds a whole fused sequence of this many steps
+  // dofs, dofs_a, t_int, dt, stream and, where the graph holds a whole fused
+  // sequence, its steps (else 0): of the graph and of the last call that asked
+  // for one
+  using GraphKey = std::tuple<void*, void*, void*, double, hipStream_t, int64_t>;
+  GraphKey graph_key{}, asked_key{};
 };
 
 namespace {
@@ -830,7 +830,6 @@ void drop_graph(edge_el_solver* s) {
   if (s->graph) (void)hipGraphDestroy(s->graph);
   s->graph_exec = nullptr;
   s->graph = nullptr;
-  s->graph_steps = 0;
 }
 
 }  // namespace
@@ -1535,6 +1534,14 @@ int release_projections(edge_el_solver* s, hipStream_t st) {
   return EDGE_OK;
 }
 
+// A graph is being recorded on st.
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return false;
+}
+
 int steps_on(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* dofs_a, void* t_int, int use_graph,
              hipStream_t st) {
   const bool fuse = n_steps >= 2 && (fused_active(s) || (sp_fuses(s) && sp_second_buffer(s, st))) &&
@@ -1551,9 +1558,16 @@ int steps_on(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* do
   // a fused sequence is captured whole (one replay per call), a single step
   // otherwise (one replay per step)
   const int64_t gsteps = fuse ? n_steps : 0;
-  if (s->graph_exec && (s->graph_dofs != dofs || s->graph_dofs_a != dofs_a || s->graph_tint != t_int ||
-                        s->graph_dt != dt || s->graph_stream != st || s->graph_steps != gsteps))
-    drop_graph(s);
+  const edge_el_solver::GraphKey key{dofs, dofs_a, t_int, dt, st, gsteps};
+  const bool held = s->graph_exec && s->graph_key == key, again = s->asked_key == key;
+  s->asked_key = key;
+  if (fuse && s->kernel == 5 && !held && !again && !capturing(st))
+    // A sequence is captured when a call repeats the one before it.  Calls of
+    // 2 and 3 steps in turn, order 3, 384 tets, one run: 257 us a pair when
+    // each was captured anew, 105 launched (202 as replays of single
+    // steps).
+    return fused_steps(s, n_steps, dt, dofs, dofs_a, t_int, st);
+  if (s->graph_exec && !held) drop_graph(s);
   if (!s->graph_exec) {
     // capture needs a non-default stream
     hipStream_t cap = st;
@@ -1581,12 +1595,7 @@ int steps_on(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* do
       drop_graph(s);
       return rc;
     }
-    s->graph_dofs = dofs;
-    s->graph_dofs_a = dofs_a;
-    s->graph_tint = t_int;
-    s->graph_dt = dt;
-    s->graph_stream = st;
-    s->graph_steps = gsteps;
+    s->graph_key = key;
   }
   if (gsteps) {
     s->proj_tint = s->kernel == 5 ? t_int : nullptr;  // as after an eager fused sequence
@@ -1603,9 +1612,7 @@ int step_impl(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* d
               hipStream_t st) {
   if (n_steps == 0) return EDGE_OK;
   if (!reads_tint(s)) return steps_on(s, n_steps, dt, dofs, dofs_a, t_int, use_graph, st);
-  hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(st, &c) != hipSuccess) (void)hipGetLastError();
-  if (!use_graph && c != hipStreamCaptureStatusNone) {
+  if (!use_graph && capturing(st)) {
     // the caller's graph may be replayed beside any other call: nothing of the handle in it
     int rc = EDGE_OK;
     for (int64_t i = 0; i < n_steps && rc == EDGE_OK; i++) rc = one_step(s, dt, dofs, dofs_a, t_int, st, false);

@@ -221,7 +221,9 @@ int edge_el_neigh(edge_el_solver *s, int64_t first, int64_t n_els, const void *t
  * runs between the launches.  The DOFs are those of n_steps full steps
  * either way; after the call t_int holds the last step's tInt and no
  * separate edge_el_neigh may follow.  Kernel 5 over the matrices' non-zeros
- * fuses the same way (a separate edge_el_neigh may follow); without room for
+ * fuses the same way (a separate edge_el_neigh may follow; with use_graph
+ * != 0 the sequence becomes a graph when a call repeats the one before it,
+ * until then it is launched); without room for
  * its second buffer, or with none yet on a stream that the caller captures,
  * it steps launch by launch.
  * Solvers that exchange face projections hold them in the handle, so calls

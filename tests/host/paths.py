@@ -247,6 +247,28 @@ def autotuner_times_what_steps_run():
         assert FAKE.fake_live() == 0
 
 
+def graphs_of_repeated_calls():
+    """Kernel 5 captures a multi-step sequence when a call repeats the one
+    before it; calls whose step counts or arrays take turns are launched, and a
+    graph that is held is replayed whenever its call comes."""
+    def kinds(s, n, dofs=DOFS):
+        assert s.step(n, dofs, TINT, 0x51, 1) == 0
+        return [e[0] for e in events() if e[0] in ("begin", "graph", "launch")]
+
+    for precision, order, runs in ((32, 4, 1), (64, 4, 1), (32, 3, 8)):
+        s = Solver(mesh(), order, runs, precision)
+        events()
+        run = lambda n: ["launch"] * (n + 1)
+        assert kinds(s, 2) == run(2) and kinds(s, 3) == run(3) and kinds(s, 2) == run(2)
+        assert kinds(s, 3, DOFS2) == run(3) and kinds(s, 3) == run(3)
+        assert kinds(s, 3) == ["begin"] + run(3) + ["graph"]
+        assert kinds(s, 3) == ["graph"] and kinds(s, 2) == run(2) and kinds(s, 3) == ["graph"]
+        assert kinds(s, 1) == ["begin", "launch", "launch", "graph"] and kinds(s, 1) == ["graph"]
+        assert kinds(s, 2) == run(2) and kinds(s, 1) == ["graph"]
+        s.close()
+        assert FAKE.fake_live() == 0
+
+
 def projections_exist():
     """Every launch of the sparse kernels has its constants, maps and
     projections, and a buffer large enough for them."""

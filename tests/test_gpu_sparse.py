@@ -238,3 +238,21 @@ def test_overlapping_steps_on_two_streams(gpu, precision, runs):
     assert rel(x.cpu().numpy(), want[0].cpu().numpy()) <= tol
     assert torch.equal(y, want[1])
     s.close()
+
+
+@pytest.mark.parametrize("precision,runs", [(32, 1), (64, 1), (32, 8)])
+def test_repeated_graph_calls(gpu, precision, runs):
+    """Calls that ask for a graph: launched, captured when the call repeats,
+    replayed, with eager and other calls between, each against the oracle."""
+    import torch
+    order, tol = 4, TOL[precision]
+    m, mat, dt, d, gd = _problem(runs, order, precision)
+    s = ElasticSolver(m, order, runs, precision, *mat)
+    mo = orc.MeshOracle(m, order, runs, rho=mat[0], lam=mat[1], mu=mat[2])
+    t, gt = np.zeros_like(d), torch.zeros_like(gd)
+    for n, graph in ((2, True), (2, True), (2, True), (3, True), (3, False), (2, True), (1, True), (1, True), (2, True)):
+        mo.step(d, t, dt, n)
+        s.step(gd, gt, dt, n, graph=graph)
+        assert rel(gd.cpu().numpy(), d) <= tol
+        assert rel(gt.cpu().numpy(), t) <= tol
+    s.close()
