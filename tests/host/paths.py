@@ -269,6 +269,16 @@ def graphs_of_repeated_calls():
         assert FAKE.fake_live() == 0
 
 
+def more_waves_than_memory():
+    """A number of plane waves that fits no memory is an error code."""
+    s = Solver(mesh(), 3, 16, 32)
+    one = np.zeros(14)  # (nothing is read before the device memory exists)
+    live = FAKE.fake_live()
+    rc = s.L.edge_el_error_norms(s.h, DOFS, 0, 2**31 - 1, one.ctypes.data, 0.0, None, None, None, None)
+    assert rc != 0 and FAKE.fake_live() == live
+    s.close()
+
+
 def projections_exist():
     """Every launch of the sparse kernels has its constants, maps and
     projections, and a buffer large enough for them."""

@@ -23,7 +23,7 @@ def runtime(tmp_path_factory):
 
 @pytest.mark.parametrize("scenario", ["one_run_without_factors", "projections_exist", "general_forms_of_a_face",
                                       "streams_do_not_share_projections", "no_room", "autotuner_times_what_steps_run",
-                                      "graphs_of_repeated_calls"])
+                                      "graphs_of_repeated_calls", "more_waves_than_memory"])
 def test_host_path(runtime, scenario):
     r = subprocess.run([sys.executable, os.path.join(HERE, "paths.py"), runtime, scenario], capture_output=True,
                        text=True, timeout=300)
