@@ -1,4 +1,5 @@
 // The sparse element kernels of order 2 in FP64.
+#define EDGE_SP_LOW_FIRST 1
 #include "kernels_sparse_impl.hpp"
 
 namespace edge {

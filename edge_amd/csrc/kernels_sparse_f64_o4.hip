@@ -1,5 +1,6 @@
 // The sparse element kernels of order 4 in FP64.
 #define EDGE_SP_WAVES 8
+#define EDGE_SP_LOW_FIRST 1
 #include "kernels_sparse_impl.hpp"
 
 namespace edge {

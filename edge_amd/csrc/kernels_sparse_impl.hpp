@@ -75,6 +75,16 @@ constexpr int kCols = 64;  // columns (lanes) per workgroup tile
 #define EDGE_SP_WAVES 4
 #endif
 constexpr int kWaves = EDGE_SP_WAVES;
+// The order of a product's sums over the input modes: in FP32 the high ones
+// first.  A smooth column's are small, so the partial sums and their roundings
+// stay small until the low modes come (error against 64 bits after 4 steps of
+// smooth waves, 3,024 tets, order 5, 16 runs: 4.16e-7 -> 3.45e-7).  FP64 keeps
+// the low ones first: its error is the same either way (order 4: 5.88e-15).
+#ifndef EDGE_SP_LOW_FIRST
+#define EDGE_SP_LOW_FIRST 0
+#endif
+constexpr bool kLowFirst = EDGE_SP_LOW_FIRST;
+constexpr int nth(int i, int n) { return kLowFirst ? i : n - 1 - i; }
 
 // The order in which the modes and face modes are dealt to the waves: wave w
 // of W owns the modes at positions j W + w, and a column's LDS row is the
@@ -181,10 +191,11 @@ __device__ __forceinline__ T dot3(T a0, T b0, T a1, T b1, T a2, T b2) {
   return fma_(a2, b2, fma_(a1, b1, a0 * b0));
 }
 
-// Output N's first non-zero among the inputs below K.
-template <typename Mat, int K, int N>
+// No input of output N that comes before K in the order of the sums (below NK)
+// has a non-zero entry.
+template <typename Mat, int K, int N, int NK>
 constexpr bool starts() {
-  for (int k = 0; N >= 0 && k < K; k++)
+  for (int k = kLowFirst ? 0 : K + 1; N >= 0 && k < (kLowFirst ? K : NK); k++)
     if (Mat::at(k, N) != 0.0) return false;
   return true;
 }
@@ -221,35 +232,35 @@ template <int O, int NN, int W, int J>
 constexpr int mode_of() {
   return Dim<O>::mode(W, J) < NN ? Dim<O>::mode(W, J) : -1;
 }
-template <int O, int NN, int W, typename Mat, int K, typename T, int... J>
+template <int O, int NN, int W, typename Mat, int K, int NK, typename T, int... J>
 __device__ __forceinline__ void terms(T x, T* out, std::integer_sequence<int, J...>) {
-  (term<Mat, K, mode_of<O, NN, W, J>(), starts<Mat, K, mode_of<O, NN, W, J>()>()>(x, out[J]), ...);
+  (term<Mat, K, mode_of<O, NN, W, J>(), starts<Mat, K, mode_of<O, NN, W, J>(), NK>()>(x, out[J]), ...);
 }
-template <int O, int W, typename Mat, int K, typename T, int... J>
+template <int O, int W, typename Mat, int K, int NK, typename T, int... J>
 __device__ __forceinline__ void face_terms(T x, T* out, std::integer_sequence<int, J...>) {
-  (term<Mat, K, Dim<O>::face(W, J), starts<Mat, K, Dim<O>::face(W, J)>()>(x, out[J]), ...);
+  (term<Mat, K, Dim<O>::face(W, J), starts<Mat, K, Dim<O>::face(W, J), NK>()>(x, out[J]), ...);
 }
 // Input K of two columns with matrix D of three: p += M x and, summed over
 // the matrices, v += M y, each entry used for both.
-template <int O, int NN, int W, typename M0, typename M1, typename M2, int K, int D, int J, typename T>
+template <int O, int NN, int W, typename M0, typename M1, typename M2, int K, int NK, int D, int J, typename T>
 __device__ __forceinline__ void pair_term(T x, T y, T& p, T& v) {
   constexpr int N = mode_of<O, NN, W, J>();
   if constexpr (N >= 0) {
     using M = std::conditional_t<D == 0, M0, std::conditional_t<D == 1, M1, M2>>;
     constexpr double m = M::at(K, N);
     if constexpr (m != 0.0) {
-      constexpr bool s = starts<M0, K, N>() && starts<M1, K, N>() && starts<M2, K, N>();
+      constexpr bool s = starts<M0, K, N, NK>() && starts<M1, K, N, NK>() && starts<M2, K, N, NK>();
       constexpr bool n0 = M0::at(K, N) != 0.0, n1 = M1::at(K, N) != 0.0;
       constexpr bool first = s && (D < 1 || !n0) && (D < 2 || !n1);
       const T c = entry<T>(m);
-      p = starts<M, K, N>() ? c * x : fma_(c, x, p);
+      p = starts<M, K, N, NK>() ? c * x : fma_(c, x, p);
       v = first ? c * y : fma_(c, y, v);
     }
   }
 }
-template <int O, int NN, int W, typename M0, typename M1, typename M2, int K, int D, typename T, int... J>
+template <int O, int NN, int W, typename M0, typename M1, typename M2, int K, int NK, int D, typename T, int... J>
 __device__ __forceinline__ void pair_terms(T x, T y, T* p, T* v, std::integer_sequence<int, J...>) {
-  (pair_term<O, NN, W, M0, M1, M2, K, D, J>(x, y, p[J], v[J]), ...);
+  (pair_term<O, NN, W, M0, M1, M2, K, NK, D, J>(x, y, p[J], v[J]), ...);
 }
 
 template <int O, bool CK, int D>
@@ -258,7 +269,7 @@ using Stiff = std::conditional_t<CK, Ck<O, D>, Vol<O, D>>;
 // The LDS reads of a product in the order of its sums, each with the columns
 // and inputs it feeds.  A wave takes them in groups of G: the next group is
 // requested before the present one's multiply-adds, which keeps the LDS
-// latency behind about 30 of them (left to itself the compiler reads just
+// latency behind 15 to 30 of them (left to itself the compiler reads just
 // ahead of each use).
 struct Read {
   int col, k;
@@ -279,7 +290,8 @@ struct Reads {
 // outputs of wave V below NN, inputs below NK.
 template <int O, bool CK, int NK, int NN, int V>
 struct StiffReads {
-  static constexpr int J = Dim<O>::own(NN), G = 64 / kWaves, ROWS = NK;
+  // (order 5, FP32: groups of 8 instead of 16, order 5, 16 runs, 24,576 tets, 4 steps 3.03 -> 2.96 ms)
+  static constexpr int J = Dim<O>::own(NN), G = O == 5 ? 8 : 64 / kWaves, ROWS = NK;
   template <int D>
   static constexpr bool feeds(int k) {
     for (int j = 0; j < J; j++) {
@@ -291,9 +303,11 @@ struct StiffReads {
   // per input the four columns, one after the other
   static constexpr Reads<4 * NK> list() {
     Reads<4 * NK> l;
-    for (int k = 0; k < NK; k++)
+    for (int i = 0; i < NK; i++) {
+      const int k = nth(i, NK);
       if (feeds<0>(k) || feeds<1>(k) || feeds<2>(k))
         for (int c = 0; c < 4; c++) l.add(c, k);
+    }
     return l;
   }
   static constexpr int row(int k) { return Dim<O>::row(k); }
@@ -304,9 +318,9 @@ struct StiffReads {
       using M1 = Stiff<O, CK, 1>;
       using M2 = Stiff<O, CK, 2>;
       using JS = std::make_integer_sequence<int, J>;
-      pair_terms<O, NN, V, M0, M1, M2, K, 0>(x[0], x[1], p[0], v, JS{});
-      pair_terms<O, NN, V, M0, M1, M2, K, 1>(x[0], x[2], p[1], v, JS{});
-      pair_terms<O, NN, V, M0, M1, M2, K, 2>(x[0], x[3], p[2], v, JS{});
+      pair_terms<O, NN, V, M0, M1, M2, K, NK, 0>(x[0], x[1], p[0], v, JS{});
+      pair_terms<O, NN, V, M0, M1, M2, K, NK, 1>(x[0], x[2], p[1], v, JS{});
+      pair_terms<O, NN, V, M0, M1, M2, K, NK, 2>(x[0], x[3], p[2], v, JS{});
     }
   }
 };
@@ -317,7 +331,8 @@ struct ProjectReads {
   static constexpr int N = Dim<O>::N, J = Dim<O>::MF, G = 48 / kWaves, ROWS = 0;
   static constexpr Reads<N> list() {
     Reads<N> l;
-    for (int k = 0; k < N; k++) {
+    for (int i = 0; i < N; i++) {
+      const int k = nth(i, N);
       bool on = false;
       for (int j = 0; j < J; j++) {
         const int n = Dim<O>::face(V, j);
@@ -330,7 +345,7 @@ struct ProjectReads {
   static constexpr int row(int k) { return Dim<O>::row(k); }
   template <int COL, int K, typename T>
   static __device__ __forceinline__ void use(const T* x, T (&u)[J]) {
-    face_terms<O, V, Prj<O, F>, K>(x[0], u, std::make_integer_sequence<int, J>{});
+    face_terms<O, V, Prj<O, F>, K, N>(x[0], u, std::make_integer_sequence<int, J>{});
   }
 };
 
@@ -340,7 +355,8 @@ struct LiftReads {
   static constexpr int NF = Dim<O>::NF, J = Dim<O>::M, G = 64 / kWaves, ROWS = 0;
   static constexpr Reads<NF> list() {
     Reads<NF> l;
-    for (int k = 0; k < NF; k++) {
+    for (int i = 0; i < NF; i++) {
+      const int k = nth(i, NF);
       bool on = false;
       for (int j = 0; j < J; j++) {
         const int n = Dim<O>::mode(V, j);
@@ -353,7 +369,7 @@ struct LiftReads {
   static constexpr int row(int k) { return Dim<O>::face_row(k); }
   template <int COL, int K, typename T>
   static __device__ __forceinline__ void use(const T* x, T (&u)[J]) {
-    terms<O, Dim<O>::N, V, Lift<O, F>, K>(x[0], u, std::make_integer_sequence<int, J>{});
+    terms<O, Dim<O>::N, V, Lift<O, F>, K, NF>(x[0], u, std::make_integer_sequence<int, J>{});
   }
 };
 
@@ -507,6 +523,25 @@ struct Tile {
   static constexpr bool HELD = R == 1 || O < 5 || sizeof(T) == 8;
   T ji1[3][3];
   Mat4<T> mat1;
+  // FP32: where registers hold it, what a step adds to the DOFs is summed first,
+  // so that fewer roundings are of the DOFs' size:
+  //   SUM: all of a side's update (with several runs it takes a wave per SIMD:
+  //   order 3, 16 runs, 48,000 tets, 4 steps 1172 -> 1274 us);
+  //   VEL: the velocities that a component lifts, one rounding instead of four
+  //   (all components' in the neighbour step: order 5, 16 runs, 24,576 tets, 4
+  //   steps 2.96 -> 3.17 ms).
+  // Error against 64 bits after 4 steps of smooth waves, 3,024 tets, without
+  // and with: order 3, one run 1.9e-7 -> 1.5e-7, order 4, one run 2.6e-7 ->
+  // 2.3e-7.
+  static constexpr bool F32 = sizeof(T) == 4, SUM = F32 && R == 1 && O <= 3;
+  static constexpr bool VEL = F32 && !SUM && (O <= 3 || (O == 4 && R == 1));
+  // The time step is multiplied into what the volume integral and the
+  // projections take and give, or (SCALED) into their constants, whose
+  // rounding then is the same in every mode.  Order 4, 16 runs, 24,576 tets, 4
+  // steps: 1.42 ms with scaled constants, 1.30 without, error 2.9e-7 -> 2.7e-7;
+  // order 5, 16 runs: 2.99 and 3.09 ms, 3.45e-7 and 3.30e-7; FP64, order 4, 16
+  // runs, 12,870 tets, 2 steps: 1.27 and 1.28 ms, the same error.
+  static constexpr bool SCALED = R > 1 && (O == 5 || !F32);
 
   static constexpr int PB = phys::block(R);
   __device__ __forceinline__ Tile(const T* phys_el, int64_t first_)
@@ -724,10 +759,10 @@ struct Tile {
   }
 
   // Component i of the faces' lifted flux, the w of all faces in the first
-  // WROWS rows of LDS: velocities into acc, gradients into g; KC: phys::kOwn
-  // (the element's side) or phys::kOth (the other side)
+  // WROWS rows of LDS: velocities into vel (VEL) or acc, gradients into g; KC:
+  // phys::kOwn (the element's side) or phys::kOth (the other side)
   template <int KC>
-  __device__ __forceinline__ void lift(int i, T (&acc)[9][M], T (&g)[3][M]) {
+  __device__ __forceinline__ void lift(int i, T (&acc)[9][M], T (&vel)[3][M], T (&g)[3][M]) {
     const T* li = lds + i * D::NF * kCols + lane;
     each(
         [&](auto F) EDGE_INLINE {
@@ -751,23 +786,58 @@ struct Tile {
 #pragma unroll
             for (int j = 0; j < M; j++) {
               g[k][j] = fma_(sn[k], u[j], g[k][j]);
-              acc[6 + k][j] = fma_(e[k], u[j], acc[6 + k][j]);
+              T& v = VEL ? vel[k][j] : acc[6 + k][j];
+              v = fma_(e[k], u[j], v);
             }
         },
         std::make_integer_sequence<int, 4>{});
   }
 
+  // acc += what f adds to its argument (SUM: to zeros)
+  template <typename F>
+  static __device__ __forceinline__ void add(T (&acc)[9][M], F f) {
+    if constexpr (SUM) {
+      T d[9][M];
+#pragma unroll
+      for (int q = 0; q < 9; q++) zero(d[q]);
+      f(d);
+#pragma unroll
+      for (int q = 0; q < 9; q++)
+#pragma unroll
+        for (int j = 0; j < M; j++) acc[q][j] += d[q][j];
+    } else {
+      f(acc);
+    }
+  }
+  static __device__ __forceinline__ void zero(T (&x)[M]) {
+#pragma unroll
+    for (int j = 0; j < M; j++) x[j] = T(0);
+  }
+  // VEL: acc += the summed velocities
+  static __device__ __forceinline__ void add_velocities(T (&acc)[9][M], const T (&vel)[3][M]) {
+    if constexpr (VEL)
+#pragma unroll
+      for (int k = 0; k < 3; k++)
+#pragma unroll
+        for (int j = 0; j < M; j++) acc[6 + k][j] += vel[k][j];
+  }
+
   // acc += the neighbours' side of the faces' flux
   __device__ __forceinline__ void neigh(T (&acc)[9][M]) {
+    add(acc, [&](T(&a)[9][M]) EDGE_INLINE {
 #pragma unroll 1
-    for (int i = 0; i < 3; i++) {
-      T g[3][M];
+      for (int i = 0; i < 3; i++) {
+        T g[3][M], vel[3][M];
 #pragma unroll
-      for (int j = 0; j < M; j++) g[0][j] = g[1][j] = g[2][j] = T(0);
-      lift<phys::kOth>(i, acc, g);
-      const Mat4<T> m = mat();
-      by_axis(i, [&](auto I) EDGE_INLINE { add_stress<decltype(I)::value>(acc, g, m); });
-    }
+        for (int k = 0; k < 3; k++) zero(g[k]);
+#pragma unroll
+        for (int k = 0; k < 3; k++) zero(vel[k]);
+        lift<phys::kOth>(i, a, vel, g);
+        add_velocities(a, vel);
+        const Mat4<T> m = mat();
+        by_axis(i, [&](auto I) EDGE_INLINE { add_stress<decltype(I)::value>(a, g, m); });
+      }
+    });
   }
 
   // acc += volume integral and the element's side of the faces' flux, one
@@ -780,21 +850,27 @@ struct Tile {
 #pragma unroll
     for (int q = 0; q < 9; q++)
 #pragma unroll
-      for (int j = 0; j < MK; j++) xk[q][j] = t[q][j];
+      for (int j = 0; j < MK; j++) xk[q][j] = SCALED ? t[q][j] : dt * t[q][j];
+    add(acc, [&](T(&a)[9][M]) EDGE_INLINE {
 #pragma unroll 1
-    for (int i = 0; i < 3; i++) {
-      T g[3][M], v[M];
-      __syncthreads();  // the previous columns have been read
-      component<false, NK, D::N, true>(i, xk, buf, g, v, dt);
-      const T irho = mat().irho;
-      by_axis(i, [&](auto I) EDGE_INLINE {
+      for (int i = 0; i < 3; i++) {
+        T g[3][M], v[M];
+        __syncthreads();  // the previous columns have been read
+        component<false, NK, D::N, SCALED>(i, xk, buf, g, v, dt);
+        const T irho = mat().irho;
+        by_axis(i, [&](auto I) EDGE_INLINE {
 #pragma unroll
-        for (int j = 0; j < M; j++) acc[6 + decltype(I)::value][j] = fma_(irho, v[j], acc[6 + decltype(I)::value][j]);
-      });
-      lift<phys::kOwn>(i, acc, g);
-      const Mat4<T> m = mat();
-      by_axis(i, [&](auto I) EDGE_INLINE { add_stress<decltype(I)::value>(acc, g, m); });
-    }
+          for (int j = 0; j < M; j++) a[6 + decltype(I)::value][j] = fma_(irho, v[j], a[6 + decltype(I)::value][j]);
+        });
+        T vel[3][M];
+#pragma unroll
+        for (int k = 0; k < 3; k++) zero(vel[k]);
+        lift<phys::kOwn>(i, a, vel, g);
+        add_velocities(a, vel);
+        const Mat4<T> m = mat();
+        by_axis(i, [&](auto I) EDGE_INLINE { add_stress<decltype(I)::value>(a, g, m); });
+      }
+    });
   }
 
   // w of every face in the element's face coordinates, to LDS rows [f][i][NF]
@@ -811,7 +887,7 @@ struct Tile {
 #pragma unroll
       for (int k = 0; k < 3; k++) n[k] = next[phys::kNrm + k];
 #pragma unroll
-      for (int k = 0; k < 4; k++) a[k] = dt * next[phys::kPrj + k];
+      for (int k = 0; k < 4; k++) a[k] = SCALED ? dt * next[phys::kPrj + k] : next[phys::kPrj + k];
 #pragma unroll
       for (int k = 0; k < 7; k++) next[k] = face(f < 3 ? f + 1 : 3, k);
       __syncthreads();  // the previous columns have been read
@@ -826,7 +902,10 @@ struct Tile {
         const T tn = dot3(n[0], tr[0], n[1], tr[1], n[2], tr[2]);
         const T b = fma_(a[2], vn, -(a[3] * tn));
 #pragma unroll
-        for (int k = 0; k < 3; k++) own[(k * N + j * W) * kCols] = fma_(n[k], b, fma_(a[0], t[6 + k][j], -(a[1] * tr[k])));
+        for (int k = 0; k < 3; k++) {
+          const T wk = fma_(n[k], b, fma_(a[0], t[6 + k][j], -(a[1] * tr[k])));
+          own[(k * N + j * W) * kCols] = SCALED ? wk : dt * wk;
+        }
       }
       __syncthreads();
 #pragma unroll 1
