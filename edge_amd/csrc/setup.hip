@@ -319,6 +319,22 @@ __global__ void k_fs_factor(int64_t n_mats, const double* fs, T* fsf, int* bad) 
   if (!rank3_factors(fs + i * 81, fsf + i * 54)) atomicOr(bad, 8);
 }
 
+// The sparse kernels take a face's waves from its normal alone, which equals
+// the flux solvers T F T^-1 only where (normal, tangents) is orthonormal.  A
+// frame that is off by d moves the result by about d.  In FP64 1e-10 passes:
+// rounding alone leaves 1e-15 on a cube's jittered box and 5e-11 on one
+// stretched by 1e5.  In FP32 1e-6, a tenth of the bound that every path is held
+// to against the oracle.
+__device__ bool orthonormal(const double* n, const double* s, const double* t, double tol) {
+  const double* f[3] = {n, s, t};
+  for (int i = 0; i < 3; i++)
+    for (int j = 0; j <= i; j++) {
+      const double d = f[i][0] * f[j][0] + f[i][1] * f[j][1] + f[i][2] * f[j][2];
+      if (!(fabs(d - (i == j)) <= tol)) return false;  // (NaN: not orthonormal)
+    }
+  return true;
+}
+
 template <typename T>
 __global__ void k_flux_solvers(int64_t n_fa, int64_t n_el, const int64_t* fa_el, const int64_t* el_fa,
                                const int32_t* fa_type, const double* normals, const double* tangents,
@@ -395,6 +411,7 @@ __global__ void k_flux_solvers(int64_t n_fa, int64_t n_el, const int64_t* fa_el,
                                       sc * (zp2 - zs2) / r1, -sc * zs1 / r1, -sc * (zp1 - zs1) / r1};
     for (int i = 0; i < phys::kPerFace; i++) o[i * pb] = (T)v[i];
   };
+  if (ph && !orthonormal(n, s, t, sizeof(T) == 8 ? 1e-10 : 1e-6)) atomicOr(bad, 16);
   emit_phys(eL, fL, 1.0, rL, lL, mL, rR, lR, mR);
   if (eR >= 0) emit_phys(eR, fR, -1.0, rR, lR, mR, rL, lL, mL);
   face_solvers(rL, rR, lL, lR, mL, mR, n, s, t, fsurf, a, b);
@@ -412,7 +429,7 @@ __global__ void k_flux_solvers(int64_t n_fa, int64_t n_el, const int64_t* fa_el,
 
 template <typename T>
 int build_setup(const SetupInput& in, T* d_star, T* d_fs, double* d_jdet, T* d_fsf, bool* rank3, T* d_star_a,
-                T* d_fs_a, T* d_fsfa, T* d_phys, int phys_block, hipStream_t st) {
+                T* d_fs_a, T* d_fsfa, T* d_phys, int phys_block, bool* frames, hipStream_t st) {
   double *d_crds = nullptr, *d_rho = nullptr, *d_lam = nullptr, *d_mu = nullptr, *d_nrm = nullptr,
          *d_tan = nullptr, *d_area = nullptr;
   int64_t *d_elve = nullptr, *d_fael = nullptr, *d_elfa = nullptr;
@@ -476,15 +493,16 @@ int build_setup(const SetupInput& in, T* d_star, T* d_fs, double* d_jdet, T* d_f
   else if (bad & 2) rc = fail(EDGE_ERR_MESH, "inconsistent face-element relations");
   else if (bad & 4) rc = fail(EDGE_ERR_MESH, "face with non-positive area");
   if (rank3) *rank3 = d_fsf && !(bad & 8);
+  if (frames) *frames = !(bad & 16);
   cleanup();
 #undef EDGE_SETUP_TRY
   return rc;
 }
 
 template int build_setup<double>(const SetupInput&, double*, double*, double*, double*, bool*, double*, double*,
-                                  double*, double*, int, hipStream_t);
+                                  double*, double*, int, bool*, hipStream_t);
 template int build_setup<float>(const SetupInput&, float*, float*, double*, float*, bool*, float*, float*, float*,
-                                 float*, int, hipStream_t);
+                                 float*, int, bool*, hipStream_t);
 
 template <typename T>
 int factor_flux_solvers(const double* h_fs, int64_t n_mats, T* d_fsf, bool* rank3) {

@@ -32,10 +32,11 @@ struct SetupInput {  // host arrays
 // and d_fsfa also the anelastic solvers' factors U_A [2][nEl][4][6][3] over
 // the elastic factors' V^T (fs_a = U_A V^T to rounding, counted in *rank3).
 // With d_phys (may be null) the per-element constants of kernels_sparse.hpp
-// in blocks of phys_block elements.
+// in blocks of phys_block elements; *frames (may be null): every face's normal
+// and tangents are orthonormal.
 template <typename T>
 int build_setup(const SetupInput& in, T* d_star, T* d_fs, double* d_jdet, T* d_fsf, bool* rank3, T* d_star_a,
-                T* d_fs_a, T* d_fsfa, T* d_phys, int phys_block, hipStream_t st);
+                T* d_fs_a, T* d_fsfa, T* d_phys, int phys_block, bool* frames, hipStream_t st);
 
 // Rank-3 factors of n_mats host FP64 flux solvers [n_mats][81] into d_fsf
 // [n_mats][54] (device); *rank3 is false when any solver is not rank 3.

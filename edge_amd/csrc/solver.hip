@@ -363,25 +363,6 @@ int finish_ec(edge_el_solver* s) {
   return EDGE_OK;
 }
 
-// The sparse kernels take a face's waves from its normal alone, which equals
-// the flux solvers T F T^-1 only where (normal, tangents) is orthonormal.  A
-// frame that is off by d moves the result by about d.  In FP64 1e-10 passes:
-// rounding alone leaves 1e-15 on a cube's jittered box and 5e-11 on one
-// stretched by 1e5.  In FP32 1e-6, a tenth of the bound that every path is
-// held to against the oracle.
-bool frames_orthonormal(const edge_mesh_in* m, int precision) {
-  const double tol = precision == 64 ? 1e-10 : 1e-6;
-  for (int64_t fa = 0; fa < m->n_fa; fa++) {
-    const double* f[3] = {m->normals + fa * 3, m->tangents + fa * 6, m->tangents + fa * 6 + 3};
-    for (int i = 0; i < 3; i++)
-      for (int j = 0; j <= i; j++) {
-        const double d = f[i][0] * f[j][0] + f[i][1] * f[j][1] + f[i][2] * f[j][2];
-        if (!(std::fabs(d - (i == j)) <= tol)) return false;  // (NaN: not orthonormal)
-      }
-  }
-  return true;
-}
-
 // The sparse kernels' data, once the flux solvers exist: geometry-built
 // solvers (their constants are in sp_phys) whose faces pair up and have
 // orthonormal frames, with one projection slot per element face.  One run exchanges its projections through
@@ -878,7 +859,6 @@ extern "C" int edge_el_create(const edge_el_config* cfg, const edge_mesh_in* mes
                         lam,         mu};
     s->sparse_star = true;  // built from the Jacobians' pattern only
     const int pb = edge::phys::block(cfg->n_runs);
-    s->frames_ok = !s->want_sp || frames_orthonormal(mesh, cfg->precision);
     if (s->want_sp && hipMalloc(&s->sp_phys, s->real_bytes * edge::phys::values(s->n_el, pb)) != hipSuccess) {
       (void)hipGetLastError();  // no room: the other kernels run without these constants
       s->sp_phys = nullptr;
@@ -889,9 +869,11 @@ extern "C" int edge_el_create(const edge_el_config* cfg, const edge_mesh_in* mes
     else
       rc = cfg->precision == 64
                ? edge::build_setup<double>(in, (double*)s->star, (double*)s->fs, s->jdet, (double*)s->fsf,
-                                           &s->fs_rank3, nullptr, nullptr, nullptr, (double*)s->sp_phys, pb, nullptr)
+                                           &s->fs_rank3, nullptr, nullptr, nullptr, (double*)s->sp_phys, pb,
+                                           &s->frames_ok, nullptr)
                : edge::build_setup<float>(in, (float*)s->star, (float*)s->fs, s->jdet, (float*)s->fsf,
-                                          &s->fs_rank3, nullptr, nullptr, nullptr, (float*)s->sp_phys, pb, nullptr);
+                                          &s->fs_rank3, nullptr, nullptr, nullptr, (float*)s->sp_phys, pb,
+                                          &s->frames_ok, nullptr);
     if (rc == EDGE_OK) rc = zero_fault_faces(s);
     if (rc == EDGE_OK) rc = finish_mfma(s);
     if (rc == EDGE_OK) rc = finish_ec(s);
@@ -1104,10 +1086,10 @@ extern "C" int edge_el_create_visco(const edge_el_config* cfg, const edge_visco_
       rc = cfg->precision == 64
                ? edge::build_setup<double>(in, (double*)s->star, (double*)s->fs, s->jdet, (double*)s->fsf,
                                            &s->fs_rank3, (double*)s->star_a, (double*)s->fs_a, (double*)s->fsfa,
-                                           nullptr, 1, nullptr)
+                                           nullptr, 1, nullptr, nullptr)
                : edge::build_setup<float>(in, (float*)s->star, (float*)s->fs, s->jdet, (float*)s->fsf,
                                           &s->fs_rank3, (float*)s->star_a, (float*)s->fs_a, (float*)s->fsfa,
-                                          nullptr, 1, nullptr);
+                                          nullptr, 1, nullptr, nullptr);
     if (rc == EDGE_OK) rc = zero_fault_faces(s);
     if (rc == EDGE_OK) rc = upload_element_data(s, mesh, rho, s->lam_e.data(), s->mu_e.data());
     if (rc == EDGE_OK && p64_ok && src_pattern && (cfg->kernel == 0 || cfg->kernel == 4)) s->kernel = 4;
