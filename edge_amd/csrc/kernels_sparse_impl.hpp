@@ -1156,7 +1156,9 @@ int launch_sp(int op, const SolverDev<T>& s, const SpDev<T>& x, int64_t first, i
       if constexpr (sizeof(T) == 4 || O < 5) return by_op<T, O, 1>(op, s, x, first, n, dt, dofs, t_int, proj_in, st);
       break;
     case 8: return by_op<T, O, 8>(op, s, x, first, n, dt, dofs, t_int, proj_in, st);
-    case 16: return by_op<T, O, 16>(op, s, x, first, n, dt, dofs, t_int, proj_in, st);
+    case 16:
+      if constexpr (sizeof(T) == 4 || O < 5) return by_op<T, O, 16>(op, s, x, first, n, dt, dofs, t_int, proj_in, st);
+      break;
   }
   return fail(EDGE_ERR_UNSUPPORTED, "runs");
 }
