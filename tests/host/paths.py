@@ -117,13 +117,17 @@ def one_run_without_factors():
 
 def general_forms_of_a_face():
     """What only the flux solvers can express stays off the sparse kernels:
-    frames that the set-up kernel finds not to be orthonormal, and a free
-    surface between two elements."""
-    for frames in (True, False):
+    frames that the set-up kernel finds not to be orthonormal, a free surface
+    between two elements, and faces whose elements are not each other's
+    neighbours though every projection has one receiver."""
+    for form in ("frames", "surface", "swap"):
         for precision, order, runs in ((32, 4, 1), (32, 3, 8), (32, 4, 16), (64, 4, 1), (64, 3, 16)):
             m = mesh()
-            if frames:
+            if form == "frames":
                 FAKE.fake_setup_flags(16)
+            elif form == "swap":
+                for a in (m.el_fa_el, m.f_id, m.v_id):
+                    a[5, 1], a[90, 2] = a[90, 2], a[5, 1]
             else:
                 m.fa_type[np.argwhere((m.fa_el >= 0).all(axis=1))[9, 0]] = 101
             s = Solver(m, order, runs, precision)
@@ -132,7 +136,7 @@ def general_forms_of_a_face():
             events()
             for rc in (s.local(), s.neigh(), s.step(1), s.step(3)):
                 assert rc == 0
-            assert not [n for n in names() if n.startswith("sparse")], (frames, precision, runs)
+            assert not [n for n in names() if n.startswith("sparse")], (form, precision, runs)
             s.close()
             assert FAKE.fake_live() == 0
 

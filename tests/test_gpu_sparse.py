@@ -2,16 +2,17 @@
 64 (element, run) columns per workgroup, against the FP64 oracle: every order
 and run count on meshes whose last tile is partly filled, element ranges that
 start inside a tile, free-surface, outflow and periodic faces in every
-orientation; and a mesh whose neighbour relations do not pair up, which takes
-the general kernels."""
+orientation; meshes that only the flux solvers describe, which take the other
+kernels; steps that overlap on streams, and graphs."""
 import numpy as np
 import pytest
 
 import oracle as orc
 from edge_amd import mesh as M
 from edge_amd import setups as S
+from edge_amd._lib import EdgeError
 from edge_amd.mesh import FA_FREE_SURFACE, FA_OUTFLOW, FA_PERIODIC
-from edge_amd.solver import KERNEL_GENERIC, ElasticSolver
+from edge_amd.solver import KERNEL_EC64, KERNEL_GENERIC, KERNEL_MFMA, PATH_PROJECTIONS, ElasticSolver
 
 pytestmark = pytest.mark.gpu
 TOL = {32: 1e-5, 64: 1e-12}  # against the FP64 oracle, as every path of the precision
@@ -36,12 +37,14 @@ def _problem(runs, order, precision=32, n=(3, 4, 3), seed=5):
 @pytest.mark.parametrize("order", [2, 3, 4, 5])
 @pytest.mark.parametrize("precision", [32, 64])
 def test_steps_match_oracle(gpu, precision, order, runs):
-    """216 elements (3.4, 27 and 54 tiles of 64, 8 and 4): local, neighbour,
-    then three steps in one call."""
+    """162 elements (2 tiles of 64 and 34, 20 of 8 and 2, 40 of 4 and 2): local,
+    neighbour, then three steps in one call."""
     import torch
-    if (precision, order, runs) == (64, 5, 16):
-        pytest.skip("refused: FP64 order 5 has at most 8 runs")
-    m, mat, dt, d, gd = _problem(runs, order, precision)
+    m, mat, dt, d, gd = _problem(runs, order, precision, n=(3, 3, 3))
+    if (precision, order, runs) == (64, 5, 16):  # no kernel that reads tInt fits
+        with pytest.raises(EdgeError, match="no kernel"):
+            ElasticSolver(m, order, runs, precision, *mat)
+        return
     tol = TOL[precision]
     s = ElasticSolver(m, order, runs, precision, *mat)
     assert s.kernel_info()[0] == (2 if (precision, runs) == (32, 16) else 5)
@@ -90,16 +93,27 @@ def test_ranges_equal_whole(gpu, precision, runs):
     s.close()
 
 
-@pytest.mark.parametrize("runs", [1, 16])
-def test_neighbours_that_do_not_pair(gpu, runs):
+@pytest.mark.parametrize("swap", [False, True])
+@pytest.mark.parametrize("runs", [1, 8, 16])
+def test_neighbours_that_do_not_pair(gpu, runs, swap):
     """One face's neighbour replaced by another element: the projections no
-    longer have one receiver each, so the general kernels run."""
+    longer have one receiver each, so a kernel runs that reads tInt.  Two faces'
+    neighbours swapped: they have, but the faces' two elements are not each
+    other's neighbours, so the kernels run that read the flux solvers."""
     import torch
     order = 3
     m, mat, dt, d, gd = _problem(runs, order)
-    el, fa = np.argwhere((m.fa_el[m.el_fa] >= 0).all(axis=2) & (m.fa_type[m.el_fa] == 0))[5]
-    m.el_fa_el[el, fa] = (m.el_fa_el[el, fa] + 7) % m.n_el
+    inner = np.argwhere((m.fa_el[m.el_fa] >= 0).all(axis=2) & (m.fa_type[m.el_fa] == 0))
+    (el, fa), (e2, f2) = inner[5], inner[90]
+    if swap:
+        for a in (m.el_fa_el, m.f_id, m.v_id):
+            a[el, fa], a[e2, f2] = a[e2, f2], a[el, fa]
+    else:
+        m.el_fa_el[el, fa] = (m.el_fa_el[el, fa] + 7) % m.n_el
     s = ElasticSolver(m, order, runs, 32, *mat)
+    kernel, flags = s.kernel_info()
+    assert kernel == {1: KERNEL_EC64 if swap else KERNEL_GENERIC, 8: KERNEL_GENERIC, 16: KERNEL_MFMA}[runs]
+    assert bool(flags & PATH_PROJECTIONS) == (swap and runs != 8)
     mo = orc.MeshOracle(m, order, runs, rho=mat[0], lam=mat[1], mu=mat[2])
     t, gt = np.zeros_like(d), torch.zeros_like(gd)
     mo.step(d, t, dt, 2)
