@@ -41,6 +41,34 @@ FLOPS = {4: {"local": 20466 + 630 + 20520 + 35280, "neigh": 35280, "proj": 4 * 2
          5: {"local": 67986 + 1260 + 54810 + 85320, "neigh": 85320, "proj": 4 * 2 * 9 * 35 * 15}}
 
 
+def sparse_flops(order):
+    """FLOPs per element, step and run that the kernels over the matrices'
+    non-zeros execute (kernels_sparse_impl.hpp): two per non-zero and column of
+    a product, and the pointwise work between the products.  local = CK +
+    volume + projections + the element's side of the faces, neigh = face
+    orientation + the neighbours' side; the fused launch performs both."""
+    from edge_amd import setups as S
+    g = S.dg_matrices(order)
+    n, n1, nf = S.n_modes(order), S.n_modes(order - 1), S.n_face_modes(order)
+
+    def nnz(a):
+        return int(np.count_nonzero(np.abs(a) > 1e-12))
+
+    def stiff(m, nk, nn):
+        # per velocity component: it and its three star-combined stress rows (published: 3 dots of 3) times the
+        # three matrices, the gradients (3 dots of 3), the stresses (5 FMAs) and the velocity (1)
+        return 3 * (2 * 2 * nnz(m[:, :nk, :nn]) + 15 * nk + (15 + 10 + 2) * nn)
+
+    ck = sum(stiff(g["stiffT"], S.n_modes(order - d + 1), S.n_modes(order - d)) + 2 * 9 * S.n_modes(order - d)
+             for d in range(1, order))
+    # tractions, normal components and the wave vector per face and mode, then its three columns to the face modes
+    project = 4 * (5 * 5 + 3 + 3 * 4) * n + 3 * 2 * nnz(g["fluxL"])
+    # per component and face the lifted column, its gradient and velocity terms; the stresses once per component
+    lift = 3 * (2 * nnz(g["fluxT"]) + 4 * 12 * n + 10 * n)
+    turn = 4 * 3 * 2 * sum((p + 1) ** 2 for p in range(order))
+    return {"local": ck + stiff(g["stiffV"], n1, n) + project + lift, "neigh": turn + lift}
+
+
 def alg_bytes(order, runs, s, s_c):
     """Compulsory bytes per element-step: DOFs read+write, tInt write+read,
     dense star + two flux-solver sets, connectivity."""
@@ -50,19 +78,20 @@ def alg_bytes(order, runs, s, s_c):
 
 def local_bytes(order, runs, prec=4, proj=False):
     """Compulsory bytes per element of one local launch: DOFs read and
-    written, tInt written, dense star matrices and local flux solvers read,
-    and with proj the face projections written (4 faces x 3 x 16 x 16)."""
+    written, tInt written, dense star matrices and local flux solvers read;
+    with proj (the kernels over the non-zeros) 69 constants instead of those,
+    and the face projections written (4 faces x 3 x 16 x 16)."""
     n = order * (order + 1) * (order + 2) // 6
-    return 3 * 9 * n * runs * prec + (3 * 81 + 4 * 81) * prec + (4 * 3 * 256 * prec if proj else 0)
+    return 3 * 9 * n * runs * prec + ((69 + 4 * 3 * 256) if proj else (3 * 81 + 4 * 81)) * prec
 
 
 def launch_bytes(order, runs, variant, prec=4):
     """Compulsory bytes per element of the dominant FP32 launch: the local
     kernel (local_bytes), or the fused one, which also reads the face
-    projections its neighbours wrote and the neighbour-side flux solvers."""
+    projections its neighbours wrote and the connectivity."""
     if variant != "fused":
         return local_bytes(order, runs, prec, proj=variant == "proj")
-    return local_bytes(order, runs, prec, proj=True) + 4 * 3 * 256 * prec + 4 * 81 * prec + 80
+    return local_bytes(order, runs, prec, proj=True) + 4 * 3 * 256 * prec + 80
 
 
 # FP32 variants: (projections exchanged, XCD-aware schedule, fused multi-step)
@@ -100,8 +129,8 @@ def read_mfma_util(path, n_el, order, runs, kernel):
     return None
 
 
-def read_traffic(path, n_el, order, runs):
-    """HBM bytes per launch of the local kernel from a committed rocprofv3
+def read_traffic(path, n_el, order, runs, launch):
+    """HBM bytes per launch ("fused" or "local") from a committed rocprofv3
     summary: FETCH_SIZE and WRITE_SIZE (KiB per dispatch), each scaled by
     bytes / counter for a copy kernel of known size.  None when the summary
     is absent or describes another workload."""
@@ -114,7 +143,7 @@ def read_traffic(path, n_el, order, runs):
                     kv[m.group(1)] = float(m.group(2))
         if (int(kv["elements"]), int(kv["order"]), int(kv["runs"])) != (n_el, order, runs):
             return None
-        return (kv["local_fetch_kib"] * kv["fetch_scale"] + kv["local_write_kib"] * kv["write_scale"]) * 1024.0
+        return (kv[f"{launch}_fetch_kib"] * kv["fetch_scale"] + kv[f"{launch}_write_kib"] * kv["write_scale"]) * 1024.0
     except (OSError, KeyError, ValueError):
         return None
 
@@ -436,7 +465,7 @@ def fault_row(args, timed):
     neighbour) per time step; beside it the fault phase alone."""
     import torch
     from edge_amd import fault as FL
-    from edge_amd.solver import ElasticSolver
+    from edge_amd.solver import PATH_PROJECTIONS, ElasticSolver
     order, runs = 4, 16
     m, rho, lam, mu, frame, glob, st0, dt = fault_problem(order, runs)
     s = ElasticSolver(m, order, runs, 32, rho, lam, mu)
@@ -449,7 +478,7 @@ def fault_row(args, timed):
     ms = timed(lambda st: s.step(d, t, dt, n_steps, graph=True, stream=st), 1) / n_steps
     st, slip = f.get()
     fault_ms = timed(lambda st: f.apply(d, t, dt, stream=st), 5)
-    fl = FLOPS[order]
+    fl = sparse_flops(order) if s.kernel_info()[1] & PATH_PROJECTIONS else FLOPS[order]
     n = s.n_modes
     step_flop = (fl["local"] + fl["neigh"]) * runs * m.n_el
     print(json.dumps({"row": "config 4: elastic + dynamic rupture (coupled step)", "elements": m.n_el,
@@ -693,6 +722,10 @@ def main():
     if fl:
         k32 = res["fp32"]["k"]
         f_step = fl["local"] + fl["neigh"]
+        # what the kernels execute: with projections the products over the non-zeros on the vector ALU (whose
+        # FP32 peak is that of MFMA), else the dense ones; the dense count stays as a rate to compare with
+        ex = sparse_flops(order) if proj else {"local": fl["local"], "neigh": fl["neigh"]}
+        f_step, d_step = ex["local"] + ex["neigh"], fl["local"] + fl["neigh"]
         if fused and "fused" in k32:
             # the fused launch: neighbour step k - 1 (projection lifts) and
             # local step k with the projections it writes: a whole step's FLOPs
@@ -701,21 +734,19 @@ def main():
             desc = ("fused neighbour step k - 1 + local step k (projection lifts; CK + volume + local surface + "
                     "neighbour-flux projections)")
         else:
-            f_loc = fl["local"] + (fl["proj"] if proj else 0)
-            dom, f_dom, t_dom = "local", f_loc, k32["local"]
+            dom, f_dom, t_dom = "local", ex["local"], k32["local"]
             t_step = k32["local"] + k32["neigh"]
             desc = "local (CK + volume + local surface" + (" + neighbour-flux projections)" if proj else ")")
         achieved = f_dom * runs * m.n_el / t_dom
         step_ach = f_step * runs * m.n_el / t_step
-        traffic = read_traffic(TRAFFIC_PROFILE[variant], m.n_el, order, runs)
-        # the kernels with projections skip the matrices' zeros on the vector ALU (same FP32 peak as
-        # MFMA); the dense FLOP count includes the zeros
+        traffic = read_traffic(TRAFFIC_PROFILE[variant], m.n_el, order, runs, dom)
         roof = {"bound": "valu" if proj else "mfma", "achieved": achieved / 1e12, "peak": PEAK["fp32_mfma"] / 1e12, "unit": "TFLOP/s",
                 "frac": achieved / PEAK["fp32_mfma"], "traffic": traffic,
                 "traffic_alg": launch_bytes(order, runs, variant) * m.n_el,
                 "kernel": desc, "kernel_ms": t_dom * 1e3, "flops_per_element_run": f_dom,
                 "kernel_ms_all": {k: v * 1e3 for k, v in k32.items()},
-                "step_tflops": step_ach / 1e12, "step_frac": step_ach / PEAK["fp32_mfma"]}
+                "step_tflops": step_ach / 1e12, "step_frac": step_ach / PEAK["fp32_mfma"],
+                "step_dense_equivalent_tflops": d_step * runs * m.n_el / t_step / 1e12}
         util = read_mfma_util(MFMA_PROFILE, m.n_el, order, runs, dom_kernel_name(variant, order))
         if util is not None:
             roof["mfma_busy"] = util
@@ -765,7 +796,8 @@ def main():
                                   res["fp32_r1"]["steps"], "local_ms": 1e3 * k1["local"], "neigh_ms": 1e3 * k1["neigh"],
                                   "kernel": res["fp32_r1"]["kernel"], "finite": res["fp32_r1"]["finite"]}
         if fl:
-            a1 = (fl["local"] + fl["neigh"]) * m.n_el / (k1["local"] + k1["neigh"])
+            f1 = sparse_flops(order) if res["fp32_r1"]["kernel"] == KERNEL_EC64 else fl
+            a1 = (f1["local"] + f1["neigh"]) * m.n_el / (k1["local"] + k1["neigh"])
             out["fp32_single_run"]["roofline_frac"] = a1 / PEAK["fp32_mfma"]
     if not args.no_cpu:
         print("[bench] cpu baseline", file=sys.stderr, flush=True)

@@ -30,18 +30,18 @@
 // map R_v (ec64_pack.hpp).
 //
 // What bounds it: vector-ALU issue (about 40,000 instructions per tile and
-// 64 columns at order 5 against 131,000 cycles of padded MFMA tiles; 46 % of
-// the issue slots are used) and the memory latency that two (order 5) or
-// three workgroups per CU leave exposed.  A load behind output stores waits
+// 64 columns at order 5 against 131,000 cycles of padded MFMA tiles; the
+// vector ALUs are busy 55 % of the time) and the memory latency that two (order
+// 5) or three workgroups per CU leave exposed.  A load behind output stores waits
 // for all of them, so constants come first, the projections leave last and
 // tInt is written while they are formed.
 // Eight waves of half the modes (128 registers) took 10.9 ms per order-5 step
 // against 7.7 for four.
 // Measured against the kernels that did the same before (ms per step): order
-// 5, 196,608 tets, 16 runs with sources and receivers 8.60 -> 6.3 (MFMA, runs
-// on N); one run 1.19 -> 0.57 (MFMA, 16 elements on N); order 5, 36,720 tets,
+// 5, 196,608 tets, 16 runs with sources and receivers 8.60 -> 6.4 (MFMA, runs
+// on N); one run 1.19 -> 0.53 (MFMA, 16 elements on N); order 5, 36,720 tets,
 // 8 runs 6.81 -> 0.69 (generic); order 4 with a fault, 331,776 tets, 16 runs
-// 10.3 -> 5.3; FP64 order 4, 12,870 tets, 16 runs 5.66 -> 0.64
+// 10.3 -> 5.1; FP64 order 4, 12,870 tets, 16 runs 5.66 -> 0.64
 // (generic); order 5, 10,368 tets, 8 runs 5.85 -> 0.73 (generic).
 //
 // Operations (src/impl/seismic/solvers/AderDg.hpp:362-533, :553-722):
