@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <memory>
+#include <new>
 #include <type_traits>
 #include <vector>
 
@@ -352,21 +354,23 @@ extern "C" int edge_el_error_norms(edge_el_solver* h, const void* dofs, int32_t 
   // one block: points and weights, basis (both in groups of kPts, the last
   // one filled up with zeros), waves; then the partial sums and the sums
   const size_t n_pt = (size_t)groups * kPts * 4, n_bs = (size_t)groups * kPts * N, n_wv = (size_t)R * n_waves * 14;
-  std::vector<double> in(n_pt + n_bs, 0.0);
+  const size_t n_in = n_pt + n_bs + n_wv;
+  hipStream_t st = (hipStream_t)stream;
+  const unsigned nblk = 1024;
+  Scratch d;
+  EDGE_HIP_TRY(hipMalloc(&d.p, sizeof(double) * (n_in + (size_t)3 * nqr * (nblk + 1))));
+  // (the number of waves is the caller's: no allocation throws for it)
+  const std::unique_ptr<double[]> in(new (std::nothrow) double[n_in]());
+  if (!in) return edge::fail(EDGE_ERR_NOMEM, "error norms: waves");
   for (int p = 0; p < np; p++) {
     for (int i = 0; i < 3; i++) in[4 * (size_t)p + i] = pts[3 * p + i];
     in[4 * (size_t)p + 3] = w[p];
     for (int n = 0; n < N; n++)
       in[n_pt + ((size_t)(p / kPts) * N + n) * kPts + p % kPts] = basis[(size_t)p * N + n];
   }
-  hipStream_t st = (hipStream_t)stream;
-  const unsigned nblk = 1024;
-  Scratch d;
-  // (the waves straight from the caller's array: their number is the caller's, and no host copy can fail here)
-  EDGE_HIP_TRY(hipMalloc(&d.p, sizeof(double) * (in.size() + n_wv + (size_t)3 * nqr * (nblk + 1))));
-  double *part = d.p + in.size() + n_wv, *out = part + (size_t)3 * nqr * nblk;
-  EDGE_HIP_TRY(hipMemcpyAsync(d.p, in.data(), sizeof(double) * in.size(), hipMemcpyHostToDevice, st));
-  if (n_wv) EDGE_HIP_TRY(hipMemcpyAsync(d.p + in.size(), waves, sizeof(double) * n_wv, hipMemcpyHostToDevice, st));
+  if (n_wv) std::copy_n(waves, n_wv, in.get() + n_pt + n_bs);
+  double *part = d.p + n_in, *out = part + (size_t)3 * nqr * nblk;
+  EDGE_HIP_TRY(hipMemcpyAsync(d.p, in.get(), sizeof(double) * n_in, hipMemcpyHostToDevice, st));
   const double *d_pt = d.p, *d_bs = d.p + n_pt, *d_wv = d_bs + n_bs;
   auto launch = [&](auto t, auto n) {
     using T = decltype(t);
