@@ -1505,10 +1505,15 @@ extern "C" int edge_el_neigh_lts(edge_el_solver* s, int64_t first, int64_t n_els
 }
 
 namespace {
-// The projections of the handle (reads_tint solvers), for a call on st.
+// The projections of the handle (reads_tint solvers), for a call on st.  The
+// event orders work of this device alone, so it needs no fence that shows its
+// memory to the host and other devices (order 3, 8 FP32 runs, 480 tets, one
+// step: 22.7 us with the fence, 20.9 without, 19.3 without an event).
 int acquire_projections(edge_el_solver* s, hipStream_t st) {
-  if (!s->sp_done) EDGE_HIP_TRY(hipEventCreateWithFlags(&s->sp_done, hipEventDisableTiming));
-  else EDGE_HIP_TRY(hipStreamWaitEvent(st, s->sp_done, 0));
+  if (s->sp_done)
+    EDGE_HIP_TRY(hipStreamWaitEvent(st, s->sp_done, 0));
+  else
+    EDGE_HIP_TRY(hipEventCreateWithFlags(&s->sp_done, hipEventDisableTiming | hipEventDisableSystemFence));
   return EDGE_OK;
 }
 int release_projections(edge_el_solver* s, hipStream_t st) {
