@@ -180,7 +180,8 @@ class ElasticSolver:
     def step(self, dofs, t_int, dt, n_steps=1, graph=False, stream=None):
         """n_steps global time steps (local, then neigh); with graph=True the
         step (or a fused sequence, PATH_FUSED) is captured into a HIP graph on
-        first use and replayed."""
+        first use and replayed (fused sequences of kernel 5: when a call
+        repeats the one before it)."""
         self._check_arr(dofs)
         self._check_arr(t_int)
         _lib.check(_lib.lib().edge_el_step(self._h, int(n_steps), float(dt), dofs.data_ptr(), t_int.data_ptr(),

@@ -272,3 +272,35 @@ def test_repeated_graph_calls(gpu, precision, runs):
         assert rel(gd.cpu().numpy(), d) <= tol
         assert rel(gt.cpu().numpy(), t) <= tol
     s.close()
+
+
+@pytest.mark.parametrize("precision,runs,order", [(32, 8, 4), (64, 8, 3), (64, 16, 4)])
+def test_fault_of_several_runs(gpu, precision, runs, order):
+    """A fault between the fused launches of solvers of several runs on kernel 5
+    (their tInt is written in every step for the fault's elements only), and
+    between separate steps, against the coupled oracle."""
+    import torch
+    from edge_amd import fault as FL
+    from test_gpu_fault import _problem as fault_problem
+    m, rho, lam, mu, frame, glob, st0 = fault_problem(order, runs)
+    dt, tol = S.dt_cfl(m, rho, lam, mu, order), TOL[precision]
+    s = ElasticSolver(m, order, runs, precision, rho, lam, mu)
+    assert s.kernel_info()[0] == KERNEL_EC64
+    f = FL.Fault(s, m, rho, lam, mu, frame, glob, st0)
+    fo = orc.FaultOracle(m, order, runs, rho, lam, mu, frame, glob, st0)
+    d = 0.01 * np.random.default_rng(5).normal(size=(m.n_el, 9, S.n_modes(order), runs))
+    gd = torch.tensor(d.astype(NP[precision]), device="cuda").contiguous()
+    d = gd.double().cpu().numpy()
+    t, gt = np.zeros_like(d), torch.zeros_like(gd)
+    for n in (3, 1, 2):
+        fo.step(d, t, dt, n)
+        s.step(gd, gt, dt, n)
+        assert rel(gd.cpu().numpy(), d) <= tol
+        assert rel(gt.cpu().numpy(), t) <= tol
+    fo.step(d, t, dt, 1)
+    s.local(gd, gt, dt)
+    f.apply(gd, gt, dt)
+    s.neigh(gd, gt)
+    assert rel(gd.cpu().numpy(), d) <= tol
+    f.close()
+    s.close()
