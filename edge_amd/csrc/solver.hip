@@ -1599,7 +1599,10 @@ int step_impl(edge_el_solver* s, int64_t n_steps, double dt, void* dofs, void* d
               hipStream_t st) {
   if (n_steps == 0) return EDGE_OK;
   if (!reads_tint(s)) return steps_on(s, n_steps, dt, dofs, dofs_a, t_int, use_graph, st);
-  if (!use_graph && capturing(st)) {
+  const bool caller_captures = capturing(st);
+  if (caller_captures && use_graph)  // refused there: a stream holds one capture
+    return steps_on(s, n_steps, dt, dofs, dofs_a, t_int, use_graph, st);
+  if (caller_captures) {
     // the caller's graph may be replayed beside any other call: nothing of the handle in it
     int rc = EDGE_OK;
     for (int64_t i = 0; i < n_steps && rc == EDGE_OK; i++) rc = one_step(s, dt, dofs, dofs_a, t_int, st, false);

@@ -180,6 +180,7 @@ int hipThreadExchangeStreamCaptureMode(int* m) {
   return 0;
 }
 int hipStreamBeginCapture(void* st, int) {
+  if (st == capturing_) return last_ = 401;  // (already being captured)
   note("begin stream=" + hex(st));
   return 0;
 }

@@ -172,6 +172,9 @@ def streams_do_not_share_projections():
         assert all(isinstance(e, Launch) and e.stream == b for e in ev) and len(ev) == 6
         assert all(e.addr("proj") == 0 for e in ev if e.name == "sparse local")
         assert not [e for e in ev if e.name in ("sparse neigh", "sparse fused")]
+        for n in (1, 3):  # a graph of the solver's own is refused there, and the caller's left alone
+            assert s.step(n, DOFS2, TINT2, b, 1) != 0 and events() == []
+            FAKE.hipGetLastError()
         FAKE.fake_capturing(None)
         s.close()
         assert FAKE.fake_live() == 0
